@@ -375,22 +375,36 @@ __global__ void k_head(const uint16_t *__restrict__ x, const float *__restrict__
     }
 }
 // dx[v][c] = w[c] dout[v]; per-block partials of dw[c] = sum_v x[v][c] dout[v]
-// and db = sum_v dout[v] (17 values per block, summed later in block order)
+// and db = sum_v dout[v] (17 values per block, summed later by k_sum_rows).
+// Bound by its traffic (32 B read and written and 4 B read per voxel): a
+// voxel's 16 channels move as two 16-byte accesses each way.
 __global__ void __launch_bounds__(256) k_head_bwd(const uint16_t *__restrict__ x, const float *__restrict__ w,
                                                   const float *__restrict__ dout, uint16_t *__restrict__ dx,
                                                   float *__restrict__ part, int64_t n) {
     __shared__ float red[17][4];
-    float acc[17];
+    float acc[17], wr[16];
+#pragma unroll
     for (int c = 0; c < 17; c++) acc[c] = 0.f;
+#pragma unroll
+    for (int c = 0; c < 16; c++) wr[c] = w[c];
     for (int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x; i < n; i += (int64_t)gridDim.x * blockDim.x) {
         const float d = dout[i];
+        uint4 q[2], o[2];
+        q[0] = *reinterpret_cast<const uint4 *>(x + i * 16);
+        q[1] = *reinterpret_cast<const uint4 *>(x + i * 16 + 8);
+        const uint16_t *h = reinterpret_cast<const uint16_t *>(q);
+        uint16_t *oh = reinterpret_cast<uint16_t *>(o);
+#pragma unroll
         for (int c = 0; c < 16; c++) {
-            acc[c] += bf2f(x[i * 16 + c]) * d;
-            dx[i * 16 + c] = f2bf(w[c] * d);
+            acc[c] += bf2f(h[c]) * d;
+            oh[c] = f2bf(wr[c] * d);
         }
         acc[16] += d;
+        *reinterpret_cast<uint4 *>(dx + i * 16) = o[0];
+        *reinterpret_cast<uint4 *>(dx + i * 16 + 8) = o[1];
     }
     const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+#pragma unroll
     for (int c = 0; c < 17; c++) {
         float v = acc[c];
         for (int o = 32; o > 0; o >>= 1) v += __shfl_xor(v, o, 64);
@@ -400,6 +414,96 @@ __global__ void __launch_bounds__(256) k_head_bwd(const uint16_t *__restrict__ x
     if (threadIdx.x < 17)
         part[(size_t)blockIdx.x * 17 + threadIdx.x] =
             (red[threadIdx.x][0] + red[threadIdx.x][1]) + (red[threadIdx.x][2] + red[threadIdx.x][3]);
+}
+
+// out[c] = sum over the nrows rows of part[nrows][C] (C <= 128) in row order,
+// one workgroup per job.  The sum is one chain of FP32 additions per column
+// (its order is part of the result); what it cost was a load latency per
+// row, with a launch of one thread per column for each tensor: 593 us per
+// bias gradient, 1.44 and 0.61 ms for the head's at 4 x 128^3.  Here the
+// workgroup streams the rows through two LDS tiles, the next one's loads in
+// flight during the current one's additions, so a row costs an addition, and
+// all tensors of a backward pass run side by side in one launch.
+constexpr int kSumTile = 8192;   // floats per LDS tile
+struct SumRowsJob {
+    const float *part;
+    float *out;
+    int nrows, C;
+};
+constexpr int kSumRowsJobs = 15;
+struct SumRowsArgs {
+    SumRowsJob job[kSumRowsJobs];
+};
+__global__ void __launch_bounds__(256) k_sum_rows(SumRowsArgs a) {
+    __shared__ float tile[2][kSumTile];
+    const SumRowsJob J = a.job[blockIdx.x];
+    const int tid = threadIdx.x, rows = kSumTile / J.C, per = rows * J.C;
+    const int64_t total = (int64_t)J.nrows * J.C;
+    constexpr int NL = kSumTile / 256;
+    float pre[NL];
+    auto fetch = [&](int64_t base) {
+#pragma unroll
+        for (int u = 0; u < NL; u++) {
+            const int k = tid + 256 * u;
+            pre[u] = k < per && base + k < total ? J.part[base + k] : 0.f;
+        }
+    };
+    float acc = 0.f;
+    fetch(0);
+    int buf = 0;
+    for (int r0 = 0; r0 < J.nrows; r0 += rows, buf ^= 1) {
+#pragma unroll
+        for (int u = 0; u < NL; u++) tile[buf][tid + 256 * u] = pre[u];
+        __syncthreads();   // the other tile's readers were done before the tile before this one was stored
+        fetch((int64_t)(r0 + rows) * J.C);
+        if (tid < J.C) {
+            const float *t = tile[buf] + tid;
+            const int n = min(rows, J.nrows - r0);
+            int r = 0;
+            for (; r + 16 <= n; r += 16) {
+                float v[16];
+#pragma unroll
+                for (int u = 0; u < 16; u++) v[u] = t[(r + u) * J.C];
+#pragma unroll
+                for (int u = 0; u < 16; u++) acc += v[u];
+            }
+            for (; r < n; r++) acc += t[r * J.C];
+        }
+    }
+    if (tid < J.C) J.out[tid] = acc;
+}
+
+// Partial sums of a [n][C] BF16 tensor (C a power of two, 16..128): partial
+// q of nq sums the rows r with (r / L) mod nq = q, L = 256 / C, row class
+// r mod L by row class, the classes then in order.  A partial is 32 threads'
+// work (a thread takes 8 channels, one 16-byte load, of one row class), a
+// workgroup eight partials.
+__global__ void __launch_bounds__(256) k_chan_sum_part(const uint16_t *__restrict__ x, int C, int64_t n, int nq,
+                                                       float *__restrict__ part) {
+    __shared__ float red[256][9];
+    const int ng = C >> 3, L = 256 / C;
+    const int sub = threadIdx.x >> 5, t32 = threadIdx.x & 31, grp = t32 % ng, r0 = t32 / ng;
+    const int q = blockIdx.x * 8 + sub;
+    float s[8];
+#pragma unroll
+    for (int j = 0; j < 8; j++) s[j] = 0.f;
+    if (q < nq)
+        for (int64_t i = (int64_t)q * L + r0; i < n; i += (int64_t)nq * L) {
+            const uint4 w = *reinterpret_cast<const uint4 *>(x + i * C + grp * 8);
+            const uint16_t *h = reinterpret_cast<const uint16_t *>(&w);
+#pragma unroll
+            for (int j = 0; j < 8; j++) s[j] += bf2f(h[j]);
+        }
+#pragma unroll
+    for (int j = 0; j < 8; j++) red[threadIdx.x][j] = s[j];
+    __syncthreads();
+    for (int k = threadIdx.x; k < 8 * C; k += 256) {
+        const int qs = k / C, c = k % C;
+        if (blockIdx.x * 8 + qs >= nq) continue;
+        float t = 0.f;
+        for (int r = 0; r < L; r++) t += red[qs * 32 + r * ng + (c >> 3)][c & 7];
+        part[(size_t)(blockIdx.x * 8 + qs) * C + c] = t;
+    }
 }
 
 // Input features of the network per voxel (8 BF16 channels):
@@ -707,6 +811,7 @@ struct UNet {
     uint16_t *X = nullptr, *A[kNL] = {}, *Pl[3] = {}, *dA[kNL] = {}, *dP[3] = {}, *dcat[3] = {};
     float *out = nullptr, *dout = nullptr, *wpart = nullptr, *hpart = nullptr, *cpart = nullptr;
     size_t wpart_n = 0;
+    size_t cpart_off[kNL] = {};   // each layer's bias-gradient partials in cpart
 
     UNet() {
         int64_t o = 0;
@@ -802,7 +907,12 @@ struct UNet {
         UCHK(dalloc(&out, nvox(0)));
         UCHK(dalloc(&dout, nvox(0)));
         UCHK(dalloc(&hpart, (size_t)unet_head_bwd_blocks(nvox(0)) * 17));
-        UCHK(dalloc(&cpart, (size_t)4096 * 256));
+        size_t cp = 0;
+        for (int i = 0; i < kNL; i++) {
+            cpart_off[i] = cp;
+            cp += (size_t)chan_parts(nvox(kLayers[i].level)) * kLayers[i].co;
+        }
+        UCHK(dalloc(&cpart, cp));
         return hipSuccess;
     }
     const uint16_t *input_of(int idx) const {
@@ -833,14 +943,14 @@ struct UNet {
         return launch_unet_head(A[kNL - 1], par + hw, par + hb, out, nvox(0), s);
     }
 
-    // per-channel sums of a [n][C] BF16 tensor into g[C] (bias gradients)
-    hipError_t chan_sum(const uint16_t *x, int C, int64_t n, float *g, hipStream_t s);
+    // partials of the per-channel sums of dA[layer] (its bias gradient)
+    static int chan_parts(int64_t n);
+    hipError_t chan_sum(int layer, hipStream_t s);
 
     hipError_t backward(hipStream_t s) {
         const int64_t n0 = nvox(0);
         const int hbk = unet_head_bwd_blocks(n0);
         UCHK(launch_unet_head_bwd(A[kNL - 1], par + hw, dout, dA[kNL - 1], hpart, n0, s));
-        UCHK(head_bias(hbk, s));
         for (int i = kNL - 1; i >= 0; i--) {
             const LayerDef &d = kLayers[i];
             const int l = d.level;
@@ -871,7 +981,7 @@ struct UNet {
             g.per = per;
             UCHK(launch_unet_wgrad(g, d.c1, d.c2, d.co, d.up2, nch, s));
             UCHK(launch_unet_sum_chunks(wpart, nch, 27LL * cin * d.co, grad + woff[i], s));
-            UCHK(chan_sum(dA[i], d.co, n, grad + boff[i], s));
+            UCHK(chan_sum(i, s));
             if (i == 0) break;
             // input gradient: the transposed convolution of dA[i]
             ConvArgs a{};
@@ -898,65 +1008,29 @@ struct UNet {
                 UCHK(launch_unet_conv(a, d.co, 0, cin, false, false, batch, s));
             }
         }
-        return hipSuccess;
+        return sum_rows(hbk, s);
     }
-    hipError_t head_bias(int hbk, hipStream_t s);
+    // sums the partials of the head's and every layer's bias gradients
+    hipError_t sum_rows(int hbk, hipStream_t s);
 };
 
-__global__ void k_chan_sum_part(const uint16_t *__restrict__ x, int C, int64_t n, float *__restrict__ part) {
-    // block b sums rows b, b + gridDim.x, ... for channel threadIdx.x % C
-    const int c = threadIdx.x % C, lanes = blockDim.x / C, r0 = threadIdx.x / C;
-    __shared__ float red[256];
-    float s = 0.f;
-    if (r0 < lanes)
-        for (int64_t i = (int64_t)blockIdx.x * lanes + r0; i < n; i += (int64_t)gridDim.x * lanes)
-            s += unet::bf2f(x[i * C + c]);
-    red[threadIdx.x] = s;
-    __syncthreads();
-    if (threadIdx.x < C) {
-        float t = 0.f;
-        for (int r = 0; r < lanes; r++) t += red[r * C + threadIdx.x];
-        part[(size_t)blockIdx.x * C + threadIdx.x] = t;
-    }
-}
-// part[b][C] -> out[c] = sum_b part[b][c] in block order
-__global__ void k_chan_sum_final(const float *__restrict__ part, int nb, int C, float *__restrict__ out) {
-    const int c = blockIdx.x * blockDim.x + threadIdx.x;
-    if (c >= C) return;
-    float t = 0.f;
-    for (int b = 0; b < nb; b++) t += part[(size_t)b * C + c];
-    out[c] = t;
-}
+int UNet::chan_parts(int64_t n) { return (int)(n / 64 < 1 ? 1 : (n / 64 > 4096 ? 4096 : n / 64)); }
 
-hipError_t UNet::chan_sum(const uint16_t *x, int C, int64_t n, float *g, hipStream_t s) {
-    const int threads = C >= 256 ? C : 256 / C * C;
-    int64_t nb = n / 64;
-    nb = nb < 1 ? 1 : (nb > 4096 ? 4096 : nb);
-    hipLaunchKernelGGL(k_chan_sum_part, dim3((unsigned)nb), dim3((unsigned)threads), 0, s, x, C, n, cpart);
-    UCHK(hipGetLastError());
-    hipLaunchKernelGGL(k_chan_sum_final, dim3((unsigned)((C + 127) / 128)), dim3(128), 0, s, cpart, (int)nb, C, g);
+hipError_t UNet::chan_sum(int layer, hipStream_t s) {
+    const LayerDef &d = kLayers[layer];
+    const int nq = chan_parts(nvox(d.level));
+    hipLaunchKernelGGL(k_chan_sum_part, dim3((unsigned)((nq + 7) / 8)), dim3(256), 0, s, dA[layer], d.co,
+                       nvox(d.level), nq, cpart + cpart_off[layer]);
     return hipGetLastError();
 }
 
-// the head's bias gradient: entry 16 of each block's 17 partials
-__global__ void k_head_bias(const float *__restrict__ part, int nb, float *__restrict__ out) {
-    if (threadIdx.x != 0 || blockIdx.x != 0) return;
-    float t = 0.f;
-    for (int b = 0; b < nb; b++) t += part[(size_t)b * 17 + 16];
-    out[0] = t;
-}
-// the head's weight gradient from the 17-strided partials
-__global__ void k_head_w(const float *__restrict__ part, int nb, float *__restrict__ out) {
-    const int c = threadIdx.x;
-    if (c >= 16) return;
-    float t = 0.f;
-    for (int b = 0; b < nb; b++) t += part[(size_t)b * 17 + c];
-    out[c] = t;
-}
-hipError_t UNet::head_bias(int hbk, hipStream_t s) {
-    hipLaunchKernelGGL(k_head_w, dim3(1), dim3(64), 0, s, hpart, hbk, grad + hw);
-    UCHK(hipGetLastError());
-    hipLaunchKernelGGL(k_head_bias, dim3(1), dim3(64), 0, s, hpart, hbk, grad + hb);
+hipError_t UNet::sum_rows(int hbk, hipStream_t s) {
+    SumRowsArgs a{};
+    for (int i = 0; i < kNL; i++)
+        a.job[i] = {cpart + cpart_off[i], grad + boff[i], chan_parts(nvox(kLayers[i].level)), kLayers[i].co};
+    a.job[kNL] = {hpart, grad + hw, hbk, 17};   // the head's 16 weights, then its bias (hb = hw + 16)
+    static_assert(kNL + 1 == kSumRowsJobs, "a job per layer and the head");
+    hipLaunchKernelGGL(k_sum_rows, dim3(kSumRowsJobs), dim3(256), 0, s, a);
     return hipGetLastError();
 }
 
