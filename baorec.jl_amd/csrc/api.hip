@@ -883,19 +883,20 @@ double *votherd(MGPyr &P, int l) { return P.cur[l] ? P.Ad[l] : P.Bd[l]; }
 // n damped Jacobi sweeps (jacobi!, src/multigrid.jl:193-210) ping-ponging
 // between a (the input) and b; returns the one holding the result.  On
 // grids of at least 128^3 cells whose sides are multiples of 64, 16 and 8,
-// sweeps run 3 (or 2) per launch, temporally blocked (the same bits).
+// sweeps run two per z-marching launch, and an odd one as such a launch of
+// its own (the same bits).
 static float *jacobi_sweeps(baorec_ctx *c, const MGLevel &L, int64_t R, float *a, float *b, const float *f,
                             const baorec_params *p, int n) {
     const bool tb = mg_jacobi_tb_ok(L) && R >= ((int64_t)1 << 21);
     for (int left = n; left > 0;) {
-        const int k = !tb || left == 1 ? 1 : (left == 2 || left == 4 ? 2 : 3);
+        const int k = tb && left >= 2 ? 2 : 1;
         ProfScope ps(c, k == 1 ? "mg_jacobi" : "mg_jacobi_tb", 12.0 * R);
-        if (k == 1)
+        if (!tb)
             hipchk(c, launch_mg_jacobi(b, a, f, L, p->beta, p->jacobi_damping_factor, p->has_los, c->stream),
                    "jacobi");
         else
             hipchk(c, launch_mg_jacobi_tb(b, a, f, L, p->beta, p->jacobi_damping_factor, p->has_los, k, c->stream),
-                   "jacobi (blocked)");
+                   "jacobi (z-marching)");
         std::swap(a, b);
         left -= k;
     }

@@ -331,8 +331,8 @@ hipError_t launch_mg_xvec(float *xv, const Slot *slot, int nx, int ny, int nz, h
 template <typename T>
 hipError_t launch_mg_rbgs(T *v, const T *f, const MGLevel &L, float beta, int has_los, int color,
                           hipStream_t s);
-// 2 or 3 damped Jacobi sweeps in one launch, out of place (vout != vin),
-// bitwise that many launch_mg_jacobi calls; sides multiples of 64, 16, 8.
+// 1 or 2 damped Jacobi sweeps in one z-marching launch, out of place (vout !=
+// vin), bitwise that many launch_mg_jacobi calls; sides multiples of 64, 16, 8.
 bool mg_jacobi_tb_ok(const MGLevel &L);
 hipError_t launch_mg_jacobi_tb(float *vout, const float *vin, const float *f, const MGLevel &L, float beta,
                                float omega, int has_los, int sweeps, hipStream_t s);

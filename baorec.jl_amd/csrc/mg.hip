@@ -602,184 +602,264 @@ __global__ void __launch_bounds__(kGsThreads) k_mg_gs4(float *__restrict__ vout,
     }
 }
 
-// S damped Jacobi sweeps in one launch (temporal blocking), out of place:
-// vout is what S launches of k_mg_jacobi leave (the same cell arithmetic on
-// the same values, so the same bits).  A workgroup owns a 64 x 16 column of
-// tz planes and marches up z; sweep level t (t = 1..S) of the tile, grown by
-// S - t cells in x and y, lives in a ring of 4 LDS planes (level 0: the old
-// values, loaded).  Step k loads plane P = z0 - S + k and computes level t
-// on plane P - 2t + 1: level t - 1 there and on both neighbouring planes was
-// finished in earlier steps, and the stages of one step touch disjoint
-// planes, so one barrier per step orders them.  Level S (the tile itself)
-// goes straight to vout, a row per wave.
-constexpr int kJbTX = 64, kJbTY = 16, kJbRing = 4, kJbMaxTz = 128;
+// The reciprocal of b for div_by: one Newton step on v_rcp_f32.
+__device__ __forceinline__ float refined_rcp(float b) {
+    const float y = __builtin_amdgcn_rcpf(b);
+    return __builtin_fmaf(__builtin_fmaf(-b, y, 1.0f), y, y);
+}
+// a / b from y = refined_rcp(b): the correction steps of the IEEE division, so
+// its result where no operand needs scaling (|a| >= 2^-104 or 0, normal b and
+// quotient); zeros, infinities and NaN by v_div_fixup_f32.
+__device__ __forceinline__ float div_by(float a, float b, float y) {
+    float q = a * y;
+    q = __builtin_fmaf(__builtin_fmaf(-b, q, a), y, q);
+    q = __builtin_fmaf(__builtin_fmaf(-b, q, a), y, q);
+    return __builtin_amdgcn_div_fixupf(q, b, a);
+}
+
+// S = 1 or 2 damped Jacobi sweeps in one launch, out of place: vout is what S
+// launches of k_mg_jacobi leave (the same cell arithmetic on the same
+// values, so the same bits).  A workgroup owns a 64 x TY column of tz planes
+// and marches up z; sweep level t (t = 1..S) of the tile, grown by S - t cells
+// in x and y, lives in a ring of 4 LDS planes (level 0: the old values,
+// loaded).  Step k loads plane P = z0 - S + k and computes level t on plane
+// P - 2t + 1: level t - 1 there and on both neighbouring planes was finished
+// in earlier steps, and the stages of one step touch disjoint planes, so one
+// barrier per step orders them.  Level S goes straight to vout.
+//
+// What bounds it is the arithmetic (about 65 operations per update in the
+// reference's order, two of them divisions), so the mapping saves
+// instructions: a wave owns 4 rows of the tile, a column per lane, at every
+// level.  Its y and z coefficients are uniform, a row's loads serve the row
+// beside it (28 LDS reads per 2 cells instead of 38), and a cell's g and f stay
+// in registers from level 1 to level 2, two steps later: one IEEE division
+// per cell and pass.  The division by the diagonal has no scaling steps
+// (div_by).  The tile's halo cells of level 1 (rows -1 and TY, columns -1 and
+// 64) are one extra cell per lane.  Three waves per SIMD, 168 VGPRs: with the
+// reciprocals kept as well it spilled (401 against 324 us per sweep), and tiles
+// of 32 rows, one workgroup per CU, ran 376-430 us.
+// Per sweep, local LOS, 512^3 / 256^3 / 128^3: 324 / 47 / 12 us; with two
+// divisions per update and cells dealt to the threads level by level, 2 or 3
+// sweeps per launch, 560 / 73 / 14 us.
+constexpr int kJbTX = 64, kJbRing = 4, kJbMaxTz = 128;
 
 template <int S>
 struct JbShape {
-    // 512 threads at S = 3 keep its per-thread cell lists short enough for
-    // two waves per SIMD without spills
-    static constexpr int Threads = S == 3 ? 512 : 256;
-    static constexpr int CPT = kJbTX * kJbTY / Threads;   // level-S cells per thread (one column)
-    static constexpr int RS = Threads / kJbTX;             // rows between them
-    static constexpr int W = kJbTX + 2 * S, H = kJbTY + 2 * S, Plane = W * H;
-    // cells of the levels below S: level t covers (64 + 2e) x (16 + 2e), e = S - t
-    static constexpr int cells(int t) { return (kJbTX + 2 * (S - t)) * (kJbTY + 2 * (S - t)); }
-    static constexpr int Inner = S == 2 ? cells(1) : cells(1) + cells(2);
-    static constexpr int Iters = (Inner + Threads - 1) / Threads;
-    static constexpr int Chunks = (W + 3) / 4 * H;   // float4 columns per plane row (last may overhang)
+    static constexpr int TY = 16, Waves = TY / 4, Threads = 64 * Waves;
+    static constexpr int W0 = kJbTX + 2 * S, H0 = TY + 2 * S, Plane0 = W0 * H0;
+    static constexpr int W1 = kJbTX + 2, H1 = TY + 2, Plane1 = S == 2 ? W1 * H1 : 0;
+    static constexpr int Loads = (Plane0 + Threads - 1) / Threads;
+    static constexpr int Lds = kJbRing * (Plane0 + Plane1);
 };
 
 // LOS: a fixed line of sight (has_los), as a template constant
 template <int S, int LOS>
-__global__ void __launch_bounds__(JbShape<S>::Threads, 2) k_mg_jacobi_tb(float *__restrict__ vout, const float *__restrict__ vin,
-                                                             const float *__restrict__ f, MGLevel L, float beta,
-                                                             float omega, int tz) {
-    static_assert(S == 2 || S == 3, "2 or 3 sweeps per pass");
-    constexpr int has_los = LOS;
+__global__ void __launch_bounds__(JbShape<S>::Threads, 3) k_mg_jacobi_zm(float *__restrict__ vout,
+                                                                            const float *__restrict__ vin,
+                                                                            const float *__restrict__ f, MGLevel L,
+                                                                            float beta, float omega, int tz) {
+    static_assert(S == 1 || S == 2, "1 or 2 sweeps per pass");
     using J = JbShape<S>;
-    __shared__ __align__(16) float lds[S * kJbRing * J::Plane];
-    __shared__ float ptab[J::W + J::H + kJbMaxTz + 2 * S];
+    constexpr int TY = J::TY;
+    __shared__ __align__(16) float lds[J::Lds];
     const int nx = L.n[0], ny = L.n[1], nz = L.n[2];
     int tile_x, tile_y, tile_z;
     mg_tile(tile_x, tile_y, tile_z);
-    const int x0 = tile_x * kJbTX, y0 = tile_y * kJbTY, z0 = tile_z * tz;
-    const int64_t sy = nx, sz = (int64_t)nx * ny;
-    const int tid = threadIdx.x;
-    float *pz_tab = ptab + J::W + J::H;
-    if (!has_los)
-        for (int q = tid; q < J::W + J::H + tz + 2 * S; q += J::Threads) {
-            int g;
-            if (q < J::W)
-                g = gs_wrap(x0 - S + q, nx);
-            else if (q < J::W + J::H)
-                g = nx + gs_wrap(y0 - S + q - J::W, ny);
-            else
-                g = nx + ny + gs_wrap(z0 - S + q - J::W - J::H, nz);
-            ptab[q] = L.pv[g];
-        }
-    auto plane = [&](int t, int Pl) {   // level t, local plane Pl = P - z0 + S >= 0
-        return lds + (t * kJbRing + (Pl & (kJbRing - 1))) * J::Plane;
-    };
-    // level-0 loads: element q = row * W + col, one float per element (W is
-    // not a multiple of 4 at S = 3); threads past the plane reload element 0
-    constexpr int NL = (J::Plane + J::Threads - 1) / J::Threads;
-    int64_t ld_off[NL];
+    const int x0 = tile_x * kJbTX, y0 = tile_y * TY, z0 = tile_z * tz;
+    const uint32_t sy = nx;
+    const int64_t sz = (int64_t)nx * ny;
+    const int tid = threadIdx.x, lane = tid & 63;
+    const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+    float *ring0 = lds, *ring1 = lds + kJbRing * J::Plane0;
+    // level-0 loads: element q = row * W0 + col (threads past the plane reload 0)
+    uint32_t ld_off[J::Loads];   // in a plane (the grid has < 2^31 cells)
 #pragma unroll
-    for (int u = 0; u < NL; u++) {
-        const int q = tid + J::Threads * u, qq = q < J::Plane ? q : 0;
-        ld_off[u] = gs_wrap(x0 - S + qq % J::W, nx) + sy * gs_wrap(y0 - S + qq / J::W, ny);
+    for (int u = 0; u < J::Loads; u++) {
+        const int q = tid + J::Threads * u, qq = q < J::Plane0 ? q : 0;
+        ld_off[u] = (uint32_t)gs_wrap(x0 - S + qq % J::W0, nx) +
+                    (uint32_t)nx * (uint32_t)gs_wrap(y0 - S + qq / J::W0, ny);
     }
-    float pre[NL];
+    float pre[J::Loads];
     auto fetch = [&](int P) {
         const float *src = vin + sz * gs_wrap(min(P, z0 + tz - 1 + S), nz);
 #pragma unroll
-        for (int u = 0; u < NL; u++) pre[u] = src[ld_off[u]];
+        for (int u = 0; u < J::Loads; u++) pre[u] = src[ld_off[u]];
     };
-    auto store = [&](int Pl) {
-        float *pl = plane(0, Pl);
+    auto store = [&](int slot) {
+        float *pl = ring0 + slot * J::Plane0;
 #pragma unroll
-        for (int u = 0; u < NL; u++) {
+        for (int u = 0; u < J::Loads; u++) {
             const int q = tid + J::Threads * u;
-            if (q < J::Plane) pl[q] = pre[u];
+            if (q < J::Plane0) pl[q] = pre[u];
         }
     };
-    // inner levels: iteration it handles cell jc = tid + 256 it of the list
-    // (level 1 cells, then level 2 at S = 3); cpos = xl | yl << 8 | t << 16
-    // (t = 0: no cell) and the cell's offset in a plane of f (32-bit: the
-    // grid has < 2^31 cells)
-    int cpos[J::Iters];
-    uint32_t foff[J::Iters];
+    // the lane's column and the wave's rows 4 wave .. 4 wave + 3
+    const int row0 = 4 * wave;
+    const float px = LOS ? L.losn[0] : L.pv[x0 + lane], px2 = px * px, qx = L.cell2[0] * px2;
+    float py[4];
 #pragma unroll
-    for (int it = 0; it < J::Iters; it++) {
-        const int jc = tid + J::Threads * it;
-        int t = 1, jj = jc;
-        if (S == 3 && jc >= J::cells(1)) {
-            t = 2;
-            jj = jc - J::cells(1);
+    for (int j = 0; j < 4; j++) py[j] = LOS ? L.losn[1] : L.pv[nx + y0 + row0 + j];
+    const uint32_t f_off = (uint32_t)(x0 + lane) + sy * (uint32_t)(y0 + row0);
+    // the extra cell of level 1 (S = 2): rows -1 and TY by the first and last
+    // wave, columns -1 and 64 (rows -1 .. TY) by the second and third
+    bool ex_on = false;
+    int ex_w0 = 0, ex_w1 = 0;
+    float ex_px = 0.f, ex_py = 0.f, ex_f = 0.f;
+    uint32_t ex_foff = 0;
+    if constexpr (S == 2) {
+        int xl = lane, yl = 0;
+        if (wave == 0 || wave == J::Waves - 1) {
+            ex_on = true;
+            yl = wave == 0 ? -1 : TY;
+        } else if (wave <= 2) {
+            ex_on = lane < TY + 2;
+            xl = wave == 1 ? -1 : kJbTX;
+            yl = ex_on ? lane - 1 : 0;
         }
-        const int e = S - t, w = kJbTX + 2 * e;
-        const int yl = S - e + jj / w, xl = S - e + jj % w;
-        cpos[it] = jc < J::Inner ? (xl | (yl << 8) | (t << 16)) : (S | (S << 8));
-        foff[it] = (uint32_t)gs_wrap(x0 - S + xl, nx) + (uint32_t)nx * gs_wrap(y0 - S + yl, ny);
+        const int gx = gs_wrap(x0 + xl, nx), gy = gs_wrap(y0 + yl, ny);
+        ex_w0 = (yl + S) * J::W0 + xl + S;
+        ex_w1 = (yl + 1) * J::W1 + xl + 1;
+        ex_px = LOS ? L.losn[0] : L.pv[gx];
+        ex_py = LOS ? L.losn[1] : L.pv[nx + gy];
+        ex_foff = (uint32_t)gx + (uint32_t)nx * (uint32_t)gy;
     }
-    const uint32_t sz32 = (uint32_t)sz;
-    // level t is computed on plane Q = z0 - S + k - 2t + 1, needed on
-    // z0 - (S - t) .. z0 + tz - 1 + (S - t)
-    auto active = [&](int t, int k) { return t > 0 && k >= 3 * t - 1 && k <= tz + 2 * S + t - 2; };
-    auto fetch_f = [&](int k, float *fr) {
+    // ring slots of the planes in flight (slot = k mod 4): f and g per row
+    float fr[4][4], gr[4][4];
+    auto fetch_f = [&](int slot, int P) {   // f of plane P (the next step's level 1)
+        const float *src = f + sz * gs_wrap(min(max(P, z0 - (S - 1)), z0 + tz - 1 + (S - 1)), nz);
 #pragma unroll
-        for (int it = 0; it < J::Iters; it++) {
-            const int t = cpos[it] >> 16;
-            const uint32_t off =
-                active(t, k) ? foff[it] + sz32 * (uint32_t)gs_wrap(z0 - S + k - 2 * t + 1, nz) : 0u;
-            fr[it] = f[off];
+        for (int j = 0; j < 4; j++) fr[slot][j] = src[f_off + sy * j];
+        if constexpr (S == 2) ex_f = src[ex_on ? ex_foff : 0u];
+    };
+    // p of a plane of the tile or of its halo
+    auto pz_of = [&](int P) { return LOS ? L.losn[2] : L.pv[nx + ny + gs_wrap(P, nz)]; };
+    // the new value of a cell from its coefficients, diagonal, f, neighbour
+    // sums and value (jacobi_value's operations in its order)
+    auto update = [&](const Coef<float> &c, float D, float fv, const Nbr<float> &s, float v) {
+        float j = fv + s.A + s.B + s.C + s.X;
+        if (!LOS) j += s.G;
+        j = div_by(j, D, refined_rcp(D));
+        return (1.0f - omega) * v + omega * j;
+    };
+    // four rows of one level: from the ring planes below, at and above, row
+    // pitch W, at word w (row0 of the lane's column); level 1 (FIRST) makes
+    // the coefficients, a later level takes them from the ring
+    auto rows = [&](auto first, auto wpitch, const float *pm, const float *p0, const float *pp, int w, float pz,
+                    int slot, float (&out)[4]) {
+        constexpr bool FIRST = decltype(first)::value;
+        constexpr int W = decltype(wpitch)::value;
+        const float pz2 = pz * pz, qz = L.cell2[2] * pz2;
+        // two rows at a time (all four rows' values at once cost registers and
+        // with them a wave per SIMD); the level's start and end are kept apart
+        // from the other level's, whose loads would otherwise be hoisted
+        __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+        for (int h = 0; h < 4; h += 2) {
+            float c0[4], l0[4], r0[4], cm[4], cp[4], lm[2], rm[2], lp[2], rp[2];
+            const int wh = w + h * W;
+#pragma unroll
+            for (int j = 0; j < 4; j++) {
+                c0[j] = p0[wh + (j - 1) * W];
+                l0[j] = p0[wh + (j - 1) * W - 1];
+                r0[j] = p0[wh + (j - 1) * W + 1];
+                cm[j] = pm[wh + (j - 1) * W];
+                cp[j] = pp[wh + (j - 1) * W];
+            }
+#pragma unroll
+            for (int j = 0; j < 2; j++) {
+                lm[j] = pm[wh + j * W - 1];
+                rm[j] = pm[wh + j * W + 1];
+                lp[j] = pp[wh + j * W - 1];
+                rp[j] = pp[wh + j * W + 1];
+            }
+#pragma unroll
+            for (int j = 0; j < 2; j++) {
+                const int jr = h + j;
+                const float py2 = py[jr] * py[jr];
+                Coef<float> c;
+                c.px = px;
+                c.py = py[jr];
+                c.pz = pz;
+                if constexpr (FIRST)
+                    c.g = beta / ((qx + L.cell2[1] * py2) + qz);
+                else
+                    c.g = gr[slot][jr];
+                c.gpx2 = L.icell2[0] + c.g * px2;
+                c.gpy2 = L.icell2[1] + c.g * py2;
+                c.gpz2 = L.icell2[2] + c.g * pz2;
+                const float D = 2.0f * (c.gpx2 + c.gpy2 + c.gpz2);
+                if constexpr (FIRST) gr[slot][jr] = c.g;
+                const Nbr<float> s =
+                    nbr_of<float>(c, r0[j + 1], l0[j + 1], c0[j + 2], c0[j], cp[j + 1], cm[j + 1], r0[j + 2], l0[j],
+                                  l0[j + 2], r0[j], rp[j], lm[j], lp[j], rm[j], cp[j + 2], cm[j], cp[j], cm[j + 2]);
+                out[jr] = update(c, D, fr[slot][jr], s, c0[j + 1]);
+            }
         }
+        __builtin_amdgcn_sched_barrier(0);
     };
-    // level S: cells (ox, oy + RS j), j < CPT, of the tile: a wave takes a
-    // row, a column per lane, so its LDS reads are consecutive words
-    struct FV {
-        float v[J::CPT];
-    };
-    const int ox = tid % kJbTX, oy = tid / kJbTX;
-    const int64_t o_off = (x0 + ox) + sy * (y0 + oy);
-    auto fetch_fo = [&](int k, FV &fo) {
-        const int Q = z0 - S + k - 2 * S + 1;
-        const float *src = f + sz * (active(S, k) ? Q : z0) + o_off;
+    using True = std::integral_constant<bool, true>;
+    using False = std::integral_constant<bool, false>;
+    const int nsteps = tz + 3 * S - 1;
+    const int w0 = (row0 + S) * J::W0 + lane + S, w1 = (row0 + 1) * J::W1 + lane + 1;
+    // step k, slot SL = k mod 4 of the rings
+    auto step = [&](int k, auto slc) {
+        constexpr int SL = decltype(slc)::value, M1 = (SL + 3) & 3, M2 = (SL + 2) & 3, M3 = (SL + 1) & 3;
+        const int P = z0 - S + k;
+        if (k <= tz + 2 * S - 1) store(SL);
+        fetch(P + 1);
+        const float exf = ex_f;
+        fetch_f(SL, P);   // of this step's plane, which level 1 takes in the next step
+        __syncthreads();
+        // level 1 on plane Q = P - 1 (ring slots of P - 2, P - 1, P)
+        if (k >= 2 && k <= tz + 2 * S - 1) {
+            const float *pm = ring0 + M2 * J::Plane0, *p0 = ring0 + M1 * J::Plane0, *pp = ring0 + SL * J::Plane0;
+            const float pz = pz_of(P - 1);
+            float o[4];
+            rows(True{}, std::integral_constant<int, J::W0>{}, pm, p0, pp, w0, pz, M1, o);
+            if constexpr (S == 1) {
+                float *dst = vout + sz * (P - 1) + f_off;
 #pragma unroll
-        for (int j = 0; j < J::CPT; j++) fo.v[j] = src[sy * J::RS * j];
-    };
-    // one cell of level t from level t - 1 (local cell xl, yl, local plane ql)
-    auto cell = [&](int t, int xl, int yl, int ql, float fv) {
-        const float *pm = plane(t - 1, ql - 1), *p0 = plane(t - 1, ql), *pp = plane(t - 1, ql + 1);
-        const int wc = yl * J::W + xl;
-        const Coef<float> c = coef_p<float>(L, has_los ? L.losn[0] : ptab[xl], has_los ? L.losn[1] : ptab[J::W + yl],
-                                            has_los ? L.losn[2] : pz_tab[ql], beta);
-#define A0(o) p0[wc + (o)]
-#define AM(o) pm[wc + (o)]
-#define AP(o) pp[wc + (o)]
-        const Nbr<float> sn = nbr_of<float>(c, A0(1), A0(-1), A0(J::W), A0(-J::W), AP(0), AM(0), A0(J::W + 1),
-                                            A0(-J::W - 1), A0(J::W - 1), A0(-J::W + 1), AP(1), AM(-1), AP(-1),
-                                            AM(1), AP(J::W), AM(-J::W), AP(-J::W), AM(J::W));
-        const float v = jacobi_value(c, fv, sn, A0(0), omega, has_los);
+                for (int j = 0; j < 4; j++) dst[sy * j] = o[j];
+            } else {
+                float *pl = ring1 + M1 * J::Plane1;
+#pragma unroll
+                for (int j = 0; j < 4; j++) pl[w1 + j * J::W1] = o[j];
+                if (ex_on) {
+                    const Coef<float> c = coef_p<float>(L, ex_px, ex_py, pz, beta);
+                    const float D = 2.0f * (c.gpx2 + c.gpy2 + c.gpz2);
+#define A0(q) p0[ex_w0 + (q)]
+#define AM(q) pm[ex_w0 + (q)]
+#define AP(q) pp[ex_w0 + (q)]
+                    const Nbr<float> s = nbr_of<float>(
+                        c, A0(1), A0(-1), A0(J::W0), A0(-J::W0), AP(0), AM(0), A0(J::W0 + 1), A0(-J::W0 - 1),
+                        A0(J::W0 - 1), A0(-J::W0 + 1), AP(1), AM(-1), AP(-1), AM(1), AP(J::W0), AM(-J::W0),
+                        AP(-J::W0), AM(J::W0));
+                    pl[ex_w1] = update(c, D, exf, s, A0(0));
 #undef A0
 #undef AM
 #undef AP
-        return v;
-    };
-
-    auto step = [&](int k, const float *fcur, float *fnext, const FV &focur, FV &fonext) {
-        if (k <= tz + 2 * S - 1) store(k);
-        fetch(z0 - S + k + 1);
-        fetch_f(k + 1, fnext);
-        fetch_fo(k + 1, fonext);
-        __syncthreads();
-#pragma unroll
-        for (int it = 0; it < J::Iters; it++) {
-            const int t = cpos[it] >> 16;
-            if (!active(t, k)) continue;
-            const int xl = cpos[it] & 255, yl = (cpos[it] >> 8) & 255, ql = k - 2 * t + 1;
-            plane(t, ql)[yl * J::W + xl] = cell(t, xl, yl, ql, fcur[it]);
+                }
+            }
         }
-        if (active(S, k)) {
-            const int ql = k - 2 * S + 1;
-            float *dst = vout + sz * (z0 - S + ql) + o_off;
+        if constexpr (S == 2) {
+            // level 2 on plane P - 3 (ring slots of P - 4, P - 3, P - 2)
+            if (k >= 5 && k <= tz + 4) {
+                const float *pm = ring1 + SL * J::Plane1, *p0 = ring1 + M3 * J::Plane1, *pp = ring1 + M2 * J::Plane1;
+                float o[4];
+                rows(False{}, std::integral_constant<int, J::W1>{}, pm, p0, pp, w1, pz_of(P - 3), M3, o);
+                float *dst = vout + sz * (P - 3) + f_off;
 #pragma unroll
-            for (int j = 0; j < J::CPT; j++) dst[sy * J::RS * j] = cell(S, S + ox, S + oy + J::RS * j, ql, focur.v[j]);
+                for (int j = 0; j < 4; j++) dst[sy * j] = o[j];
+            }
         }
     };
-
-    float fa[J::Iters], fb[J::Iters];
-    FV foa, fob;
     fetch(z0 - S);
-    fetch_f(0, fa);
-    fetch_fo(0, foa);
-    const int nsteps = tz + 3 * S - 1;
-    int k = 0;
-    for (; k + 1 < nsteps; k += 2) {   // the f buffers alternate
-        step(k, fa, fb, foa, fob);
-        step(k + 1, fb, fa, fob, foa);
+    for (int k = 0; k < nsteps; k += 4) {
+        step(k, std::integral_constant<int, 0>{});
+        if (k + 1 < nsteps) step(k + 1, std::integral_constant<int, 1>{});
+        if (k + 2 < nsteps) step(k + 2, std::integral_constant<int, 2>{});
+        if (k + 3 < nsteps) step(k + 3, std::integral_constant<int, 3>{});
     }
-    if (k < nsteps) step(k, fa, fb, foa, fob);
 }
 
 // One FP64 refinement pass of the RBGS solve (z-marching, LDS ring):
@@ -1761,30 +1841,29 @@ hipError_t launch_mg_gs4(float *vout, const float *vin, const float *f, const MG
     return hipGetLastError();
 }
 
-// z planes per workgroup of k_mg_jacobi_tb<S> (tz + 3 S - 1 steps)
 template <int S>
-static int jacobi_tb_tz(const MGLevel &L) {
-    static const int per_cu = blocks_per_cu(k_mg_jacobi_tb<S, 0>, JbShape<S>::Threads);
-    return zm_tz((int64_t)(L.n[0] / kJbTX) * (L.n[1] / kJbTY), L.n[2], kJbMaxTz, 8, per_cu, 3 * S - 1);
+static hipError_t jacobi_zm(float *vout, const float *vin, const float *f, const MGLevel &L, float beta, float omega,
+                            int has_los, hipStream_t s) {
+    using J = JbShape<S>;
+    // z planes per workgroup (tz + 3 S - 1 steps)
+    static const int per_cu = blocks_per_cu(k_mg_jacobi_zm<S, 0>, J::Threads);
+    const int tz = zm_tz((int64_t)(L.n[0] / kJbTX) * (L.n[1] / J::TY), L.n[2], kJbMaxTz, 8, per_cu, 3 * S - 1);
+    const dim3 grid((unsigned)(L.n[0] / kJbTX), (unsigned)(L.n[1] / J::TY), (unsigned)(L.n[2] / tz));
+    hipLaunchKernelGGL((has_los ? k_mg_jacobi_zm<S, 1> : k_mg_jacobi_zm<S, 0>), grid, dim3(J::Threads), 0, s, vout,
+                       vin, f, L, beta, omega, tz);
+    return hipGetLastError();
 }
 
 bool mg_jacobi_tb_ok(const MGLevel &L) {
-    return L.n[0] % kJbTX == 0 && L.n[1] % kJbTY == 0 && L.n[2] % 8 == 0 && L.n[2] >= 8 &&
+    return L.n[0] % kJbTX == 0 && L.n[1] % JbShape<1>::TY == 0 && L.n[2] % 8 == 0 && L.n[2] >= 8 &&
            (int64_t)L.n[0] * L.n[1] * L.n[2] < ((int64_t)1 << 31);
 }
 
 hipError_t launch_mg_jacobi_tb(float *vout, const float *vin, const float *f, const MGLevel &L, float beta,
                                float omega, int has_los, int sweeps, hipStream_t s) {
-    if (!mg_jacobi_tb_ok(L) || vout == vin || (sweeps != 2 && sweeps != 3)) return hipErrorInvalidValue;
-    const int tz = sweeps == 2 ? jacobi_tb_tz<2>(L) : jacobi_tb_tz<3>(L);
-    const dim3 grid((unsigned)(L.n[0] / kJbTX), (unsigned)(L.n[1] / kJbTY), (unsigned)(L.n[2] / tz));
-    if (sweeps == 2)
-        hipLaunchKernelGGL((has_los ? k_mg_jacobi_tb<2, 1> : k_mg_jacobi_tb<2, 0>), grid, dim3(JbShape<2>::Threads), 0,
-                           s, vout, vin, f, L, beta, omega, tz);
-    else
-        hipLaunchKernelGGL((has_los ? k_mg_jacobi_tb<3, 1> : k_mg_jacobi_tb<3, 0>), grid, dim3(JbShape<3>::Threads), 0,
-                           s, vout, vin, f, L, beta, omega, tz);
-    return hipGetLastError();
+    if (!mg_jacobi_tb_ok(L) || vout == vin || (sweeps != 1 && sweeps != 2)) return hipErrorInvalidValue;
+    return sweeps == 1 ? jacobi_zm<1>(vout, vin, f, L, beta, omega, has_los, s)
+                       : jacobi_zm<2>(vout, vin, f, L, beta, omega, has_los, s);
 }
 
 int64_t mg_refine_blocks(const MGLevel &L) {

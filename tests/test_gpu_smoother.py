@@ -85,6 +85,30 @@ def test_blocked_jacobi_bitwise_single_sweeps(ctx, shape, los, sweeps):
     np.testing.assert_array_equal(got, exp)
 
 
+@pytest.mark.parametrize("shape,los,sweeps", [
+    ((128, 128, 128), None, 1),
+    ((8, 16, 16384), None, 2),
+    ((2048, 16, 64), [0.3, -0.4, 0.866], 2),
+    ((72, 208, 192), None, 5),
+])
+def test_zmarching_jacobi_matches_oracle(ctx, shape, los, sweeps):
+    """The z-marching Jacobi launches (one and two sweeps) on grids whose
+    tiles' halos wrap onto themselves in y or z, odd numbers of tiles
+    included, against the FP32 oracle's sweeps (jacobi!, src/multigrid.jl:
+    193-210): the same operations in the same order, so at most the rounding
+    of one update (a few 1e-7 of the largest value) per sweep apart."""
+    v, f = fields(shape, 11 + sweeps)
+    rec = recon(shape, los, ctx)
+    rec.jacobi_niterations = sweeps
+    o = orc.MultigridRecon(bias=2.0, f=0.8, smoothing_radius=15.0, box_size=rec.box_size, box_min=rec.box_min,
+                           los=los)
+    got = bh.jacobi_(v.copy(), f, rec)
+    exp = orc.mg_jacobi(v.copy(), f, o.box_size, o.box_min, o.beta, 0.4, sweeps, los=o.los)
+    err = float(np.max(np.abs(got - exp)) / np.abs(exp).max())
+    print(f"{shape} los {los} x{sweeps}: max |diff| / max |v| {err:.1e}")
+    assert err < 5e-7 * sweeps
+
+
 @pytest.mark.parametrize("shape,los", [((128, 128, 128), None), ((64, 64, 512), [0.0, 0.0, 1.0]),
                                        ((32, 256, 256), [0.6, 0.0, 0.8])])
 def test_zmarching_residual_and_prolongation_match_oracle(ctx, shape, los):
