@@ -794,7 +794,8 @@ struct MGPyr {
     std::vector<int> cur;              // 0: A holds v, 1: B holds v
     std::vector<int> dbl;
     std::vector<int> zero;             // 1: v is zero and not stored (its next fused sweep reads none)
-    int lc = 0;                        // levels >= lc run in one k_mg_coarse launch
+    int lc = 0;                        // levels >= lc run in one k_mg_coarse or k_mg_small launch
+    bool small = false;                // k_mg_small: levels >= lc stay in LDS
 };
 
 // Levels of at most this many cells are latency-bound: they run inside one
@@ -803,6 +804,17 @@ constexpr int64_t kMGCoarseCells = 512;
 
 bool mg_recurse(const Grid &G) {
     return G.nx > 4 && G.nx % 2 == 0 && G.ny > 4 && G.ny % 2 == 0 && G.nz > 4 && G.nz % 2 == 0;
+}
+
+// Levels [l0, nl) of P as k_mg_small takes them.
+MGSmall mg_small_args(const MGPyr &P, int l0) {
+    MGSmall a{};
+    a.nl = (int)P.g.size() - l0;
+    for (int i = 0; i < a.nl && i < kMGSmallLevels; i++) {
+        a.L[i] = P.L[l0 + i];
+        a.dbl[i] = P.dbl[l0 + i];
+    }
+    return a;
 }
 
 MGPyr mg_build(baorec_ctx *c, const Grid &G0, const baorec_params *p, Slot *slot, float *v0,
@@ -871,6 +883,14 @@ MGPyr mg_build(baorec_ctx *c, const Grid &G0, const baorec_params *p, Slot *slot
     for (int i = nl - 1; i >= 0; i--) {
         if (P.g[i].R() > kMGCoarseCells || P.dbl[i] != P.dbl[nl - 1] || nl - i > kMGCoarseLevels) break;
         P.lc = i;
+    }
+    // first level from which the levels fit one workgroup's LDS
+    for (int i = std::max(0, nl - kMGSmallLevels); i < nl; i++) {
+        MGSmall a = mg_small_args(P, i);
+        if (!mg_small_layout(a)) continue;
+        P.lc = i;
+        P.small = true;
+        break;
     }
     return P;
 }
@@ -951,6 +971,27 @@ void mg_coarse(baorec_ctx *c, MGPyr &P, const baorec_params *p, int fmg, int gs)
     // number (pre + post), so P.cur is unchanged
 }
 
+// Levels [P.lc, nl) as one k_mg_small launch, as mg_coarse (zero: v of level
+// lc is zero and not stored).
+void mg_small(baorec_ctx *c, MGPyr &P, const baorec_params *p, int fmg, int gs, bool zero) {
+    const int l = P.lc;
+    MGSmall a = mg_small_args(P, l);
+    void *const v = P.dbl[l] ? static_cast<void *>(vcurd(P, l)) : static_cast<void *>(vcur(P, l));
+    a.f = P.dbl[l] ? static_cast<const void *>(P.Fd[l]) : static_cast<const void *>(P.F[l]);
+    a.vin = zero || fmg ? nullptr : v;
+    a.vout = v;
+    a.fmg = fmg;
+    a.gs = gs;
+    a.beta = p->beta;
+    a.omega = p->jacobi_damping_factor;
+    a.has_los = p->has_los;
+    a.jacobi_n = p->jacobi_niterations;
+    a.rb_sweeps = p->rb_sweeps;
+    a.vcycles = p->vcycle_niterations;
+    ProfScope ps(c, "mg_small", 0.0);
+    hipchk(c, launch_mg_small(a, c->stream), "mg small levels");
+}
+
 // The FP32 residual of level l restricted to the right-hand side of level
 // l + 1 (residual! + reduce!, src/multigrid.jl:378-395, 641-651): on grids of
 // >= 128^3 cells one fused pass with the same bits (the residual is not
@@ -981,8 +1022,14 @@ static void mg_residual_reduce(baorec_ctx *c, MGPyr &P, int l, const baorec_para
         hipchk(c, launch_mg_reduce_t<double, float>(P.Fd[l + 1], r, fn, c->stream), "reduce");
 }
 
-// vcycle! (src/multigrid.jl:689-719), reference schedule, FP32
-void mg_vcycle_ref(baorec_ctx *c, MGPyr &P, int l, const baorec_params *p) {
+// vcycle! (src/multigrid.jl:689-719), reference schedule, FP32.  zero: v of
+// level l is zero (and not stored yet)
+void mg_vcycle_ref(baorec_ctx *c, MGPyr &P, int l, const baorec_params *p, bool zero = false) {
+    if (l == P.lc && P.small) {
+        mg_small(c, P, p, 0, 0, zero);
+        return;
+    }
+    if (zero) zero_level(c, P, l);
     if (l == P.lc) {
         mg_coarse<float>(c, P, p, 0, 0);
         return;
@@ -990,8 +1037,7 @@ void mg_vcycle_ref(baorec_ctx *c, MGPyr &P, int l, const baorec_params *p) {
     mg_jacobi_n(c, P, l, p, p->jacobi_niterations);
     if (l + 1 < (int)P.g.size()) {
         mg_residual_reduce(c, P, l, p, P.F[l + 1]);
-        zero_level(c, P, l + 1);
-        mg_vcycle_ref(c, P, l + 1, p);
+        mg_vcycle_ref(c, P, l + 1, p, true);
         const int cn[3] = {P.g[l + 1].nx, P.g[l + 1].ny, P.g[l + 1].nz};
         {
             ProfScope ps(c, "mg_prolong", 8.5 * P.g[l].R());
@@ -1004,7 +1050,10 @@ void mg_vcycle_ref(baorec_ctx *c, MGPyr &P, int l, const baorec_params *p) {
 // fmg (src/multigrid.jl:722-752), reference schedule
 void mg_fmg_ref(baorec_ctx *c, MGPyr &P, int l, const baorec_params *p) {
     if (l == P.lc) {
-        mg_coarse<float>(c, P, p, 1, 0);
+        if (P.small)
+            mg_small(c, P, p, 1, 0, true);
+        else
+            mg_coarse<float>(c, P, p, 1, 0);
         return;
     }
     if (l + 1 < (int)P.g.size()) {
@@ -1025,11 +1074,19 @@ void mg_fmg_ref(baorec_ctx *c, MGPyr &P, int l, const baorec_params *p) {
 static bool mg_use_gs4(const MGPyr &P, int l) {
     return !P.dbl[l] && mg_gs4_ok(P.L[l]) && P.g[l].R() >= ((int64_t)1 << 21);
 }
+// smaller FP32 levels: a whole sweep per launch by 8^3 tiles (6.0 us at 64^3 and
+// 5.3 us at 32^3, where the four colour launches take 13.2 us)
+static bool mg_use_gs_tile(const MGPyr &P, int l) {
+    return !P.dbl[l] && !mg_use_gs4(P, l) && mg_gs_tile_ok(P.L[l]) && P.g[l].R() < ((int64_t)1 << 21) &&
+           (((uintptr_t)P.A[l] | (uintptr_t)P.B[l]) & 15) == 0;
+}
 
-// v = 0 on level l before an RBGS V-cycle: on levels of fused sweeps no
-// fill, the first sweep reads no v (mg_smooth_rb); otherwise zero_level.
+// v = 0 on level l before an RBGS V-cycle: on levels of whole sweeps per
+// launch no fill, the first sweep reads no v (mg_smooth_rb), and the levels
+// in LDS start from zero by themselves; otherwise zero_level.
 void zero_level_rb(baorec_ctx *c, MGPyr &P, int l) {
-    if (l != P.lc && mg_use_gs4(P, l))
+    if (l == P.lc && P.small) return;
+    if (l != P.lc && (mg_use_gs4(P, l) || mg_use_gs_tile(P, l)))
         P.zero[l] = 1;
     else
         zero_level(c, P, l);
@@ -1039,12 +1096,18 @@ void zero_level_rb(baorec_ctx *c, MGPyr &P, int l) {
 // per-workgroup sums of the result there (mg_gs4_blocks partials).  Leaves
 // v stored (P.zero[l] cleared).
 void mg_smooth_rb(baorec_ctx *c, MGPyr &P, int l, const baorec_params *p, int sweeps, double *sum_part = nullptr) {
-    if (mg_use_gs4(P, l)) {
+    const bool tile = mg_use_gs_tile(P, l);
+    if (tile || mg_use_gs4(P, l)) {
         for (int s = 0; s < sweeps; s++) {
-            ProfScope ps(c, "mg_gs4", (P.zero[l] ? 8.0 : 12.0) * P.g[l].R());
-            hipchk(c, launch_mg_gs4(vother(P, l), P.zero[l] ? nullptr : vcur(P, l), P.F[l], P.L[l], p->beta,
+            ProfScope ps(c, tile ? "mg_gs_tile" : "mg_gs4", (P.zero[l] ? 8.0 : 12.0) * P.g[l].R());
+            if (tile)
+                hipchk(c, launch_mg_gs_tile(vother(P, l), P.zero[l] ? nullptr : vcur(P, l), P.F[l], P.L[l], p->beta,
+                                            p->has_los, c->stream),
+                       "gs tile");
+            else
+                hipchk(c, launch_mg_gs4(vother(P, l), P.zero[l] ? nullptr : vcur(P, l), P.F[l], P.L[l], p->beta,
                                     p->has_los, c->stream, s + 1 == sweeps ? sum_part : nullptr),
-                   "gs4");
+                       "gs4");
             P.cur[l] ^= 1;
             P.zero[l] = 0;
         }
@@ -1071,7 +1134,9 @@ void mg_smooth_rb(baorec_ctx *c, MGPyr &P, int l, const baorec_params *p, int sw
 // sum_part: as mg_smooth_rb's, for the post-smoothing of level l
 void mg_vcycle_rb(baorec_ctx *c, MGPyr &P, int l, const baorec_params *p, double *sum_part = nullptr) {
     if (l == P.lc) {
-        if (P.dbl[l])
+        if (P.small)
+            mg_small(c, P, p, 0, 1, true);
+        else if (P.dbl[l])
             mg_coarse<double>(c, P, p, 0, 1);
         else
             mg_coarse<float>(c, P, p, 0, 1);

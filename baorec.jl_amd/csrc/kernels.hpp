@@ -307,6 +307,29 @@ struct MGCoarse {
 template <typename T>
 hipError_t launch_mg_coarse(const MGCoarse<T> &a, hipStream_t s);
 
+// The same for levels [0, nl) of at most kMGSmallCells cells with power-of-two
+// sides, kept in the LDS of one workgroup (mg_small_layout says whether they
+// fit and fills lg and the offsets); with gs, levels may be FP32 above and FP64
+// below.  f and vin (NULL: zero) are level 0's, vout receives its v; types by
+// dbl[0].
+constexpr int kMGSmallLevels = 5;
+constexpr int64_t kMGSmallCells = 4096;
+struct MGSmall {
+    int nl;
+    MGLevel L[kMGSmallLevels];
+    int dbl[kMGSmallLevels];
+    int lg[kMGSmallLevels][3];   // log2 of the sides
+    int off_v[kMGSmallLevels], off_f[kMGSmallLevels], off_r[kMGSmallLevels],
+        off_p[kMGSmallLevels];   // bytes
+    const void *f, *vin;
+    void *vout;
+    int fmg, gs;
+    float beta, omega;
+    int has_los, jacobi_n, rb_sweeps, vcycles;
+};
+bool mg_small_layout(MGSmall &a);
+hipError_t launch_mg_small(const MGSmall &a, hipStream_t s);
+
 hipError_t launch_mg_jacobi(float *vout, const float *vin, const float *f, const MGLevel &L,
                             float beta, float omega, int has_los, hipStream_t s);
 hipError_t launch_mg_residual(float *r, const float *v, const float *f, const MGLevel &L,
@@ -345,6 +368,11 @@ bool mg_gs4_ok(const MGLevel &L);
 int64_t mg_gs4_blocks(const MGLevel &L);
 hipError_t launch_mg_gs4(float *vout, const float *vin, const float *f, const MGLevel &L, float beta, int has_los,
                          hipStream_t s, double *part = nullptr);
+// The same on small levels (sides multiples of 8, 16-byte aligned arrays), by
+// 8^3 tiles.
+bool mg_gs_tile_ok(const MGLevel &L);
+hipError_t launch_mg_gs_tile(float *vout, const float *vin, const float *f, const MGLevel &L, float beta, int has_los,
+                             hipStream_t s);
 template <typename T>
 hipError_t launch_mg_residual_t(T *r, const T *v, const T *f, const MGLevel &L, float beta,
                                 int has_los, hipStream_t s);

@@ -184,9 +184,9 @@ __device__ __forceinline__ GsCoef<T> gs_coef_p(const MGLevel &L, T px, T py, T p
                       beta);
 }
 
-// the new value from f and the 18 neighbour values (argument order of nbr_of)
+// f + neighbour sums from f and the 18 neighbour values (argument order of nbr_of)
 template <typename T>
-__device__ __forceinline__ T gs_update(const GsCoef<T> &c, T f, T vxp, T vxm, T vyp, T vym, T vzp, T vzm, T xpyp,
+__device__ __forceinline__ T gs_sum(const GsCoef<T> &c, T f, T vxp, T vxm, T vyp, T vym, T vzp, T vzm, T xpyp,
                                        T xmym, T xmyp, T xpym, T xpzp, T xmzm, T xmzp, T xpzm, T ypzp, T ymzm, T ymzp,
                                        T ypzm, int has_los) {
     T j = mg_fma(c.gz, vzp + vzm, mg_fma(c.gy, vyp + vym, mg_fma(c.gx, vxp + vxm, f)));
@@ -195,6 +195,15 @@ __device__ __forceinline__ T gs_update(const GsCoef<T> &c, T f, T vxp, T vxm, T 
     const T x = mg_fma(c.py * c.pz, eyz, mg_fma(c.px * c.pz, exz, (c.px * c.py) * exy));
     j = mg_fma((T)0.5 * c.g, x, j);
     if (!has_los) j = mg_fma(c.g, mg_fma(c.pz, vzp - vzm, mg_fma(c.py, vyp - vym, c.px * (vxp - vxm))), j);
+    return j;
+}
+// the new value
+template <typename T>
+__device__ __forceinline__ T gs_update(const GsCoef<T> &c, T f, T vxp, T vxm, T vyp, T vym, T vzp, T vzm, T xpyp,
+                                       T xmym, T xmyp, T xpym, T xpzp, T xmzm, T xmzp, T xpzm, T ypzp, T ymzm, T ymzp,
+                                       T ypzm, int has_los) {
+    const T j = gs_sum<T>(c, f, vxp, vxm, vyp, vym, vzp, vzm, xpyp, xmym, xmyp, xpym, xpzp, xmzm, xmzp, xpzm, ypzp,
+                          ymzm, ymzp, ypzm, has_los);
     return mg_div<T, true>(j, (T)2 * ((c.gx + c.gy) + c.gz));
 }
 
@@ -599,6 +608,96 @@ __global__ void __launch_bounds__(kGsThreads) k_mg_gs4(float *__restrict__ vout,
             for (int w = 0; w < kGsThreads / 64; w++) t += red[w];
             part[tile] = t;
         }
+    }
+}
+
+// One whole 4-colour Gauss-Seidel sweep of a small FP32 level in one launch,
+// out of place: vout holds what the four in-place colour passes of k_mg_mcgs
+// leave in v (the same cell arithmetic on the same values, so the same bits).
+// A workgroup owns an 8^3 tile: it loads the tile with a halo of 4 (16^3
+// values, 16 KB of LDS) and updates colour s = 0..3 on the tile grown by 3 - s,
+// with a barrier between colours (2.9 updates per cell, the halo's repeated by
+// the neighbours).  On levels below 128^3 the four colour launches are bound
+// by launch latency, not by their work: 13.2 us per sweep at 64^3 and at 32^3;
+// this one 6.0 and 5.3 us, bound by its own four barrier phases.
+// ZIN: the sweep starts from v = 0 and reads no v.
+constexpr int kGbT = 8, kGbH = 4, kGbN = kGbT + 2 * kGbH, kGbThreads = 512;
+constexpr int kGbP = 20, kGbPlane = kGbP * kGbN;   // LDS row: even x (8 words), odd x (8), 4 spare
+constexpr int kGbRounds = 5;                       // cells per thread: stage 0 twice, stages 1..3 once
+
+template <int LOS, int ZIN>
+__global__ void __launch_bounds__(kGbThreads) k_mg_gs_tile(float *__restrict__ vout, const float *__restrict__ vin,
+                                                           const float *__restrict__ f, MGLevel L, float beta) {
+    __shared__ __align__(16) float lds[kGbPlane * kGbN];
+    __shared__ float ptab[3 * kGbN];
+    const int nx = L.n[0], ny = L.n[1], nz = L.n[2];
+    const int x0 = blockIdx.x * kGbT, y0 = blockIdx.y * kGbT, z0 = blockIdx.z * kGbT;
+    const int tid = threadIdx.x;
+    // the tile and its halo in float4 chunks (rows of 16: 4 chunks)
+    float4 pre[2];
+#pragma unroll
+    for (int u = 0; u < 2; u++) {
+        const int q = tid + kGbThreads * u, j = q & 3, row = (q >> 2) & 15, pl = q >> 6;
+        if constexpr (ZIN) {
+            pre[u] = make_float4(0.f, 0.f, 0.f, 0.f);
+        } else {
+            const int gx = gs_wrap(x0 - kGbH + 4 * j, nx), gy = gs_wrap(y0 - kGbH + row, ny),
+                      gz = gs_wrap(z0 - kGbH + pl, nz);
+            pre[u] = *reinterpret_cast<const float4 *>(vin + gx + (int64_t)nx * (gy + (int64_t)ny * gz));
+        }
+    }
+    // the thread's cells: local x, y, z and f
+    int word[kGbRounds], pos[kGbRounds];
+    float fv[kGbRounds];
+#pragma unroll
+    for (int r = 0; r < kGbRounds; r++) {
+        const int s = r < 2 ? 0 : r - 1, n = 7 - s, lo = 1 + s;
+        const int idx = r == 1 ? tid + kGbThreads : tid;
+        const bool on = idx < 2 * n * n * n;
+        const int c = on ? idx : 0;
+        const int i = c % n, j = (c / n) % n, z = lo + c / (n * n);
+        const int y = lo + 2 * j + ((lo + z + (s >> 1)) & 1), x = lo + 2 * i + ((lo + y + (s & 1)) & 1);
+        word[r] = on ? z * kGbPlane + y * kGbP + (x & 1) * 8 + (x >> 1) : -1;
+        pos[r] = x | (y << 8) | (z << 16);
+        const int gx = gs_wrap(x0 - kGbH + x, nx), gy = gs_wrap(y0 - kGbH + y, ny), gz = gs_wrap(z0 - kGbH + z, nz);
+        fv[r] = f[gx + (int64_t)nx * (gy + (int64_t)ny * gz)];
+    }
+    if (!LOS && tid < 3 * kGbN) {
+        const int a = tid / kGbN, k = tid % kGbN;
+        ptab[tid] = L.pv[a == 0 ? gs_wrap(x0 - kGbH + k, nx)
+                                : (a == 1 ? nx + gs_wrap(y0 - kGbH + k, ny) : nx + ny + gs_wrap(z0 - kGbH + k, nz))];
+    }
+#pragma unroll
+    for (int u = 0; u < 2; u++) {
+        const int q = tid + kGbThreads * u, j = q & 3, row = (q >> 2) & 15, pl = q >> 6;
+        float *d = lds + pl * kGbPlane + row * kGbP + 2 * j;
+        d[0] = pre[u].x;
+        d[1] = pre[u].z;
+        d[8] = pre[u].y;
+        d[9] = pre[u].w;
+    }
+    __syncthreads();
+#pragma unroll
+    for (int r = 0; r < kGbRounds; r++) {
+        if (r >= 2) __syncthreads();   // the colour before is complete
+        if (word[r] < 0) continue;
+        const int x = pos[r] & 255, y = (pos[r] >> 8) & 255, z = pos[r] >> 16;
+        const GsCoef<float> c = LOS ? gs_coef_p<float>(L, L.losn[0], L.losn[1], L.losn[2], beta)
+                                    : gs_coef_p<float>(L, ptab[x], ptab[kGbN + y], ptab[2 * kGbN + z], beta);
+        // x - 1 and x + 1 sit in the other half of the row, at words ob and ob + 1
+        float *a0 = lds + word[r];
+        const float *b0 = a0 + ((x & 1) ? -8 : 7);
+        a0[0] = gs_update<float>(
+            c, fv[r], b0[1], b0[0], a0[kGbP], a0[-kGbP], a0[kGbPlane], a0[-kGbPlane], b0[kGbP + 1], b0[-kGbP], b0[kGbP],
+            b0[-kGbP + 1], b0[kGbPlane + 1], b0[-kGbPlane], b0[kGbPlane], b0[-kGbPlane + 1], a0[kGbPlane + kGbP],
+            a0[-kGbPlane - kGbP], a0[kGbPlane - kGbP], a0[-kGbPlane + kGbP], LOS);
+    }
+    __syncthreads();
+    if (tid < kGbT * kGbT * 2) {   // the tile's rows of 8 as two float4
+        const int h = tid & 1, row = (tid >> 1) & 7, pl = tid >> 4;
+        const float *d = lds + (kGbH + pl) * kGbPlane + (kGbH + row) * kGbP + 2 + 2 * h;
+        *reinterpret_cast<float4 *>(vout + x0 + 4 * h + (int64_t)nx * (y0 + row + (int64_t)ny * (z0 + pl))) =
+            make_float4(d[0], d[8], d[1], d[9]);
     }
 }
 
@@ -1577,6 +1676,467 @@ __global__ void __launch_bounds__(1024) k_mg_coarse(MGCoarse<T> a) {
     }
 }
 
+// ------------------------------------------------------------ coarse levels in LDS
+//
+// The levels of at most kMGSmallCells cells with power-of-two sides in one
+// 1024-thread workgroup that keeps them in LDS: one V-cycle from the top one
+// (gs: four-colour Gauss-Seidel, FP32 and FP64 levels mixed; else damped
+// Jacobi, FP32) or the whole FMG (fmg), the per-cell arithmetic and the order
+// of k_mg_coarse.  These levels are bound by latency: through k_mg_coarse every
+// stage is a round trip to the L2 and levels above 512 cells a launch per
+// stage.  Every address is an index into `pool` from masked coordinates; the
+// host checks that the levels' arrays fit (mg_small_layout).  What remains is
+// the coarsest FP64 level's serial colour passes (256 per V-cycle).  Measured
+// for 16^3 (FP32) | 8^3 | 4^3 (FP64): 71 us per V-cycle, against 138 us in
+// k_mg_coarse for the lower two alone and eight launches for 16^3; the Jacobi
+// levels 16^3 .. 4^3 of a reference V-cycle 58 us.
+constexpr int kMGSmallPool = 120 * 1024;   // bytes
+
+template <typename T>
+struct LdsLevel {
+    T *v, *f, *r;        // value, right-hand side, residual / second Jacobi buffer
+    const T *p;          // LOS component in cell units of each x | y | z (as coef)
+    int lx, ly, lz, n;   // log2 of the sides, cells
+    __device__ __forceinline__ T px(const MGLevel &L, int x, int los) const { return los ? (T)L.losn[0] : p[x]; }
+    __device__ __forceinline__ T py(const MGLevel &L, int y, int los) const {
+        return los ? (T)L.losn[1] : p[(1 << lx) + y];
+    }
+    __device__ __forceinline__ T pz(const MGLevel &L, int z, int los) const {
+        return los ? (T)L.losn[2] : p[(1 << lx) + (1 << ly) + z];
+    }
+};
+// a cell's coefficients (gs_coef_at, coef) from the level's table
+template <typename T>
+__device__ __forceinline__ GsCoef<T> small_gs_coef(const LdsLevel<T> &l, const MGLevel &L, int x, int y, int z,
+                                                   float beta, int has_los) {
+    return gs_coef_p<T>(L, l.px(L, x, has_los), l.py(L, y, has_los), l.pz(L, z, has_los), (T)beta);
+}
+template <typename T>
+__device__ __forceinline__ Coef<T> small_coef(const LdsLevel<T> &l, const MGLevel &L, int x, int y, int z, float beta,
+                                              int has_los) {
+    return coef_p<T>(L, l.px(L, x, has_los), l.py(L, y, has_los), l.pz(L, z, has_los), (T)beta);
+}
+
+__device__ __forceinline__ void small_xyz(int c, int lx, int ly, int &x, int &y, int &z) {
+    x = c & ((1 << lx) - 1);
+    y = (c >> lx) & ((1 << ly) - 1);
+    z = c >> (lx + ly);
+}
+
+// the neighbour offsets of a cell of a periodic power-of-two grid
+struct SmallNbr {
+    int xm, xp, ym, yp, zm, zp, x, y, z;   // words of each coordinate
+    __device__ __forceinline__ SmallNbr(int cx, int cy, int cz, int lx, int ly, int lz) {
+        const int mx = (1 << lx) - 1, my = (1 << ly) - 1, mz = (1 << lz) - 1;
+        x = cx;
+        xm = (cx - 1) & mx;
+        xp = (cx + 1) & mx;
+        y = cy << lx;
+        ym = ((cy - 1) & my) << lx;
+        yp = ((cy + 1) & my) << lx;
+        z = cz << (lx + ly);
+        zm = ((cz - 1) & mz) << (lx + ly);
+        zp = ((cz + 1) & mz) << (lx + ly);
+    }
+};
+// the 18 neighbour values in the argument order of nbr_of and gs_update
+#define SMALL_NBRS(v, o)                                                                                      \
+    (v)[(o).xp + (o).y + (o).z], (v)[(o).xm + (o).y + (o).z], (v)[(o).x + (o).yp + (o).z],                    \
+        (v)[(o).x + (o).ym + (o).z], (v)[(o).x + (o).y + (o).zp], (v)[(o).x + (o).y + (o).zm],                \
+        (v)[(o).xp + (o).yp + (o).z], (v)[(o).xm + (o).ym + (o).z], (v)[(o).xm + (o).yp + (o).z],             \
+        (v)[(o).xp + (o).ym + (o).z], (v)[(o).xp + (o).y + (o).zp], (v)[(o).xm + (o).y + (o).zm],             \
+        (v)[(o).xm + (o).y + (o).zp], (v)[(o).xp + (o).y + (o).zm], (v)[(o).x + (o).yp + (o).zp],             \
+        (v)[(o).x + (o).ym + (o).zm], (v)[(o).x + (o).ym + (o).zp], (v)[(o).x + (o).yp + (o).zm]
+
+// A cell's part of gs_update that does not change from pass to pass.
+template <typename T>
+struct SmallCell {
+    GsCoef<T> k;
+    T rD;   // reciprocal of the diagonal (FP32: mg_div's v_rcp_f32)
+    int me;
+    __device__ __forceinline__ void set(const LdsLevel<T> &l, const MGLevel &L, const SmallNbr &o, int x, int y, int z,
+                                        float beta, int has_los) {
+        k = small_gs_coef<T>(l, L, x, y, z, beta, has_los);
+        rD = mg_div<T, true>((T)1, (T)2 * ((k.gx + k.gy) + k.gz));
+        me = o.x + o.y + o.z;
+    }
+    // gs_update without its division
+    __device__ __forceinline__ T update(T f, T vxp, T vxm, T vyp, T vym, T vzp, T vzm, T xpyp, T xmym, T xmyp, T xpym,
+                                        T xpzp, T xmzm, T xmzp, T xpzm, T ypzp, T ymzm, T ymzp, T ypzm,
+                                        int has_los) const {
+        return gs_sum<T>(k, f, vxp, vxm, vyp, vym, vzp, vzm, xpyp, xmym, xmyp, xpym, xpzp, xmzm, xmzp, xpzm, ypzp, ymzm,
+                         ymzp, ypzm, has_los) * rD;
+    }
+};
+
+// cell c (of n / 4) of a colour
+__device__ __forceinline__ void small_colour_xyz(int c, int col, int lx, int ly, int &x, int &y, int &z) {
+    const int hx = lx - 1, hy = ly - 1;
+    z = c >> (hx + hy);
+    y = 2 * ((c >> hx) & ((1 << hy) - 1)) + ((z + (col >> 1)) & 1);
+    x = 2 * (c & ((1 << hx) - 1)) + ((y + (col & 1)) & 1);
+}
+
+// Gauss-Seidel sweeps on a level of n <= 4096 cells.  Coefficients and
+// neighbour offsets are formed once per call: up to 1024 cells a thread owns a
+// cell, above (FP32) one of each colour; FP64 levels above 1024 cells form
+// them per update.
+template <typename T>
+__device__ __forceinline__ void small_gs(const LdsLevel<T> &l, const MGLevel &L, int sweeps, float beta, int has_los) {
+    const int n4 = l.n >> 2, tid = threadIdx.x;
+    if (l.n <= 1024) {
+        int x, y, z;
+        small_xyz(tid < l.n ? tid : 0, l.lx, l.ly, x, y, z);
+        const int mine = tid < l.n ? mg_color(x, y, z) : -1;
+        const SmallNbr o(x, y, z, l.lx, l.ly, l.lz);
+        SmallCell<T> c;
+        c.set(l, L, o, x, y, z, beta, has_los);
+        const T fv = l.f[c.me];
+        for (int s = 0; s < sweeps; s++)
+            for (int col = 0; col < 4; col++) {
+                if (mine == col) l.v[c.me] = c.update(fv, SMALL_NBRS(l.v, o), has_los);
+                __syncthreads();
+            }
+        return;
+    }
+    if constexpr (sizeof(T) == 4) {
+        const int cc = tid < n4 ? tid : 0;
+        SmallCell<T> c[4];
+#pragma unroll
+        for (int col = 0; col < 4; col++) {
+            int x, y, z;
+            small_colour_xyz(cc, col, l.lx, l.ly, x, y, z);
+            c[col].set(l, L, SmallNbr(x, y, z, l.lx, l.ly, l.lz), x, y, z, beta, has_los);
+        }
+        for (int s = 0; s < sweeps; s++)
+#pragma unroll
+            for (int col = 0; col < 4; col++) {
+                if (tid < n4) {
+                    int x, y, z;
+                    small_colour_xyz(cc, col, l.lx, l.ly, x, y, z);
+                    const SmallNbr o(x, y, z, l.lx, l.ly, l.lz);
+                    l.v[c[col].me] = c[col].update(l.f[c[col].me], SMALL_NBRS(l.v, o), has_los);
+                }
+                __syncthreads();
+            }
+        return;
+    }
+    for (int s = 0; s < sweeps; s++)
+        for (int col = 0; col < 4; col++) {
+            for (int i = tid; i < n4; i += blockDim.x) {
+                int x, y, z;
+                small_colour_xyz(i, col, l.lx, l.ly, x, y, z);
+                const SmallNbr o(x, y, z, l.lx, l.ly, l.lz);
+                SmallCell<T> c;
+                c.set(l, L, o, x, y, z, beta, has_los);
+                l.v[c.me] = c.update(l.f[c.me], SMALL_NBRS(l.v, o), has_los);
+            }
+            __syncthreads();
+        }
+}
+
+// the value of the lane that quad_perm CTRL names, within quads of lanes
+template <int CTRL>
+__device__ __forceinline__ double quad_swap(double a) {
+    const uint64_t u = __builtin_bit_cast(uint64_t, a);
+    const uint32_t lo = (uint32_t)__builtin_amdgcn_update_dpp(0, (int)(uint32_t)u, CTRL, 0xf, 0xf, true);
+    const uint32_t hi = (uint32_t)__builtin_amdgcn_update_dpp(0, (int)(uint32_t)(u >> 32), CTRL, 0xf, 0xf, true);
+    return __builtin_bit_cast(double, ((uint64_t)hi << 32) | lo);
+}
+
+// Sweeps on a coarsest FP64 level of at most 64 cells (32 of them before and
+// after): one wave, four lanes per cell of the current colour.  The update is
+// linear, v = f / D + sum_k w_k v_k; lane q of a cell's quad keeps the weights
+// and offsets of neighbours q, q + 4, .. for its cell of each colour, and the
+// quad's partial sums meet by two cross-lane adds.
+__device__ __forceinline__ void small_gs_wave(const LdsLevel<double> &l, const MGLevel &L, int sweeps, float beta,
+                                              int has_los) {
+    if (threadIdx.x < 64) {
+        const int lane = threadIdx.x, quad = lane >> 2, q = lane & 3, n4 = l.n >> 2;
+        double w[4][5], fd[4];
+        int off[4][5], me[4];
+#pragma unroll
+        for (int col = 0; col < 4; col++) {
+            int x, y, z;
+            small_colour_xyz(quad < n4 ? quad : 0, col, l.lx, l.ly, x, y, z);
+            const SmallNbr o(x, y, z, l.lx, l.ly, l.lz);
+            const GsCoef<double> k = small_gs_coef<double>(l, L, x, y, z, beta, has_los);
+            const double rD = 1.0 / (2.0 * ((k.gx + k.gy) + k.gz)), hg = 0.5 * k.g, g = has_los ? 0.0 : k.g;
+            const double wxy = hg * (k.px * k.py), wxz = hg * (k.px * k.pz), wyz = hg * (k.py * k.pz);
+            const double wt[20] = {k.gx + g * k.px, k.gx - g * k.px, k.gy + g * k.py, k.gy - g * k.py,
+                                   k.gz + g * k.pz, k.gz - g * k.pz, wxy, wxy, -wxy, -wxy, wxz, wxz, -wxz, -wxz,
+                                   wyz, wyz, -wyz, -wyz, 0.0, 0.0};
+            const int ot[20] = {o.xp + o.y + o.z,  o.xm + o.y + o.z,  o.x + o.yp + o.z,  o.x + o.ym + o.z,
+                                o.x + o.y + o.zp,  o.x + o.y + o.zm,  o.xp + o.yp + o.z, o.xm + o.ym + o.z,
+                                o.xm + o.yp + o.z, o.xp + o.ym + o.z, o.xp + o.y + o.zp, o.xm + o.y + o.zm,
+                                o.xm + o.y + o.zp, o.xp + o.y + o.zm, o.x + o.yp + o.zp, o.x + o.ym + o.zm,
+                                o.x + o.ym + o.zp, o.x + o.yp + o.zm, 0, 0};
+#pragma unroll
+            for (int i = 0; i < 5; i++) {
+                // entry 4 i + q by selects (the arrays stay in registers)
+                w[col][i] = rD * (q == 0 ? wt[4 * i] : q == 1 ? wt[4 * i + 1] : q == 2 ? wt[4 * i + 2] : wt[4 * i + 3]);
+                off[col][i] = q == 0 ? ot[4 * i] : q == 1 ? ot[4 * i + 1] : q == 2 ? ot[4 * i + 2] : ot[4 * i + 3];
+            }
+            me[col] = o.x + o.y + o.z;
+            fd[col] = q == 0 ? l.f[me[col]] * rD : 0.0;
+        }
+        // within a wave the LDS takes the accesses in order: a pass reads what
+        // the passes before wrote
+        double *v = l.v;
+        for (int s = 0; s < sweeps; s++)
+#pragma unroll
+            for (int col = 0; col < 4; col++) {
+                double t[5];
+#pragma unroll
+                for (int i = 0; i < 5; i++) t[i] = v[off[col][i]];
+                double a = mg_fma(w[col][0], t[0], fd[col]), b = w[col][1] * t[1];
+                a = mg_fma(w[col][2], t[2], a);
+                b = mg_fma(w[col][3], t[3], b);
+                a = mg_fma(w[col][4], t[4], a) + b;
+                a += quad_swap<0xB1>(a);   // lane ^ 1
+                a += quad_swap<0x4E>(a);   // lane ^ 2
+                if (q == 0 && quad < n4) v[me[col]] = a;
+                __builtin_amdgcn_wave_barrier();
+            }
+    }
+    __syncthreads();
+}
+
+// n damped Jacobi sweeps, ping-ponging between l.v (the input) and l.r: the
+// result is in l.r after an odd number.  A thread owns up to 4 cells and forms
+// their coefficients, with the IEEE divisions, once per call.
+__device__ __forceinline__ void small_jacobi(const LdsLevel<float> &l, const MGLevel &L, int n, float beta, float omega,
+                                             int has_los) {
+    Coef<float> k[4];
+    float y[4], fv[4];
+#pragma unroll
+    for (int u = 0; u < 4; u++) {
+        const int c = threadIdx.x + 1024 * u;
+        if (c < l.n) {
+            int cx, cy, cz;
+            small_xyz(c, l.lx, l.ly, cx, cy, cz);
+            k[u] = small_coef<float>(l, L, cx, cy, cz, beta, has_los);
+            y[u] = refined_rcp(2.0f * (k[u].gpx2 + k[u].gpy2 + k[u].gpz2));
+            fv[u] = l.f[c];
+        }
+    }
+    float *in = l.v, *out = l.r;
+    for (int i = 0; i < n; i++) {
+#pragma unroll
+        for (int u = 0; u < 4; u++) {
+            const int c = threadIdx.x + 1024 * u;
+            if (c < l.n) {
+                int cx, cy, cz;
+                small_xyz(c, l.lx, l.ly, cx, cy, cz);
+                const SmallNbr o(cx, cy, cz, l.lx, l.ly, l.lz);
+                const Nbr<float> s = nbr_of<float>(k[u], SMALL_NBRS(in, o));
+                // jacobi_value's operations in its order
+                float j = fv[u] + s.A + s.B + s.C + s.X;
+                if (!has_los) j += s.G;
+                j = div_by(j, 2.0f * (k[u].gpx2 + k[u].gpy2 + k[u].gpz2), y[u]);
+                out[c] = (1.0f - omega) * in[c] + omega * j;
+            }
+        }
+        __syncthreads();
+        float *t = in;
+        in = out;
+        out = t;
+    }
+}
+
+template <typename T>
+__device__ __forceinline__ void small_residual(const LdsLevel<T> &l, const MGLevel &L, float beta, int has_los) {
+    for (int c = threadIdx.x; c < l.n; c += blockDim.x) {
+        int x, y, z;
+        small_xyz(c, l.lx, l.ly, x, y, z);
+        const SmallNbr o(x, y, z, l.lx, l.ly, l.lz);
+        const Coef<T> k = small_coef<T>(l, L, x, y, z, beta, has_los);
+        const Nbr<T> s = nbr_of<T>(k, SMALL_NBRS(l.v, o));
+        T t = (T)2 * (k.gpx2 + k.gpy2 + k.gpz2) * l.v[c] - (s.A + s.B + s.C + s.X);
+        if (!has_los) t -= s.G;
+        l.r[c] = l.f[c] - t;
+    }
+    __syncthreads();
+}
+
+// cl.f = the restriction of w (the finer level l's r or f), cell_reduce's sums
+template <typename T, typename U>
+__device__ __forceinline__ void small_reduce(const LdsLevel<T> &cl, const LdsLevel<U> &l, const U *w) {
+    for (int c = threadIdx.x; c < cl.n; c += blockDim.x) {
+        int x, y, z;
+        small_xyz(c, cl.lx, cl.ly, x, y, z);
+        const SmallNbr o(2 * x + 1, 2 * y + 1, 2 * z + 1, l.lx, l.ly, l.lz);
+#define W(a, b, d) ((T)w[o.a + o.b + o.d])
+        const T s = (T)8 * W(x, y, z) +
+                    (T)4 * (W(xp, y, z) + W(xm, y, z) + W(x, yp, z) + W(x, ym, z) + W(x, y, zp) + W(x, y, zm)) +
+                    (T)2 * (W(xp, yp, z) + W(xm, yp, z) + W(xp, ym, z) + W(xm, ym, z) + W(xp, y, zp) + W(xm, y, zp) +
+                            W(xp, y, zm) + W(xm, y, zm) + W(x, yp, zp) + W(x, ym, zp) + W(x, yp, zm) + W(x, ym, zm)) +
+                    W(xp, yp, zp) + W(xm, yp, zp) + W(xp, ym, zp) + W(xm, ym, zp) + W(xp, yp, zm) + W(xm, yp, zm) +
+                    W(xp, ym, zm) + W(xm, ym, zm);
+#undef W
+        cl.f[c] = (T)((double)s / 64.0);
+    }
+    __syncthreads();
+}
+
+template <typename T>
+__device__ __forceinline__ void small_zero(const LdsLevel<T> &l) {
+    for (int c = threadIdx.x; c < l.n; c += blockDim.x) l.v[c] = (T)0;
+    __syncthreads();
+}
+
+// l.v (+)= the prolongation of cl.v, prolong_value's sums
+template <typename T, typename U>
+__device__ __forceinline__ void small_prolong(const LdsLevel<T> &l, const LdsLevel<U> &cl, bool add) {
+    for (int c = threadIdx.x; c < l.n; c += blockDim.x) {
+        int x, y, z;
+        small_xyz(c, l.lx, l.ly, x, y, z);
+        const U val = prolong_value<U>(cl.v, 1 << cl.lx, 1 << cl.ly, 1 << cl.lz, x, y, z);
+        l.v[c] = add ? (T)(l.v[c] + (T)val) : (T)val;
+    }
+    __syncthreads();
+}
+
+// GS: four-colour Gauss-Seidel V-cycle (levels of both precisions); else
+// damped Jacobi in FP32, one V-cycle or (fmg) the whole FMG
+template <int GS>
+__global__ void __launch_bounds__(1024) k_mg_small(MGSmall a) {
+    __shared__ __align__(16) char pool[kMGSmallPool];
+    const int nl = a.nl;
+    uint32_t swapped = 0;   // bit l: an odd number of Jacobi sweeps so far, v and r exchanged
+    auto lev = [&](auto tag, int l) {
+        using T = decltype(tag);
+        LdsLevel<T> d;
+        const bool s = (swapped >> l) & 1;
+        d.v = reinterpret_cast<T *>(pool + (s ? a.off_r[l] : a.off_v[l]));
+        d.r = reinterpret_cast<T *>(pool + (s ? a.off_v[l] : a.off_r[l]));
+        d.f = reinterpret_cast<T *>(pool + a.off_f[l]);
+        d.p = reinterpret_cast<const T *>(pool + a.off_p[l]);
+        d.lx = a.lg[l][0];
+        d.ly = a.lg[l][1];
+        d.lz = a.lg[l][2];
+        d.n = 1 << (d.lx + d.ly + d.lz);
+        return d;
+    };
+    auto smooth = [&](int l) __attribute__((always_inline)) {
+        if constexpr (GS) {
+            const int n = l + 1 == nl ? 16 * a.rb_sweeps : a.rb_sweeps;
+            if (a.dbl[l]) {
+                const auto d = lev(double(), l);
+                if (l + 1 == nl && d.n <= 64)
+                    small_gs_wave(d, a.L[l], n, a.beta, a.has_los);
+                else
+                    small_gs<double>(d, a.L[l], n, a.beta, a.has_los);
+            } else {
+                small_gs<float>(lev(float(), l), a.L[l], n, a.beta, a.has_los);
+            }
+        } else {
+            small_jacobi(lev(float(), l), a.L[l], a.jacobi_n, a.beta, a.omega, a.has_los);
+            if (a.jacobi_n > 0 && (a.jacobi_n & 1)) swapped ^= 1u << l;
+        }
+    };
+    // down: residual of level l restricted into f of level l + 1, v there zero
+    auto down = [&](int l) __attribute__((always_inline)) {
+        if (GS && a.dbl[l]) {
+            const auto d = lev(double(), l), e = lev(double(), l + 1);
+            small_residual<double>(d, a.L[l], a.beta, a.has_los);
+            small_reduce<double, double>(e, d, d.r);
+            small_zero<double>(e);
+        } else {
+            const auto d = lev(float(), l);
+            small_residual<float>(d, a.L[l], a.beta, a.has_los);
+            if (GS && a.dbl[l + 1]) {
+                const auto e = lev(double(), l + 1);
+                small_reduce<double, float>(e, d, d.r);
+                small_zero<double>(e);
+            } else {
+                const auto e = lev(float(), l + 1);
+                small_reduce<float, float>(e, d, d.r);
+                small_zero<float>(e);
+            }
+        }
+    };
+    auto up = [&](int l, bool add) __attribute__((always_inline)) {
+        if (GS && a.dbl[l])
+            small_prolong<double, double>(lev(double(), l), lev(double(), l + 1), add);
+        else if (GS && a.dbl[l + 1])
+            small_prolong<float, double>(lev(float(), l), lev(double(), l + 1), add);
+        else
+            small_prolong<float, float>(lev(float(), l), lev(float(), l + 1), add);
+    };
+    // down from level top (pre-smooth, residual, restrict) to the coarsest,
+    // which smooths twice, and up again (prolong and add, post-smooth)
+    auto vcycle = [&](int top) __attribute__((always_inline)) {
+        bool pre = true;
+        for (int l = top;;) {
+            smooth(l);
+            if (pre && l + 1 < nl) {
+                down(l);
+                l++;
+            } else if (pre) {
+                pre = false;
+            } else if (l == top) {
+                break;
+            } else {
+                l--;
+                up(l, true);
+            }
+        }
+    };
+    // the LOS tables
+    if (!a.has_los)
+        for (int l = 0; l < nl; l++) {
+            const MGLevel &L = a.L[l];
+            for (int i = threadIdx.x; i < L.n[0] + L.n[1] + L.n[2]; i += blockDim.x) {
+                if (GS && a.dbl[l]) {
+                    const float cell = i < L.n[0] ? L.cell[0] : (i < L.n[0] + L.n[1] ? L.cell[1] : L.cell[2]);
+                    reinterpret_cast<double *>(pool + a.off_p[l])[i] = (double)L.xv[i] / (double)cell;
+                } else {
+                    reinterpret_cast<float *>(pool + a.off_p[l])[i] = L.pv[i];
+                }
+            }
+        }
+    // the top level in: f, and v (zero without one)
+    auto in = [&](auto tag) {
+        using T = decltype(tag);
+        const auto d = lev(tag, 0);
+        const T *f = static_cast<const T *>(a.f), *v = static_cast<const T *>(a.vin);
+        for (int c = threadIdx.x; c < d.n; c += blockDim.x) {
+            d.f[c] = f[c];
+            d.v[c] = v ? v[c] : (T)0;
+        }
+        __syncthreads();
+    };
+    auto out = [&](auto tag) {
+        using T = decltype(tag);
+        const auto d = lev(tag, 0);
+        T *v = static_cast<T *>(a.vout);
+        for (int c = threadIdx.x; c < d.n; c += blockDim.x) v[c] = d.v[c];
+    };
+    if (GS && a.dbl[0])
+        in(double());
+    else
+        in(float());
+    int first = 0, reps = 1;
+    if (!GS && a.fmg) {
+        for (int l = 0; l + 1 < nl; l++) {
+            const auto d = lev(float(), l);
+            small_reduce<float, float>(lev(float(), l + 1), d, d.f);
+        }
+        small_zero<float>(lev(float(), nl - 1));
+        first = nl - 1;
+        reps = a.vcycles;
+    }
+    for (int l = first; l >= 0; l--) {
+        if (l < first) up(l, false);
+        for (int i = 0; i < reps; i++) vcycle(l);
+    }
+    if (GS && a.dbl[0])
+        out(double());
+    else
+        out(float());
+}
+
 // Cell centres of every level (x_vec per level, src/multigrid.jl:656).
 __global__ void k_mg_xvec(float *xv, const Slot *slot, int nx, int ny, int nz) {
     const int n3[3] = {nx, ny, nz};
@@ -1902,6 +2462,60 @@ hipError_t launch_mg_rbgs(T *v, const T *f, const MGLevel &L, float beta, int ha
     dim3 grid, block;
     stencil_shape(L, grid, block);
     hipLaunchKernelGGL(k_mg_mcgs<T>, grid, block, 0, s, v, f, L, beta, has_los, color);
+    return hipGetLastError();
+}
+
+bool mg_gs_tile_ok(const MGLevel &L) {
+    return L.n[0] % kGbT == 0 && L.n[1] % kGbT == 0 && L.n[2] % kGbT == 0 && L.n[1] / kGbT < 65536 &&
+           L.n[2] / kGbT < 65536;
+}
+
+hipError_t launch_mg_gs_tile(float *vout, const float *vin, const float *f, const MGLevel &L, float beta, int has_los,
+                             hipStream_t s) {
+    if (!mg_gs_tile_ok(L) || vout == vin || !vout || ((uintptr_t)vout & 15) || ((uintptr_t)vin & 15))
+        return hipErrorInvalidValue;
+    const dim3 grid((unsigned)(L.n[0] / kGbT), (unsigned)(L.n[1] / kGbT), (unsigned)(L.n[2] / kGbT));
+    using K = decltype(&k_mg_gs_tile<0, 0>);
+    static const K kernels[4] = {k_mg_gs_tile<0, 0>, k_mg_gs_tile<0, 1>, k_mg_gs_tile<1, 0>, k_mg_gs_tile<1, 1>};
+    hipLaunchKernelGGL(kernels[(has_los ? 2 : 0) + (vin ? 0 : 1)], grid, dim3(kGbThreads), 0, s, vout, vin, f, L, beta);
+    return hipGetLastError();
+}
+
+bool mg_small_layout(MGSmall &a) {
+    size_t o = 0;
+    if (a.nl < 1 || a.nl > kMGSmallLevels) return false;
+    for (int l = 0; l < a.nl; l++) {
+        int64_t n = 1;
+        for (int k = 0; k < 3; k++) {
+            const int side = a.L[l].n[k];
+            if (side < 2 || (side & (side - 1))) return false;
+            if (l > 0 && 2 * side != a.L[l - 1].n[k]) return false;
+            a.lg[l][k] = __builtin_ctz((unsigned)side);
+            n *= side;
+        }
+        if (n > kMGSmallCells || (l > 0 && a.dbl[l - 1] && !a.dbl[l])) return false;
+        const size_t bytes = ((size_t)n * (a.dbl[l] ? 8 : 4) + 15) & ~(size_t)15;
+        a.off_v[l] = (int)o;
+        a.off_f[l] = (int)(o + bytes);
+        a.off_r[l] = (int)(o + 2 * bytes);
+        a.off_p[l] = (int)(o + 3 * bytes);
+        const size_t sides = (size_t)a.L[l].n[0] + a.L[l].n[1] + a.L[l].n[2];
+        o += 3 * bytes + ((sides * (a.dbl[l] ? 8 : 4) + 15) & ~(size_t)15);
+    }
+    return o <= (size_t)kMGSmallPool;
+}
+
+hipError_t launch_mg_small(const MGSmall &a0, hipStream_t s) {
+    MGSmall a = a0;
+    if (!mg_small_layout(a) || !a.f || !a.vout) return hipErrorInvalidValue;
+    if (a.gs) {
+        if (a.fmg) return hipErrorInvalidValue;
+        hipLaunchKernelGGL(k_mg_small<1>, dim3(1), dim3(1024), 0, s, a);
+    } else {
+        for (int l = 0; l < a.nl; l++)
+            if (a.dbl[l]) return hipErrorInvalidValue;
+        hipLaunchKernelGGL(k_mg_small<0>, dim3(1), dim3(1024), 0, s, a);
+    }
     return hipGetLastError();
 }
 

@@ -168,3 +168,47 @@ def test_fused_residual_restriction_rejects_unsupported_shape(ctx):
     with pytest.raises(bh.BaorecError):
         bh.residual_restrict_(c, v, f, recon(shape, None, ctx), fused=True)
     bh.residual_restrict_(c, v, f, recon(shape, None, ctx), fused=False)
+
+
+@pytest.mark.parametrize("shape", [(16, 16, 16), (8, 16, 32), (64, 32, 16), (8, 8, 64), (24, 24, 24), (40, 64, 96)])
+@pytest.mark.parametrize("los", [None, [0.3, -0.4, 0.866]])
+@pytest.mark.parametrize("fp64_coarse_max", [0, 8, 16])
+def test_small_levels_rbgs_solves(ctx, shape, los, fp64_coarse_max):
+    """RBGS solves whose levels run in one workgroup's LDS (power-of-two
+    sides, at most 4096 cells, either precision), by 8^3 tiles (sides
+    multiples of 8) or by the general kernels (24^3 halves to odd sides):
+    the solution satisfies the FP64 oracle's operator to the tolerance, up
+    to the solve's reported shift of f."""
+    f = np.random.default_rng(sum(shape)).standard_normal(shape).astype(F32)
+    f -= f.mean()
+    rec = recon(shape, los, ctx)
+    rec.schedule, rec.tolerance, rec.fp64_coarse_max, rec.rb_sweeps = "rbgs", 1e-5, fp64_coarse_max, 2
+    phi = bh.fmg(f, rec)
+    assert rec.final_residual <= 1e-5 and rec.vcycles_done <= 30
+    r = orc.mg_residual(phi.astype(np.float64), f.astype(np.float64) - rec.rhs_shift, rec.box_size, rec.box_min,
+                        rec.beta, los=los)
+    rel = float(np.linalg.norm(r) / np.linalg.norm(f))
+    print(f"{shape} los {los} fp64 <= {fp64_coarse_max}: {rec.vcycles_done} V-cycles, residual {rel:.1e}")
+    assert rel < 3e-5   # the tolerance, and phi's FP32 rounding (|A| |phi| 2^-24 / |f|, about 1e-6)
+
+
+@pytest.mark.parametrize("shape", [(16, 16, 16), (8, 16, 32), (8, 8, 8), (32, 32, 32)])
+@pytest.mark.parametrize("sweeps", [5, 2])
+def test_small_levels_fmg_matches_oracle(ctx, shape, sweeps):
+    """The reference's schedule on levels in one workgroup's LDS against the
+    FP32 oracle (odd and even sweeps per smoothing: the result in either
+    buffer): the same operations in the same order, so the schedules stay
+    within the growth of single roundings, 2e-5 of the solution's norm."""
+    f = np.random.default_rng(7).standard_normal(shape).astype(F32)
+    f -= f.mean()
+    rec = recon(shape, None, ctx)
+    rec.jacobi_niterations, rec.vcycle_niterations = sweeps, 3
+    got = bh.fmg(f, rec)
+    exp = orc.fmg(f, rec.box_size, rec.box_min, rec.beta, 0.4, sweeps, 3)
+    err = float(np.linalg.norm(got - exp) / np.linalg.norm(exp))
+    print(f"{shape} x{sweeps}: {err:.1e}")
+    assert err < 2e-5
+    v = f.copy()
+    bh.vcycle_(v, f, rec)
+    exp = orc.mg_vcycle(f.copy(), f, rec.box_size, rec.box_min, rec.beta, 0.4, sweeps)
+    assert np.linalg.norm(v - exp) < 2e-5 * np.linalg.norm(exp)
