@@ -19,6 +19,7 @@
 #include <math.h>
 #include <string.h>
 
+#include <algorithm>
 #include <vector>
 
 #include "kernels.hpp"
@@ -137,111 +138,203 @@ __global__ void __launch_bounds__(256) k_conv(ConvArgs a) {
     }
 }
 
-// Weight gradient.  Workgroup: 16 input channels (block blockIdx.y / NBO), 16
+// Weight gradient.  Workgroup: 16 input channels (block blockIdx.y / NBO), 16 NB
 // output channels (block blockIdx.y % NBO), all 27 taps, bricks
-// [chunk * per, (chunk + 1) * per) of 16 x 4 x 4 voxels.  Wave w owns taps
-// 7w .. 7w + 6.  A = dout^T (rows: output channels, K: the brick's voxels in
-// x-fastest order), B = the input at the tap's offset (columns: input
-// channels); both come from LDS.
+// [chunk * per, (chunk + 1) * per) of 16 x 4 x 4 voxels.  A = dout^T (rows:
+// output channels, K: the brick's voxels in x-fastest order, 32 per product),
+// B = the input at the tap's offset (columns: input channels).  Both stand in
+// LDS channels last, as in memory, and reach the matrix cores through the
+// transposing LDS read (16 lanes fetch 4 voxels x 16 channels and each gets
+// one channel's 4 voxels), so a product's operands cost 64-bit reads and no
+// element moves.  Wave w owns the 9 taps with dy = w - 1: an input row pair
+// read once (10 voxels per lane: the three dx are register shifts) feeds three
+// dx times the up to three dz whose voxels lie in the brick; dout of the whole
+// brick stays in registers.  Every tap's products run in ascending voxel
+// order, one accumulator chain per chunk.  The next brick's global loads are
+// in flight during the products; with one workgroup per chunk (a CU then has
+// only this one) LDS is double buffered.
+//
+// LDS reads are free of bank conflicts: an input row has 128 spare bytes after
+// every 8 voxels, so that the two 8-voxel halves a read touches lie in
+// different halves of the banks, and dout's voxel 4-groups change places in
+// every second 8-group.
+//
+// Measured on a batch of four 128^3 grids: 16 -> 16 channels 226 us (537 MB of
+// inputs, 115 us at the copy rate; with element-wise LDS reads 1337), 48 -> 16
+// 511 us (2517), 96 -> 32 at 64^3 269 us (1187).  With one workgroup of three
+// waves per CU the finest layers are bound by the brick's load, store and
+// barrier not fully hidden behind its 72 products per wave; the coarse ones by
+// the partial sums of their chunks (up to 340 MB).
+typedef short s16x4 __attribute__((ext_vector_type(4)));
+__device__ __forceinline__ uint2 lds_read_tr(const uint16_t *p) {
+    const s16x4 v = __builtin_amdgcn_ds_read_tr16_b64_v4i16(
+        (__attribute__((address_space(3))) s16x4 *)(__attribute__((address_space(3))) void *)p);
+    return __builtin_bit_cast(uint2, v);
+}
+constexpr int kWgThreads = 192, kWgRow = 448;   // threads; uint16 per LDS row of 18 voxels (and 2 never used)
+__host__ __device__ constexpr int wgrad_nb(int co) { return co >= 32 ? 2 : 1; }
+
 template <int C1, int C2, int CO, bool UP2>
-__global__ void __launch_bounds__(256) k_conv_wgrad(WgradArgs a) {
+__global__ void __launch_bounds__(kWgThreads, 1) k_conv_wgrad(WgradArgs a) {
     constexpr int CIN = C1 + C2;
-    constexpr int NBO = CO / 16;
-    __shared__ __align__(16) uint16_t sIn[16][6][6][18];
-    __shared__ __align__(16) uint16_t sDo[16][256];
-    const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+    constexpr int NB = wgrad_nb(CO), NBO = CO / (16 * NB);
+    constexpr int BUFS = ((CIN + 15) / 16) * NBO == 1 ? 2 : 1;
+    constexpr int NIN = 7, NDO = (512 * NB + kWgThreads - 1) / kWgThreads;   // 16-byte loads per thread
+    __shared__ __align__(16) uint16_t sIn[BUFS][36 * kWgRow];
+    __shared__ __align__(16) uint16_t sDo[BUFS][NB * 4096];
+    const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
     const int r16 = lane & 15, g = lane >> 4;
     const int cib = blockIdx.y / NBO, cob = blockIdx.y % NBO;
     const int nx = 1 << a.lx, ny = 1 << a.ly, nz = 1 << a.lz;
-    const int bx = (nx + 15) >> 4, by = (ny + 3) >> 2, bz = (nz + 3) >> 2;
-    const int64_t nbricks = (int64_t)bx * by * bz * a.batch;
-    const int t0 = wave * 7, tn = wave == 3 ? 6 : 7;
-    f32x4 acc[7];
+    // log2 of the bricks along each axis
+    const int lbx = a.lx > 4 ? a.lx - 4 : 0, lby = a.ly > 2 ? a.ly - 2 : 0, lbz = a.lz > 2 ? a.lz - 2 : 0;
+    const int nbricks = a.batch << (lbx + lby + lbz);
+    f32x4 acc[NB][3][3];   // [][dz][dx]
 #pragma unroll
-    for (int i = 0; i < 7; i++) acc[i] = f32x4{0.f, 0.f, 0.f, 0.f};
-    const int64_t beg = (int64_t)blockIdx.x * a.per;
-    const int64_t end = beg + a.per < nbricks ? beg + a.per : nbricks;
-    for (int64_t br = beg; br < end; br++) {
-        int64_t q = br;
-        const int ix = (int)(q % bx); q /= bx;
-        const int iy = (int)(q % by); q /= by;
-        const int iz = (int)(q % bz);
-        const int b = (int)(q / bz);
-        const int x0 = ix * 16, y0 = iy * 4, z0 = iz * 4;
-        __syncthreads();
-        // the input block with a one-cell halo, transposed to [c][z][y][x]
-        for (int idx = threadIdx.x; idx < 648 * 2; idx += 256) {
-            const int v = idx >> 1, half = idx & 1;
+    for (int n = 0; n < NB; n++)
+#pragma unroll
+        for (int i = 0; i < 9; i++) acc[n][i / 3][i % 3] = f32x4{0.f, 0.f, 0.f, 0.f};
+    const int beg = blockIdx.x * (int)a.per;
+    const int end = nbricks - beg > a.per ? beg + (int)a.per : nbricks;
+
+    // this thread's 16-byte pieces of a brick: half = 8 channels of voxel v of
+    // the input with its one-cell halo (18 x 6 x 6), and of dout (16 x 4 x 4)
+    const int half = tid & 1;
+    const bool skip = CIN < 16 && half == 1;   // 8 input channels: the rest are zero
+    const int c = cib * 16 + half * 8;
+    uint4 rin[NIN], rdo[NDO];
+    // voxel index on the grid of sides halved l times
+    auto vox = [&](uint32_t b, uint32_t z, uint32_t y, uint32_t x, int l) {
+        const uint32_t zy = (((b << (a.lz - l)) + z) << (a.ly - l)) + y;
+        return (zy << (a.lx - l)) + x;
+    };
+    auto load = [&](int br) {
+        const int x0 = (br & ((1 << lbx) - 1)) * 16, y0 = ((br >> lbx) & ((1 << lby) - 1)) * 4;
+        const int z0 = ((br >> (lbx + lby)) & ((1 << lbz) - 1)) * 4;
+        const uint32_t b = (uint32_t)br >> (lbx + lby + lbz);
+#pragma unroll
+        for (int u = 0; u < NIN; u++) {
+            const int v = (tid >> 1) + (kWgThreads / 2) * u;
+            rin[u] = make_uint4(0u, 0u, 0u, 0u);
+            if (v >= 648 || skip) continue;
             const int hx = v % 18, hy = (v / 18) % 6, hz = v / 108;
             const int xs = (x0 - 1 + hx) & (nx - 1), ys = (y0 - 1 + hy) & (ny - 1), zs = (z0 - 1 + hz) & (nz - 1);
-            const int c = cib * 16 + half * 8;
-            uint4 q4 = make_uint4(0u, 0u, 0u, 0u);
-            if (c < CIN) {
-                const uint16_t *src;
-                if (C2 == 0 || c < C1) {
-                    src = a.in1 + ((((size_t)b * nz + zs) * ny + ys) * nx + xs) * C1 + c;
-                } else if (UP2) {
-                    const int cx = nx >> 1, cy = ny >> 1, cz = nz >> 1;
-                    src = a.in2 + ((((size_t)b * cz + (zs >> 1)) * cy + (ys >> 1)) * cx + (xs >> 1)) * C2 + (c - C1);
-                } else {
-                    src = a.in2 + ((((size_t)b * nz + zs) * ny + ys) * nx + xs) * C2 + (c - C1);
-                }
-                q4 = *reinterpret_cast<const uint4 *>(src);
+            const uint16_t *src;
+            if (C2 == 0 || cib * 16 < C1) {
+                src = a.in1 + vox(b, zs, ys, xs, 0) * C1 + c;
+            } else if (UP2) {
+                src = a.in2 + vox(b, zs >> 1, ys >> 1, xs >> 1, 1) * C2 + (c - C1);
+            } else {
+                src = a.in2 + vox(b, zs, ys, xs, 0) * C2 + (c - C1);
             }
-            const uint16_t *h = reinterpret_cast<const uint16_t *>(&q4);
-#pragma unroll
-            for (int j = 0; j < 8; j++) sIn[half * 8 + j][hz][hy][hx] = h[j];
+            rin[u] = *reinterpret_cast<const uint4 *>(src);
         }
-        // the output gradient of the brick, transposed to [c][voxel]
-        for (int idx = threadIdx.x; idx < 512; idx += 256) {
-            const int v = idx >> 1, half = idx & 1;
+#pragma unroll
+        for (int u = 0; u < NDO; u++) {
+            const int i = tid + kWgThreads * u, h = i % (2 * NB), v = i / (2 * NB);
+            rdo[u] = make_uint4(0u, 0u, 0u, 0u);
             const int x = x0 + (v & 15), y = y0 + ((v >> 4) & 3), z = z0 + (v >> 6);
-            uint4 q4 = make_uint4(0u, 0u, 0u, 0u);
-            if (x < nx && y < ny && z < nz)
-                q4 = *reinterpret_cast<const uint4 *>(a.dout + ((((size_t)b * nz + z) * ny + y) * nx + x) * CO +
-                                                     cob * 16 + half * 8);
-            const uint16_t *h = reinterpret_cast<const uint16_t *>(&q4);
-#pragma unroll
-            for (int j = 0; j < 8; j++) sDo[half * 8 + j][v] = h[j];
+            if (v < 256 && x < nx && y < ny && z < nz)
+                rdo[u] = *reinterpret_cast<const uint4 *>(a.dout + vox(b, z, y, x, 0) * CO +
+                                                          cob * 16 * NB + h * 8);
         }
-        __syncthreads();
-        for (int kb = 0; kb < 8; kb++) {
-            const bf16x8 av = *reinterpret_cast<const bf16x8 *>(&sDo[r16][kb * 32 + g * 8]);
-            const int k0 = kb * 32 + g * 8;
-            const int xk = k0 & 15, yk = (k0 >> 4) & 3, zk = k0 >> 6;
+    };
+    auto store = [&](int buf) {
 #pragma unroll
-            for (int i = 0; i < 7; i++) {
-                if (i >= tn) break;
-                const int t = t0 + i;
-                const int dx = t % 3 - 1, dy = (t / 3) % 3 - 1, dz = t / 9 - 1;
-                const uint16_t *row = &sIn[r16][zk + dz + 1][yk + dy + 1][xk + dx + 1];
-                uint16_t e[8];
+        for (int u = 0; u < NIN; u++) {
+            const int v = (tid >> 1) + (kWgThreads / 2) * u;
+            const int hx = v % 18, row = v / 18;   // row = hz * 6 + hy
+            if (v < 648)
+                *reinterpret_cast<uint4 *>(&sIn[buf][row * kWgRow + hx * 16 + (hx >> 3) * 64 + half * 8]) = rin[u];
+        }
 #pragma unroll
-                for (int j = 0; j < 8; j++) e[j] = row[j];
-                bf16x8 bv;
-                memcpy(&bv, e, 16);
-                acc[i] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(av, bv, acc[i], 0, 0, 0);
+        for (int u = 0; u < NDO; u++) {
+            const int i = tid + kWgThreads * u, h = i % (2 * NB), v = i / (2 * NB);
+            if (v < 256)
+                *reinterpret_cast<uint4 *>(
+                    &sDo[buf][(h >> 1) * 4096 + (v ^ ((v >> 1) & 4)) * 16 + (h & 1) * 8]) = rdo[u];
+        }
+    };
+    auto compute = [&](int buf) {
+        uint4 av[NB][8];
+        const uint16_t *d0 = &sDo[buf][g * 128 + (g & 1) * 64 + r16 * 4];
+        const uint16_t *d1 = &sDo[buf][g * 128 + 64 - (g & 1) * 64 + r16 * 4];
+#pragma unroll
+        for (int n = 0; n < NB; n++)
+#pragma unroll
+            for (int kb = 0; kb < 8; kb++) {
+                const uint2 lo = lds_read_tr(d0 + n * 4096 + kb * 512), hi = lds_read_tr(d1 + n * 4096 + kb * 512);
+                av[n][kb] = make_uint4(lo.x, lo.y, hi.x, hi.y);
             }
-        }
+        const uint16_t *in0 = &sIn[buf][((g >> 1) + wave) * kWgRow + (g & 1) * 192 + r16 * 4];
+#pragma unroll
+        for (int zi = 0; zi < 6; zi++)
+#pragma unroll
+            for (int yp = 0; yp < 2; yp++) {
+                const uint16_t *row = in0 + (zi * 6 + 2 * yp) * kWgRow;
+                const uint2 p = lds_read_tr(row), q = lds_read_tr(row + 64), r = lds_read_tr(row + 192);
+                const uint4 bv[3] = {make_uint4(p.x, p.y, q.x, q.y),
+                                     make_uint4(__builtin_amdgcn_alignbit(p.y, p.x, 16),
+                                                __builtin_amdgcn_alignbit(q.x, p.y, 16),
+                                                __builtin_amdgcn_alignbit(q.y, q.x, 16),
+                                                __builtin_amdgcn_alignbit(r.x, q.y, 16)),
+                                     make_uint4(p.y, q.x, q.y, r.x)};
+#pragma unroll
+                for (int dz = 0; dz < 3; dz++) {
+                    const int zk = zi - dz;
+                    if (zk < 0 || zk > 3) continue;
+#pragma unroll
+                    for (int n = 0; n < NB; n++)
+#pragma unroll
+                        for (int dx = 0; dx < 3; dx++)
+                            acc[n][dz][dx] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(
+                                __builtin_bit_cast(bf16x8, av[n][2 * zk + yp]), __builtin_bit_cast(bf16x8, bv[dx]),
+                                acc[n][dz][dx], 0, 0, 0);
+                }
+            }
+    };
+    load(beg);
+    store(0);
+    __syncthreads();
+    int buf = 0;
+    for (int br = beg; br < end; br++) {
+        const bool more = br + 1 < end;
+        if (more) load(br + 1);
+        compute(buf);
+        if (BUFS == 2) buf ^= 1;
+        else __syncthreads();
+        if (more) store(buf);
+        __syncthreads();
     }
     // D[row = output channel 4g + r][column = input channel r16]
     const int ci = cib * 16 + r16;
     if (ci >= CIN) return;
     float *part = a.part + (size_t)blockIdx.x * 27 * CIN * CO;
 #pragma unroll
-    for (int i = 0; i < 7; i++) {
-        if (i >= tn) break;
-        const int t = t0 + i;
+    for (int n = 0; n < NB; n++)
 #pragma unroll
-        for (int r = 0; r < 4; r++) part[((size_t)t * CIN + ci) * CO + cob * 16 + 4 * g + r] = acc[i][r];
-    }
+        for (int dz = 0; dz < 3; dz++)
+#pragma unroll
+            for (int dx = 0; dx < 3; dx++) {
+                const int t = dz * 9 + wave * 3 + dx;
+                *reinterpret_cast<f32x4 *>(part + ((size_t)t * CIN + ci) * CO + (cob * NB + n) * 16 + 4 * g) =
+                    acc[n][dz][dx];
+            }
 }
 
 // out[i] = sum over chunks c of part[c][i], c in order
 __global__ void k_sum_chunks(const float *__restrict__ part, int nch, int64_t n, float *__restrict__ out) {
     for (int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x; i < n; i += (int64_t)gridDim.x * blockDim.x) {
         float s = 0.f;
-        for (int c = 0; c < nch; c++) s += part[(size_t)c * n + i];
+        int c = 0;
+        for (; c + 16 <= nch; c += 16) {   // 16 loads in flight, added in order
+            float v[16];
+#pragma unroll
+            for (int j = 0; j < 16; j++) v[j] = part[(size_t)(c + j) * n + i];
+#pragma unroll
+            for (int j = 0; j < 16; j++) s += v[j];
+        }
+        for (; c < nch; c++) s += part[(size_t)c * n + i];
         out[i] = s;
     }
 }
@@ -621,7 +714,8 @@ static inline unsigned blocks(int64_t n) {
 
 using namespace unet;
 
-#define CONV_CASES(X)          \
+// the layers; and the input gradients that are no layer's shape
+#define LAYER_CASES(X)         \
     X(8, 0, 16, false)         \
     X(16, 0, 16, false)        \
     X(16, 0, 32, false)        \
@@ -632,7 +726,9 @@ using namespace unet;
     X(128, 0, 128, false)      \
     X(64, 128, 64, true)       \
     X(32, 64, 32, true)        \
-    X(16, 32, 16, true)        \
+    X(16, 32, 16, true)
+#define CONV_CASES(X)          \
+    LAYER_CASES(X)             \
     X(32, 0, 16, false)        \
     X(64, 0, 32, false)        \
     X(128, 0, 64, false)       \
@@ -661,14 +757,17 @@ hipError_t launch_unet_conv(const ConvArgs &a, int c1, int c2, int co, bool relu
 }
 
 hipError_t launch_unet_wgrad(const WgradArgs &a, int c1, int c2, int co, bool up2, int nchunks, hipStream_t s) {
-    const int cib = (c1 + c2 + 15) / 16, cob = co / 16;
+    // k_conv_wgrad addresses its inputs with 32-bit element offsets
+    const int cmax = std::max(std::max(c1, c2), co);
+    if (((int64_t)a.batch * cmax << (a.lx + a.ly + a.lz)) >= ((int64_t)1 << 31)) return hipErrorInvalidValue;
+    const int cib = (c1 + c2 + 15) / 16, cob = co / (16 * wgrad_nb(co));
     dim3 grid((unsigned)nchunks, (unsigned)(cib * cob));
 #define LAUNCH(C1_, C2_, CO_, UP_)                                                                        \
     if (c1 == C1_ && c2 == C2_ && co == CO_ && up2 == UP_) {                                              \
-        hipLaunchKernelGGL((k_conv_wgrad<C1_, C2_, CO_, UP_>), grid, dim3(256), 0, s, a);                 \
+        hipLaunchKernelGGL((k_conv_wgrad<C1_, C2_, CO_, UP_>), grid, dim3(kWgThreads), 0, s, a);          \
         return hipGetLastError();                                                                         \
     }
-    CONV_CASES(LAUNCH)
+    LAYER_CASES(LAUNCH)
 #undef LAUNCH
     return hipErrorInvalidValue;
 }

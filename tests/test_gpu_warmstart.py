@@ -120,6 +120,52 @@ def test_unet_layers_match_oracle_on_their_inputs(ctx, shape):
             assert_bf16_close(U.bf16_bits(dA[i1]), dx * (A[i1] > 0), f"input gradient {i}")
 
 
+@pytest.mark.parametrize("shape", [(3, 64, 64, 64), (5, 32, 16, 128)])
+def test_weight_gradients_over_many_bricks(ctx, shape):
+    """Weight gradients where a workgroup streams several bricks (and the last
+    one fewer), against FP64 sums over the GPU's own layer inputs and masked
+    output gradients.  A sum is a chain of FP32 additions: 8 products of 32
+    terms per brick, the chunks' sums, and the additions inside a product."""
+    import torch
+
+    B, Z, Y, Xn = shape
+    Xb = features(shape, 21)
+    T = np.random.default_rng(22).standard_normal(shape).astype(F32)
+    bh.warmstart_init(seed=4, h_train=1.0, ctx=ctx)
+    bh.warmstart_eval(Xb, T, ctx=ctx)
+    grads = torch.from_numpy(bh.warmstart_params("grads", ctx=ctx)).double()
+
+    def tensor(kind, i, level, c):
+        b = bh.warmstart_tensor(kind, i, (B, Z >> level, Y >> level, Xn >> level, c), ctx=ctx)
+        return torch.from_numpy(U.from_bits(b)).double()
+
+    offs, _, _ = U.offsets()
+    for i, (c1, c2, co, lvl, i1, i2) in enumerate(U.LAYERS):
+        if i1 == -1:
+            x = torch.from_numpy(U.from_bits(Xb)).double()
+        elif i1 <= -2:
+            x = tensor("pool", -i1 - 2, lvl, c1)
+        else:
+            x = tensor("act", i1, U.LAYERS[i1][3], c1)
+        if i2 is not None:
+            u = tensor("act", i2, U.LAYERS[i2][3], c2)
+            for d in (1, 2, 3):
+                u = u.repeat_interleave(2, dim=d)
+            x = torch.cat([x, u], dim=-1)
+        d = tensor("grad", i, lvl, co).reshape(-1, co)
+        wo, bo = offs[i]
+        got = grads[wo:bo].reshape(27, c1 + c2, co)
+        n = d.shape[0]
+        nbricks = max(1, n // 256)
+        steps = 8 * -(-nbricks // 256) + min(nbricks, 256) + 32
+        for t in range(27):
+            off = (t // 9 - 1, (t // 3) % 3 - 1, t % 3 - 1)
+            xt = torch.roll(x, [-o for o in off], dims=(1, 2, 3)).reshape(n, -1)
+            err = (got[t] - xt.T.contiguous() @ d).abs()
+            bound = steps * 2.0 ** -24 * (xt.abs().T.contiguous() @ d.abs())
+            assert bool((err <= bound).all()), (i, t, float((err - bound).max()))
+
+
 def test_unet_gradients_within_bf16_rounding(ctx):
     """The whole network's output and gradients against the exact FP64
     network: per layer no further from it than 1.5x (plus 0.02) what the
