@@ -428,7 +428,10 @@ struct ConvArgs {
     const uint16_t *in2;   // C2 channels, half resolution when up2 (nearest upsampling on read)
     const uint16_t *w;     // packed B operand (launch_unet_pack)
     const float *bias;     // CO entries or NULL
-    uint16_t *out;         // CO channels
+    uint16_t *out;         // channels [0, csplit)
+    uint16_t *out2;        // channels [csplit, CO)
+    int csplit;            // CO: all of them in out
+    const uint16_t *mask;  // input gradient of a ReLU: its output (CO channels), or NULL
     int lx, ly, lz;
 };
 struct WgradArgs {
@@ -450,13 +453,12 @@ hipError_t launch_unet_conv(const ConvArgs &a, int c1, int c2, int co, bool relu
 hipError_t launch_unet_wgrad(const WgradArgs &a, int c1, int c2, int co, bool up2, int nchunks, hipStream_t s);
 hipError_t launch_unet_sum_chunks(const float *part, int nch, int64_t n, float *out, hipStream_t s);
 hipError_t launch_unet_pack(const float *w, int cin, int co, int transposed, uint16_t *out, hipStream_t s);
-hipError_t launch_unet_relu_mask(uint16_t *dy, const uint16_t *y, int64_t n, hipStream_t s);
 hipError_t launch_unet_pool(const uint16_t *in, uint16_t *out, int lx, int ly, int lz, int lc, int batch,
                             hipStream_t s);
-hipError_t launch_unet_pool_bwd(const uint16_t *dc, uint16_t *df, int lx, int ly, int lz, int lc, int batch,
-                                hipStream_t s);
-hipError_t launch_unet_split(const uint16_t *dcat, uint16_t *dskip, uint16_t *dcoarse, int c1, int c2, int lx,
-                             int ly, int lz, int batch, hipStream_t s);
+hipError_t launch_unet_pool_bwd(const uint16_t *dc, const uint16_t *y, uint16_t *df, int lx, int ly, int lz, int lc,
+                                int batch, hipStream_t s);
+hipError_t launch_unet_upsample_bwd(const uint16_t *dup, const uint16_t *y, uint16_t *dcoarse, int lx, int ly, int lz,
+                                    int lc, int batch, hipStream_t s);
 hipError_t launch_unet_head(const uint16_t *x, const float *w, const float *b, float *out, int64_t n,
                             hipStream_t s);
 int unet_head_bwd_blocks(int64_t n);

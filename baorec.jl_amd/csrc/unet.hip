@@ -20,6 +20,7 @@
 #include <string.h>
 
 #include <algorithm>
+#include <type_traits>
 #include <vector>
 
 #include "kernels.hpp"
@@ -31,109 +32,213 @@ typedef __bf16 bf16x8 __attribute__((ext_vector_type(8)));
 typedef float f32x4 __attribute__((ext_vector_type(4)));
 
 __device__ __forceinline__ float bf2f(uint16_t h) { return __uint_as_float((uint32_t)h << 16); }
-// round to nearest even (finite inputs; NaN stays NaN)
-__device__ __forceinline__ uint16_t f2bf(float f) {
-    uint32_t u = __float_as_uint(f);
-    if ((u & 0x7f800000u) == 0x7f800000u) return (uint16_t)((u >> 16) | ((u & 0xffffu) ? 0x40u : 0u));
-    u += 0x7fffu + ((u >> 16) & 1u);
-    return (uint16_t)(u >> 16);
-}
+// round to nearest even, the conversion instruction (the bit operations it
+// replaces were a fourth of a convolution's vector instructions)
+__device__ __forceinline__ uint16_t f2bf(float f) { return __builtin_bit_cast(uint16_t, (__bf16)f); }
 
 __device__ __forceinline__ bf16x8 load8(const uint16_t *p) {
     const uint4 q = *reinterpret_cast<const uint4 *>(p);
     return __builtin_bit_cast(bf16x8, q);
 }
 
+// zeroes the gradients h of outputs y of a ReLU that are not positive
+template <int N>
+__device__ __forceinline__ void relu_mask(uint16_t *h, const uint16_t *y) {
+#pragma unroll
+    for (int j = 0; j < N; j++)
+        if (!(bf2f(y[j]) > 0.f)) h[j] = 0;
+}
+
 // ------------------------------------------------------------ convolution
 
-// Output-channel blocks of 16 per workgroup of k_conv: all of them up to 32
-// channels; one from 64 on (the coarse levels' grids have few voxels, so
-// splitting the channels over workgroups fills the GPU: at 16^3 a launch has
-// 32 voxel workgroups).  Each output keeps its K order, so the same bits.
-__host__ __device__ constexpr int conv_split(int co) { return co >= 64 ? co / 16 : 1; }
+// Tiling of k_conv: a workgroup of four waves computes 16 x MB x ZW voxels
+// (wave: one z plane, MB rows of 16 voxels) times 16 NB CW output channels
+// (CW waves share a plane), the output channels split over NSPLIT workgroups.
+// An operand read from LDS (1 KB) feeds NB products, a weight read (1 KB from
+// L1) MB of them, so MB and NB are as large as LDS (18 (MB + 2) (ZW + 2)
+// voxels) and registers allow with at least two workgroups per CU where the
+// channels permit; the coarse levels' many channels split over workgroups
+// instead, since their grids are few voxels.
+//
+// The whole tile with its halo stands in LDS before the products start (each
+// input voxel is an operand 27 times; read from memory each time, L1 delivered
+// 64 bytes per cycle and CU and bound the kernel).  Weights are the products'
+// first operand and voxels their second, so that a lane ends with four
+// channels of one voxel and stores 8 bytes.  Products per output run in
+// ascending K, one chain.
+//
+// Measured on a batch of four 128^3 grids (before: operands from L1): 16 -> 16
+// channels 156 us (436; 537 MB, 115 us at the copy rate), with a ReLU mask 199,
+// 48 -> 16 532 (1357), 16 -> 48 353 (828; 1.07 GB, 225 us), 96 -> 32 at 64^3
+// 245 (541).  The 16-channel outputs are bound by LDS: every product needs
+// 1 KB at 128 bytes per cycle and CU, 104 us for 16 -> 16, 305 us for 48 -> 16.
+template <int CIN, int CO>
+struct ConvTile {
+    static constexpr int MB = CIN <= 16 ? 8 : CIN <= 96 ? 4 : 2;
+    static constexpr int ZW = CIN == 64 || CIN >= 128 ? 2 : 4, CW = 4 / ZW;
+    static constexpr int NBW = CO / 16 / CW;   // blocks of 16 output channels per wave, over all splits
+    static constexpr int NB = CIN == 128 ? 1 : NBW % 3 == 0 ? 3 : NBW % 2 == 0 ? 2 : 1;
+    static constexpr int NSPLIT = NBW / NB;
+    // uint16 per voxel in LDS.  An operand read (16 voxels at this stride, lane
+    // groups 1 and 3 a piece of 16 bytes further than 0 and 2) is free of bank
+    // conflicts at 2 mod 4 pieces, or at 4 mod 8 with piece p of voxel hx stored
+    // at p ^ swz(hx); 128 channels take 17, for two workgroups per CU.
+    static constexpr bool SWZ = CIN % 64 == 32;
+    static constexpr int VS = CIN == 128 ? CIN + 8 : CIN % 64 == 0 ? CIN + 16 : CIN;
+    static __device__ __forceinline__ int swz(int hx) { return SWZ ? (hx >> 1) & 2 : 0; }
+    static constexpr int HY = MB + 2, HZ = ZW + 2;
+    static constexpr int LDS = 18 * HY * HZ * VS;
+    // the layers' input gradients that may carry a ReLU mask
+    static constexpr bool maskable(bool relu) { return !relu && CIN == CO; }
+    static constexpr int FIT = 160 * 1024 / (2 * LDS);   // workgroups per CU
+    static constexpr int WGS = MB * NB < 16 && FIT >= 3 ? (FIT >= 4 ? 4 : 3) : FIT >= 2 ? 2 : 1;
+};
 
 template <int C1, int C2, int CO, bool RELU, bool UP2>
-__global__ void __launch_bounds__(256) k_conv(ConvArgs a) {
+__global__ void __launch_bounds__(256, (ConvTile<C1 + C2, CO>::WGS)) k_conv(ConvArgs a) {
     constexpr int CIN = C1 + C2;
+    using T = ConvTile<CIN, CO>;
     constexpr int KB = (27 * CIN + 31) / 32;
-    constexpr int NBT = CO / 16, NSPLIT = conv_split(CO), NB = NBT / NSPLIT;
-    constexpr int MB = 2;
-    static_assert(C1 % 8 == 0 && C2 % 8 == 0 && CO % 16 == 0, "channel blocks");
-    const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+    constexpr bool MASKED = T::maskable(RELU);
+    constexpr int NBT = CO / 16, NB = T::NB, MB = T::MB, HY = T::HY, HZ = T::HZ, VS = T::VS;
+    static_assert(C1 % 8 == 0 && C2 % 8 == 0 && CO % 16 == 0 && NB * T::CW * T::NSPLIT == NBT, "channel blocks");
+    __shared__ __align__(16) uint16_t tile[T::LDS];
+    const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
     const int r16 = lane & 15, g = lane >> 4;
     const int nx = 1 << a.lx, ny = 1 << a.ly, nz = 1 << a.lz;
-    const int x = (blockIdx.x * 16 + r16) & (nx - 1);
-    const int y0 = (blockIdx.y * 4 + wave) * MB;
-    const int zb = blockIdx.z / NSPLIT, nb0 = (blockIdx.z % NSPLIT) * NB;   // first output block
-    const int z = zb & (nz - 1), b = zb >> a.lz;
+    const int x0 = blockIdx.x * 16, y0 = blockIdx.y * MB;
+    const int split = blockIdx.z % T::NSPLIT, zb = blockIdx.z / T::NSPLIT;
+    const int lzt = a.lz > (T::ZW == 4 ? 2 : 1) ? a.lz - (T::ZW == 4 ? 2 : 1) : 0;   // log2 of the z tiles
+    const int z0 = (zb & ((1 << lzt) - 1)) * T::ZW;
+    const uint32_t b = zb >> lzt;
+    const int zw = wave % T::ZW, nb0 = (split * T::CW + wave / T::ZW) * NB;   // the wave's plane and first block
+    // weights of chunk kb
+    const uint16_t *wl = a.w + (((uint32_t)nb0 * 4 + g) * 16 + r16) * 8;
+    auto load_w = [&](int kb, bf16x8 *q) {
+#pragma unroll
+        for (int nb = 0; nb < NB; nb++) q[nb] = load8(wl + (uint32_t)(kb * NBT + nb) * 512);
+    };
+    // rings of operand sets, indexed statically.  Weights beyond half of L1
+    // come from L2 and are asked for about 700 cycles of products ahead.
+    constexpr int RW = KB * NBT > 16 ? (MB * NB <= 8 ? 8 : MB * NB <= 16 ? 4 : 2) : MB * NB >= 16 ? 2 : 4;
+    constexpr int RA = MB >= 4 ? 2 : 4;
+    bf16x8 wq[RW][NB], aq[RA][MB];
+#pragma unroll
+    for (int i = 0; i < RW - 1; i++) load_w(i, wq[i]);
+    // the tile and its one-cell periodic halo: channels [coff, coff + C) of it
+    // from src, a grid of sides halved l times; a thread moves one 16-byte piece
+    // of every (256 / S)-th voxel, eight loads in flight
+    auto fill = [&](auto C_, int coff, const uint16_t *src, int l) {
+        constexpr int C = decltype(C_)::value, S = C / 8, STEP = 256 / S, NV = 18 * HY * HZ;
+        constexpr int IT = (NV + STEP - 1) / STEP, U = 8;
+        const int slot = tid % S, v0 = tid / S;
+        int hx = v0 % 18, row = v0 / 18;
+        uint16_t *dst = tile + v0 * VS;
+#pragma unroll
+        for (int i0 = 0; i0 < IT; i0 += U) {
+            f32x4 q[U];
+            int off[U];
+#pragma unroll
+            for (int u = 0; u < U; u++) {
+                const int hz = row / HY, hy = row - hz * HY;
+                const uint32_t xs = (uint32_t)((x0 - 1 + hx) & (nx - 1)) >> l, ys = (uint32_t)((y0 - 1 + hy) & (ny - 1)) >> l;
+                const uint32_t zs = (uint32_t)((z0 - 1 + hz) & (nz - 1)) >> l;
+                const uint32_t zy = (((b << (a.lz - l)) + zs) << (a.ly - l)) + ys;
+                off[u] = (coff / 8 + slot ^ T::swz(hx)) * 8;
+                if (i0 + u < IT && v0 + (i0 + u) * STEP < NV)
+                    q[u] = *reinterpret_cast<const f32x4 *>(src + ((zy << (a.lx - l)) + xs) * C + slot * 8);
+                hx += STEP % 18;
+                row += STEP / 18;
+                if (STEP % 18 && hx >= 18) {
+                    hx -= 18;
+                    row++;
+                }
+            }
+#pragma unroll
+            for (int u = 0; u < U; u++)
+                if (i0 + u < IT && v0 + (i0 + u) * STEP < NV)
+                    *reinterpret_cast<f32x4 *>(dst + (i0 + u) * STEP * VS + off[u]) = q[u];
+        }
+    };
+    fill(std::integral_constant<int, C1>{}, 0, a.in1, 0);
+    if constexpr (C2 > 0) fill(std::integral_constant<int, C2>{}, C1, a.in2, UP2 ? 1 : 0);
+    __syncthreads();
+    const int x = x0 + r16, z = z0 + zw;   // the lane's voxels: y0 + m
+    const uint32_t vox0 = (((((b << a.lz) + z) << a.ly) + y0) << a.lx) + x;   // (the launcher checks the sizes)
+    uint2 mk[MB][NB];   // in flight during the products
+    if (MASKED && a.mask)
+#pragma unroll
+        for (int m = 0; m < MB; m++)
+#pragma unroll
+            for (int nb = 0; nb < NB; nb++) {
+                mk[m][nb] = make_uint2(0u, 0u);
+                if (x < nx && y0 + m < ny && z < nz)
+                    mk[m][nb] = *reinterpret_cast<const uint2 *>(a.mask + (size_t)(vox0 + m * nx) * CO +
+                                                                 (nb0 + nb) * 16 + 4 * g);
+            }
     f32x4 acc[MB][NB];
 #pragma unroll
     for (int m = 0; m < MB; m++)
 #pragma unroll
         for (int nb = 0; nb < NB; nb++) acc[m][nb] = f32x4{0.f, 0.f, 0.f, 0.f};
-    // operands of chunk kb: B (weights) and A (the input at the lane's tap and
-    // channel group), 32-bit element offsets (the launcher checks the sizes)
-    auto load_chunk = [&](int kb, bf16x8 *bv, bf16x8 *av) {
-        const int kc = kb * 32 + g * 8;
-        int t = kc / CIN;
-        const int ci = kc - t * CIN;
-        if (t > 26) t = 26;   // padding columns of K: their weights are zero
-        const int dx = t % 3 - 1, dy = (t / 3) % 3 - 1, dz = t / 9 - 1;
-        const uint32_t xs = (uint32_t)((x + dx) & (nx - 1)), zs = (uint32_t)((z + dz) & (nz - 1));
+    // inputs of chunk kb: lane group g holds channels ci .. ci + 7 of tap t
+    const uint16_t *al[3];
 #pragma unroll
-        for (int nb = 0; nb < NB; nb++) bv[nb] = load8(a.w + ((uint32_t)((kb * NBT + nb0 + nb) * 4 + g) * 16 + r16) * 8);
+    for (int dx = 0; dx < 3; dx++)
+        al[dx] = tile + (zw * HY * 18 + r16) * VS + (CIN % 16 == 0 ? (g ^ T::swz(r16 + dx)) * 8 : 0);
+    const int m1 = -(g & 1), m2 = -(g >> 1);
+    auto load_a = [&](int kb, bf16x8 *q) {
+        auto off = [&](int gg) {   // from al
+            const int kc = kb * 32 + gg * 8;
+            const int t = kc / CIN, ci = kc - t * CIN;
+            const int tt = t > 26 ? 26 : t;   // padding columns of K: their weights are zero
+            return ((tt / 9 * HY + tt / 3 % 3) * 18 + tt % 3) * VS + ci - (CIN % 16 == 0 ? gg * 8 : 0);
+        };
+        const int t0 = kb * 32 / CIN;
+        const uint16_t *p = al[t0 > 26 ? 2 : t0 % 3] + off(0);
+        // the groups' taps differ where 32 is not within one tap's channels
+        if (CIN % 32 != 0) p += m2 & (off(2) - off(0));
+        if (CIN % 16 != 0) p += (m1 & ~m2 & (off(1) - off(0))) + (m1 & m2 & (off(3) - off(2)));
 #pragma unroll
-        for (int m = 0; m < MB; m++) {
-            const uint32_t ys = (uint32_t)((y0 + m + dy) & (ny - 1));
-            const uint16_t *src;
-            if (C2 == 0 || ci < C1) {
-                src = a.in1 + ((((uint32_t)b * nz + zs) * ny + ys) * nx + xs) * C1 + ci;
-            } else if (UP2) {
-                const uint32_t cx = nx >> 1, cy = ny >> 1, cz = nz >> 1;
-                src = a.in2 + ((((uint32_t)b * cz + (zs >> 1)) * cy + (ys >> 1)) * cx + (xs >> 1)) * C2 + (ci - C1);
-            } else {
-                src = a.in2 + ((((uint32_t)b * nz + zs) * ny + ys) * nx + xs) * C2 + (ci - C1);
-            }
-            av[m] = load8(src);
-        }
+        for (int m = 0; m < MB; m++) q[m] = *reinterpret_cast<const bf16x8 *>(p + m * 18 * VS);
     };
-    // the loads of chunks kb + 1 .. kb + PF are in flight during chunk kb's
-    // products (a ring of PF + 1 operand sets, indexed statically)
-    constexpr int PF = 3, RING = PF + 1;
-    bf16x8 bq[RING][NB], aq[RING][MB];
 #pragma unroll
-    for (int i = 0; i < PF; i++)
-        if (i < KB) load_chunk(i, bq[i], aq[i]);
-    for (int kb0 = 0; kb0 < KB; kb0 += RING) {
+    for (int i = 0; i < RA - 1; i++) load_a(i, aq[i]);
 #pragma unroll
-        for (int u = 0; u < RING; u++) {
-            const int kb = kb0 + u;
-            if (kb >= KB) break;
-            if (kb + PF < KB) load_chunk(kb + PF, bq[(u + PF) % RING], aq[(u + PF) % RING]);
+    for (int kb = 0; kb < KB; kb++) {
+        if (kb + RW - 1 < KB) load_w(kb + RW - 1, wq[(kb + RW - 1) % RW]);
+        if (kb + RA - 1 < KB) load_a(kb + RA - 1, aq[(kb + RA - 1) % RA]);
 #pragma unroll
-            for (int m = 0; m < MB; m++)
+        for (int m = 0; m < MB; m++)
 #pragma unroll
-                for (int nb = 0; nb < NB; nb++)
-                    acc[m][nb] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(aq[u][m], bq[u][nb], acc[m][nb], 0, 0, 0);
-        }
+            for (int nb = 0; nb < NB; nb++)
+                acc[m][nb] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(wq[kb % RW][nb], aq[kb % RA][m], acc[m][nb], 0, 0, 0);
     }
-    // lane holds rows (voxels) 4g .. 4g+3 of column (channel) r16
+    // lane holds channels 4g .. 4g+3 of voxel r16
+    if (x >= nx || z >= nz) return;
 #pragma unroll
-    for (int m = 0; m < MB; m++) {
-        const int y = y0 + m;
-        if (y >= ny) continue;
+    for (int nb = 0; nb < NB; nb++) {
+        const int co = (nb0 + nb) * 16 + 4 * g;
+        f32x4 bias = f32x4{0.f, 0.f, 0.f, 0.f};
+        if (a.bias)
 #pragma unroll
-        for (int nb = 0; nb < NB; nb++) {
-            const int co = (nb0 + nb) * 16 + r16;
-            const float bias = a.bias ? a.bias[co] : 0.f;
+            for (int r = 0; r < 4; r++) bias[r] = a.bias[co + r];
+        // channels [csplit, CO) go to out2
+        const bool second = !RELU && (nb0 + nb) * 16 >= a.csplit;
+        const int stride = RELU ? CO : second ? CO - a.csplit : a.csplit;
+        uint16_t *dst = (second ? a.out2 - a.csplit : a.out) + ((size_t)vox0 * stride + co);
+#pragma unroll
+        for (int m = 0; m < MB; m++, dst += (size_t)nx * stride) {
+            if (y0 + m >= ny) break;
+            uint16_t h[4];
 #pragma unroll
             for (int r = 0; r < 4; r++) {
-                const int xo = blockIdx.x * 16 + 4 * g + r;
-                if (xo >= nx) continue;
-                float v = acc[m][nb][r] + bias;
+                float v = acc[m][nb][r] + bias[r];
                 if (RELU) v = fmaxf(v, 0.f);
-                a.out[((((size_t)b * nz + z) * ny + y) * nx + xo) * CO + co] = f2bf(v);
+                h[r] = f2bf(v);
             }
+            if (MASKED && a.mask) relu_mask<4>(h, reinterpret_cast<const uint16_t *>(&mk[m][nb]));
+            *reinterpret_cast<uint2 *>(dst) = make_uint2(h[0] | (uint32_t)h[1] << 16, h[2] | (uint32_t)h[3] << 16);
         }
     }
 }
@@ -371,85 +476,86 @@ __global__ void k_pack(const float *__restrict__ w, int cin, int co, int transpo
 
 // ------------------------------------------------------------ elementwise
 
-// dy *= (y > 0)
-__global__ void k_relu_mask(uint16_t *__restrict__ dy, const uint16_t *__restrict__ y, int64_t n) {
-    for (int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x; i < n; i += (int64_t)gridDim.x * blockDim.x)
-        if (!(bf2f(y[i]) > 0.f)) dy[i] = 0;
-}
+// The pooling and upsampling kernels below take a thread per voxel and 8
+// channels (16-byte accesses; c = 1 << lc channels) and are bound by their
+// traffic.
 
-// 2x2x2 average pooling of a [b][z][y][x][c] tensor (c = 1 << lc)
-__global__ void k_pool(const uint16_t *__restrict__ in, uint16_t *__restrict__ out, int lx, int ly, int lz, int lc,
+// 2x2x2 average pooling of a [b][z][y][x][c] tensor: nout voxels and 8-channel
+// groups of the result
+__global__ void k_pool(const uint16_t *__restrict__ in, uint16_t *__restrict__ out, int lx, int ly, int lc,
                        int64_t nout) {
-    const int cx = 1 << (lx - 1), cy = 1 << (ly - 1), cz = 1 << (lz - 1), C = 1 << lc;
+    const int lg = lc - 3;   // log2 of the channel groups
     for (int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x; i < nout; i += (int64_t)gridDim.x * blockDim.x) {
-        const int c = (int)(i & (C - 1));
-        int64_t v = i >> lc;
-        const int x = (int)(v % cx);
-        v /= cx;
-        const int y = (int)(v % cy);
-        v /= cy;
-        const int z = (int)(v % cz);
-        const int64_t b = v / cz;
-        const int nx = cx * 2, ny = cy * 2, nz = cz * 2;
-        float s = 0.f;
+        const int c = (int)(i & ((1 << lg) - 1));
+        const int64_t v = i >> lg;
+        const int64_t x = v & ((1 << (lx - 1)) - 1), y = (v >> (lx - 1)) & ((1 << (ly - 1)) - 1), bz = v >> (lx + ly - 2);
+        float s[8] = {0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f};
+#pragma unroll
         for (int d = 0; d < 8; d++) {
-            const int xx = 2 * x + (d & 1), yy = 2 * y + ((d >> 1) & 1), zz = 2 * z + (d >> 2);
-            s += bf2f(in[((((size_t)b * nz + zz) * ny + yy) * nx + xx) * C + c]);
+            // batch and z together: the fine z of item b is 2 (b cz + z) + dz
+            const int64_t f = ((((2 * bz + (d >> 2)) << ly) + 2 * y + ((d >> 1) & 1)) << lx) + 2 * x + (d & 1);
+            const uint4 q = *reinterpret_cast<const uint4 *>(in + (f << lc) + c * 8);
+            const uint16_t *h = reinterpret_cast<const uint16_t *>(&q);
+#pragma unroll
+            for (int j = 0; j < 8; j++) s[j] += bf2f(h[j]);
         }
-        out[i] = f2bf(s * 0.125f);
+        uint4 o;
+        uint16_t *oh = reinterpret_cast<uint16_t *>(&o);
+#pragma unroll
+        for (int j = 0; j < 8; j++) oh[j] = f2bf(s[j] * 0.125f);
+        *reinterpret_cast<uint4 *>(out + i * 8) = o;
     }
 }
 
-// dfine += dcoarse / 8 at the parent (the adjoint of k_pool), fine side given
-__global__ void k_pool_bwd(const uint16_t *__restrict__ dc, uint16_t *__restrict__ df, int lx, int ly, int lz,
-                           int lc, int64_t nfine) {
-    const int nx = 1 << lx, ny = 1 << ly, nz = 1 << lz, C = 1 << lc;
+// dfine += dcoarse / 8 at the parent (the adjoint of k_pool), then zero where
+// the fine output y is not positive: dfine's last term, so masked here
+__global__ void k_pool_bwd(const uint16_t *__restrict__ dc, const uint16_t *__restrict__ y, uint16_t *__restrict__ df,
+                           int lx, int ly, int lc, int64_t nfine) {
+    const int lg = lc - 3;
     for (int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x; i < nfine; i += (int64_t)gridDim.x * blockDim.x) {
-        const int c = (int)(i & (C - 1));
-        int64_t v = i >> lc;
-        const int x = (int)(v % nx);
-        v /= nx;
-        const int y = (int)(v % ny);
-        v /= ny;
-        const int z = (int)(v % nz);
-        const int64_t b = v / nz;
-        const float p = bf2f(dc[((((size_t)b * (nz >> 1) + (z >> 1)) * (ny >> 1) + (y >> 1)) * (nx >> 1) + (x >> 1)) * C + c]);
-        df[i] = f2bf(bf2f(df[i]) + p * 0.125f);
+        const int c = (int)(i & ((1 << lg) - 1));
+        const int64_t v = i >> lg;
+        const int64_t vx = v & ((1 << lx) - 1), vy = (v >> lx) & ((1 << ly) - 1), bz = v >> (lx + ly);
+        const int64_t p = ((((bz >> 1) << (ly - 1)) + (vy >> 1)) << (lx - 1)) + (vx >> 1);
+        const uint4 qc = *reinterpret_cast<const uint4 *>(dc + (p << lc) + c * 8);
+        const uint4 qy = *reinterpret_cast<const uint4 *>(y + i * 8);
+        uint4 qf = *reinterpret_cast<const uint4 *>(df + i * 8);
+        const uint16_t *hc = reinterpret_cast<const uint16_t *>(&qc);
+        uint16_t *hf = reinterpret_cast<uint16_t *>(&qf);
+#pragma unroll
+        for (int j = 0; j < 8; j++) hf[j] = f2bf(bf2f(hf[j]) + bf2f(hc[j]) * 0.125f);
+        relu_mask<8>(hf, reinterpret_cast<const uint16_t *>(&qy));
+        *reinterpret_cast<uint4 *>(df + i * 8) = qf;
     }
 }
 
-// Gradient of a decoder input [skip C1 | upsampled C2] (full resolution,
-// C1 + C2 channels): dskip = first C1 channels (overwrites); dcoarse = sum of
-// the last C2 channels over the 8 children of each coarse cell (overwrites).
-__global__ void k_split_skip(const uint16_t *__restrict__ dcat, uint16_t *__restrict__ dskip, int C1, int C2,
-                             int64_t nvox) {
-    const int C = C1 + C2;
-    for (int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x; i < nvox * C1; i += (int64_t)gridDim.x * blockDim.x) {
-        const int64_t v = i / C1;
-        const int c = (int)(i - v * C1);
-        dskip[i] = dcat[v * C + c];
-    }
-}
-__global__ void k_split_coarse(const uint16_t *__restrict__ dcat, uint16_t *__restrict__ dcoarse, int C1, int C2,
-                               int lx, int ly, int lz, int64_t ncoarse) {
-    const int C = C1 + C2;
-    const int cx = 1 << (lx - 1), cy = 1 << (ly - 1), cz = 1 << (lz - 1);
-    const int nx = cx * 2, ny = cy * 2, nz = cz * 2;
-    for (int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x; i < ncoarse * C2; i += (int64_t)gridDim.x * blockDim.x) {
-        const int c = (int)(i % C2);
-        int64_t v = i / C2;
-        const int x = (int)(v % cx);
-        v /= cx;
-        const int y = (int)(v % cy);
-        v /= cy;
-        const int z = (int)(v % cz);
-        const int64_t b = v / cz;
-        float s = 0.f;
+// Gradient of a decoder's upsampled input (full resolution, C channels):
+// dcoarse = its sum over the 8 children of each coarse cell (overwrites), zero
+// where the coarse output y is not positive.  C / 8 a power of two.
+__global__ void k_upsample_bwd(const uint16_t *__restrict__ dup, const uint16_t *__restrict__ y,
+                               uint16_t *__restrict__ dcoarse, int lx, int ly, int lc, int64_t ncoarse) {
+    const int lg = lc - 3;
+    for (int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x; i < ncoarse; i += (int64_t)gridDim.x * blockDim.x) {
+        const int c = (int)(i & ((1 << lg) - 1));
+        const int64_t v = i >> lg;
+        const int64_t x = v & ((1 << (lx - 1)) - 1), vy = (v >> (lx - 1)) & ((1 << (ly - 1)) - 1);
+        const int64_t bz = v >> (lx + ly - 2);
+        float s[8] = {0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f};
+#pragma unroll
         for (int d = 0; d < 8; d++) {
-            const int xx = 2 * x + (d & 1), yy = 2 * y + ((d >> 1) & 1), zz = 2 * z + (d >> 2);
-            s += bf2f(dcat[((((size_t)b * nz + zz) * ny + yy) * nx + xx) * C + C1 + c]);
+            const int64_t f = ((((2 * bz + (d >> 2)) << ly) + 2 * vy + ((d >> 1) & 1)) << lx) + 2 * x + (d & 1);
+            const uint4 q = *reinterpret_cast<const uint4 *>(dup + (f << lc) + c * 8);
+            const uint16_t *h = reinterpret_cast<const uint16_t *>(&q);
+#pragma unroll
+            for (int j = 0; j < 8; j++) s[j] += bf2f(h[j]);
         }
-        dcoarse[i] = f2bf(s);
+        const uint4 qy = *reinterpret_cast<const uint4 *>(y + i * 8);
+        uint4 o;
+        uint16_t *oh = reinterpret_cast<uint16_t *>(&o);
+#pragma unroll
+        for (int j = 0; j < 8; j++) oh[j] = f2bf(s[j]);
+        relu_mask<8>(oh, reinterpret_cast<const uint16_t *>(&qy));
+        *reinterpret_cast<uint4 *>(dcoarse + i * 8) = o;
     }
 }
 
@@ -467,7 +573,8 @@ __global__ void k_head(const uint16_t *__restrict__ x, const float *__restrict__
         out[i] = s;
     }
 }
-// dx[v][c] = w[c] dout[v]; per-block partials of dw[c] = sum_v x[v][c] dout[v]
+// dx[v][c] = w[c] dout[v], zero where x[v][c] is not positive (x a ReLU's
+// output); per-block partials of dw[c] = sum_v x[v][c] dout[v]
 // and db = sum_v dout[v] (17 values per block, summed later by k_sum_rows).
 // Bound by its traffic (32 B read and written and 4 B read per voxel): a
 // voxel's 16 channels move as two 16-byte accesses each way.
@@ -492,6 +599,7 @@ __global__ void __launch_bounds__(256) k_head_bwd(const uint16_t *__restrict__ x
             acc[c] += bf2f(h[c]) * d;
             oh[c] = f2bf(wr[c] * d);
         }
+        relu_mask<16>(oh, h);
         acc[16] += d;
         *reinterpret_cast<uint4 *>(dx + i * 16) = o[0];
         *reinterpret_cast<uint4 *>(dx + i * 16 + 8) = o[1];
@@ -742,9 +850,12 @@ hipError_t launch_unet_conv(const ConvArgs &a, int c1, int c2, int co, bool relu
     // k_conv addresses its inputs with 32-bit element offsets
     const int cmax = c1 > c2 ? c1 : c2;
     if ((int64_t)batch * nx * ny * nz * cmax >= ((int64_t)1 << 31)) return hipErrorInvalidValue;
-    dim3 grid((unsigned)((nx + 15) / 16), (unsigned)((ny + 7) / 8), (unsigned)(nz * batch * conv_split(co)));
 #define LAUNCH(C1_, C2_, CO_, UP_)                                                                        \
     if (c1 == C1_ && c2 == C2_ && co == CO_ && up2 == UP_) {                                              \
+        using T = ConvTile<C1_ + C2_, CO_>;                                                               \
+        if (a.mask && !T::maskable(relu)) return hipErrorInvalidValue;                                    \
+        const dim3 grid((unsigned)((nx + 15) / 16), (unsigned)((ny + T::MB - 1) / T::MB),                 \
+                        (unsigned)((nz + T::ZW - 1) / T::ZW * batch * T::NSPLIT));                        \
         if (relu)                                                                                         \
             hipLaunchKernelGGL((k_conv<C1_, C2_, CO_, true, UP_>), grid, dim3(256), 0, s, a);             \
         else                                                                                              \
@@ -782,30 +893,23 @@ hipError_t launch_unet_pack(const float *w, int cin, int co, int transposed, uin
     hipLaunchKernelGGL(k_pack, dim3(blocks(total)), dim3(256), 0, s, w, cin, co, transposed, out);
     return hipGetLastError();
 }
-hipError_t launch_unet_relu_mask(uint16_t *dy, const uint16_t *y, int64_t n, hipStream_t s) {
-    hipLaunchKernelGGL(k_relu_mask, dim3(blocks(n)), dim3(256), 0, s, dy, y, n);
-    return hipGetLastError();
-}
+// lx .. lz: log2 of the fine grid's sides; lc of the channels
 hipError_t launch_unet_pool(const uint16_t *in, uint16_t *out, int lx, int ly, int lz, int lc, int batch,
                             hipStream_t s) {
-    const int64_t n = ((int64_t)batch << (lx + ly + lz - 3)) << lc;
-    hipLaunchKernelGGL(k_pool, dim3(blocks(n)), dim3(256), 0, s, in, out, lx, ly, lz, lc, n);
+    const int64_t n = ((int64_t)batch << (lx + ly + lz - 3)) << (lc - 3);
+    hipLaunchKernelGGL(k_pool, dim3(blocks(n)), dim3(256), 0, s, in, out, lx, ly, lc, n);
     return hipGetLastError();
 }
-hipError_t launch_unet_pool_bwd(const uint16_t *dc, uint16_t *df, int lx, int ly, int lz, int lc, int batch,
-                                hipStream_t s) {
-    const int64_t n = ((int64_t)batch << (lx + ly + lz)) << lc;
-    hipLaunchKernelGGL(k_pool_bwd, dim3(blocks(n)), dim3(256), 0, s, dc, df, lx, ly, lz, lc, n);
+hipError_t launch_unet_pool_bwd(const uint16_t *dc, const uint16_t *y, uint16_t *df, int lx, int ly, int lz, int lc,
+                                int batch, hipStream_t s) {
+    const int64_t n = ((int64_t)batch << (lx + ly + lz)) << (lc - 3);
+    hipLaunchKernelGGL(k_pool_bwd, dim3(blocks(n)), dim3(256), 0, s, dc, y, df, lx, ly, lc, n);
     return hipGetLastError();
 }
-hipError_t launch_unet_split(const uint16_t *dcat, uint16_t *dskip, uint16_t *dcoarse, int c1, int c2, int lx,
-                             int ly, int lz, int batch, hipStream_t s) {
-    const int64_t nv = (int64_t)batch << (lx + ly + lz);
-    hipLaunchKernelGGL(k_split_skip, dim3(blocks(nv * c1)), dim3(256), 0, s, dcat, dskip, c1, c2, nv);
-    hipError_t e = hipGetLastError();
-    if (e != hipSuccess) return e;
-    const int64_t nc = nv >> 3;
-    hipLaunchKernelGGL(k_split_coarse, dim3(blocks(nc * c2)), dim3(256), 0, s, dcat, dcoarse, c1, c2, lx, ly, lz, nc);
+hipError_t launch_unet_upsample_bwd(const uint16_t *dup, const uint16_t *y, uint16_t *dcoarse, int lx, int ly, int lz,
+                                    int lc, int batch, hipStream_t s) {
+    const int64_t n = ((int64_t)batch << (lx + ly + lz - 3)) << (lc - 3);
+    hipLaunchKernelGGL(k_upsample_bwd, dim3(blocks(n)), dim3(256), 0, s, dup, y, dcoarse, lx, ly, lc, n);
     return hipGetLastError();
 }
 hipError_t launch_unet_head(const uint16_t *x, const float *w, const float *b, float *out, int64_t n,
@@ -907,7 +1011,7 @@ struct UNet {
     float h_train = 0.f;
     // activations and gradients of the last forward/backward shape
     int batch = 0, lx = -1, ly = -1, lz = -1;
-    uint16_t *X = nullptr, *A[kNL] = {}, *Pl[3] = {}, *dA[kNL] = {}, *dP[3] = {}, *dcat[3] = {};
+    uint16_t *X = nullptr, *A[kNL] = {}, *Pl[3] = {}, *dA[kNL] = {}, *dP[3] = {}, *dup[3] = {};
     float *out = nullptr, *dout = nullptr, *wpart = nullptr, *hpart = nullptr, *cpart = nullptr;
     size_t wpart_n = 0;
     size_t cpart_off[kNL] = {};   // each layer's bias-gradient partials in cpart
@@ -937,8 +1041,8 @@ struct UNet {
         for (int i = 0; i < 3; i++) {
             (void)hipFree(Pl[i]);
             (void)hipFree(dP[i]);
-            (void)hipFree(dcat[i]);
-            Pl[i] = dP[i] = dcat[i] = nullptr;
+            (void)hipFree(dup[i]);
+            Pl[i] = dP[i] = dup[i] = nullptr;
         }
         (void)hipFree(out);
         (void)hipFree(dout);
@@ -1001,7 +1105,7 @@ struct UNet {
             const int c = 16 << l;
             UCHK(dalloc(&Pl[l], (size_t)nvox(l + 1) * c));
             UCHK(dalloc(&dP[l], (size_t)nvox(l + 1) * c));
-            UCHK(dalloc(&dcat[l], (size_t)nvox(l) * (c + 2 * c)));
+            UCHK(dalloc(&dup[l], (size_t)nvox(l) * 2 * c));
         }
         UCHK(dalloc(&out, nvox(0)));
         UCHK(dalloc(&dout, nvox(0)));
@@ -1030,6 +1134,7 @@ struct UNet {
             a.w = wp[i];
             a.bias = par + boff[i];
             a.out = A[i];
+            a.csplit = d.co;
             a.lx = lv(d.level, 0);
             a.ly = lv(d.level, 1);
             a.lz = lv(d.level, 2);
@@ -1053,10 +1158,8 @@ struct UNet {
         for (int i = kNL - 1; i >= 0; i--) {
             const LayerDef &d = kLayers[i];
             const int l = d.level;
-            const int64_t n = nvox(l);
             const int x = lv(l, 0), y = lv(l, 1), z = lv(l, 2);
-            UCHK(launch_unet_relu_mask(dA[i], A[i], n * d.co, s));
-            // weight gradient
+            // weight gradient (dA[i] is complete and masked by its ReLU)
             const int cin = d.c1 + d.c2;
             const int64_t nbricks = (int64_t)(((1 << x) + 15) >> 4) * (((1 << y) + 3) >> 2) * (((1 << z) + 3) >> 2) * batch;
             int nch = (int)(nbricks < 256 ? nbricks : 256);
@@ -1091,19 +1194,22 @@ struct UNet {
             a.lx = x;
             a.ly = y;
             a.lz = z;
+            a.csplit = cin;
             if (d.c2 > 0) {   // decoder: [skip | upsampled coarse]
-                const int sl = l;   // dcat index = level
-                a.out = dcat[sl];
+                a.out = dA[d.in1];   // the pooling's part is added, and the mask applied, further down
+                a.out2 = dup[l];
+                a.csplit = d.c1;
                 UCHK(launch_unet_conv(a, d.co, 0, cin, false, false, batch, s));
-                UCHK(launch_unet_split(dcat[sl], dA[d.in1], dA[d.in2], d.c1, d.c2, x, y, z, batch, s));
+                UCHK(launch_unet_upsample_bwd(dup[l], A[d.in2], dA[d.in2], x, y, z, 5 + l, batch, s));
             } else if (d.in1 <= -2) {   // encoder input from pooling
                 const int pl = -d.in1 - 2;
                 a.out = dP[pl];
                 UCHK(launch_unet_conv(a, d.co, 0, cin, false, false, batch, s));
                 const int sk = 2 * pl + 1;   // the pooled skip layer
-                UCHK(launch_unet_pool_bwd(dP[pl], dA[sk], lv(pl, 0), lv(pl, 1), lv(pl, 2), 4 + pl, batch, s));
+                UCHK(launch_unet_pool_bwd(dP[pl], A[sk], dA[sk], lv(pl, 0), lv(pl, 1), lv(pl, 2), 4 + pl, batch, s));
             } else {
                 a.out = dA[d.in1];
+                a.mask = A[d.in1];
                 UCHK(launch_unet_conv(a, d.co, 0, cin, false, false, batch, s));
             }
         }

@@ -120,6 +120,13 @@ def test_unet_layers_match_oracle_on_their_inputs(ctx, shape):
             assert_bf16_close(U.bf16_bits(dA[i1]), dx * (A[i1] > 0), f"input gradient {i}")
 
 
+@pytest.mark.parametrize("shape", [(1, 16, 32, 64), (2, 32, 16, 32)])
+def test_unet_layers_over_several_tiles(ctx, shape):
+    """The same on grids of several convolution tiles along each axis, whose
+    halos then come from the neighbouring tiles and from the periodic wrap."""
+    test_unet_layers_match_oracle_on_their_inputs(ctx, shape)
+
+
 @pytest.mark.parametrize("shape", [(3, 64, 64, 64), (5, 32, 16, 128)])
 def test_weight_gradients_over_many_bricks(ctx, shape):
     """Weight gradients where a workgroup streams several bricks (and the last
