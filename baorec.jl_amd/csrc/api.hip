@@ -748,8 +748,8 @@ void iterate_all(baorec_ctx *c, const Grid &G, const baorec_params *p, Slot *slo
 }
 
 // compute_displacements grids of nb catalogs: 3 floats per cell (Psi_x,
-// Psi_y, Psi_z), catalog b at disp + 3 b R.  The k and x tables come from
-// slot[0] (the catalogs share one box).
+// Psi_y, Psi_z; in bricks, see GatherArgs), catalog b at disp + 3 b R.  The
+// k and x tables come from slot[0] (the catalogs share one box).
 void displacement_grid(baorec_ctx *c, const Grid &G, int kind, Slot *slot, const float *field, float *disp,
                        bool c0_ready = false, int nb = 1, const Work *Wp = nullptr) {
     FFTBufs f = fft_bufs(c, G);

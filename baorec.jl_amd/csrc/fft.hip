@@ -244,7 +244,10 @@ k_x_c2r(XInvArgs a) {
     const int64_t line = (int64_t)blockIdx.x * S::LPW + li;
     const bool valid = line < nlines;
     const int b = blockIdx.y;
-    const int iy = (int)(line % a.ny), iz = (int)(line / a.ny);
+    // displacement bricks: four consecutive lines are the 2 x 2 (y, z) rows of a row of bricks
+    const int64_t pr = line >> 2;
+    const int iy = EPI == XE_DISP ? (int)(pr % (a.ny / 2)) * 2 + (li & 1) : (int)(line % a.ny);
+    const int iz = EPI == XE_DISP ? (int)(pr / (a.ny / 2)) * 2 + ((li >> 1) & 1) : (int)(line / a.ny);
     const float *kx = a.ktab + b * a.ktabStride;
     const int64_t rbase = b * a.rstride + line * (2 * M);
     LayLine lay{li * S::LS};
@@ -366,17 +369,30 @@ k_x_c2r(XInvArgs a) {
         }
     }
     if constexpr (EPI == XE_DISP) {
-        // 12-byte cells (Psi_x, Psi_y, Psi_z): cells 2m and 2m + 1 are three
-        // float2 (rbase is even, so 3 * rbase floats is 8-byte aligned)
-        if (!valid) return;
-        float2 *o2 = reinterpret_cast<float2 *>(a.out + 3 * rbase);
+        // bricks of 2 x 2 x 2 cells (GatherArgs): register i of four lines is
+        // TPL consecutive bricks, which meet in LDS (two buffers, a barrier per
+        // register) and leave as one run of memory; 8-byte stores straight into
+        // the bricks would touch each line of memory from three instructions of
+        // two waves.  Sides are powers of two of at least 16: no partial workgroup.
+        static_assert(S::LPW % 4 == 0 && S::LPW * S::LS >= 2 * 3 * S::NT, "staging");
+        float2 *o2 = reinterpret_cast<float2 *>(a.out + 3 * b * a.rstride);
+        const int sl = ((li >> 2) * TPL + t) * 12 + 3 * (li & 3);   // x pairs of line li: y, z bits
+        const int64_t row0 = (int64_t)blockIdx.x * (S::LPW / 4) * M;   // first brick of the workgroup's rows
+        __syncthreads();
 #pragma unroll
         for (int i = 0; i < 8; i++) {
-            const int m = PI::out_pos(t, i);
+            float2 *st = lds + (i & 1) * 3 * S::NT;
             const float3 d0 = disp[i][0], d1 = disp[i][1];
-            o2[3 * m] = make_float2(d0.x, d0.y);
-            o2[3 * m + 1] = make_float2(d0.z, d1.x);
-            o2[3 * m + 2] = make_float2(d1.y, d1.z);
+            st[sl] = make_float2(d0.x, d0.y);
+            st[sl + 1] = make_float2(d0.z, d1.x);
+            st[sl + 2] = make_float2(d1.y, d1.z);
+            __syncthreads();
+            const int m0 = PI::out_pos(0, i);
+#pragma unroll
+            for (int u = 0; u < 3; u++) {
+                const int j = tid + u * S::NT, g = j / (TPL * 12), r = j - g * (TPL * 12);
+                o2[(row0 + (int64_t)g * M + m0) * 12 + r] = st[j];
+            }
         }
         return;
     }

@@ -64,7 +64,7 @@ enum XEpi : int {
     XE_OD_RAND = 2,   // data - alpha*randoms normalisation (src/recon.jl:78-85)
     XE_ITER_LOCAL = 3,// delta_r = delta_s - (x^2 a + x b + c) / x^2 (inputs A, B, C)
     XE_ITER_FIXED = 4,// delta_r = delta_s - fac * D
-    XE_DISP = 5,      // (Psi_x, Psi_y, Psi_z) per cell, 12 bytes
+    XE_DISP = 5,      // (Psi_x, Psi_y, Psi_z) per cell, 12 bytes, in bricks (GatherArgs)
 };
 
 constexpr int kMaxXIn = 6;
@@ -206,7 +206,9 @@ int scatter_tile_max();
 struct GatherArgs {
     const float *x, *y, *z;
     int64_t n;
-    const float *disp;          // displacement grid, (Psi_x, Psi_y, Psi_z) per cell
+    // displacement grid, (Psi_x, Psi_y, Psi_z) per cell in bricks of 2 x 2 x 2:
+    // float 24 (x/2 + nx/2 (y/2 + ny/2 (z/2))) + 3 (x%2 + 2 (y%2) + 4 (z%2))
+    const float *disp;
     const Slot *slot;
     int nx, ny, nz;
     int field;                  // 0 disp, 1 rsd, 2 sum

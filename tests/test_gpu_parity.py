@@ -352,6 +352,32 @@ def test_read_shifts_explicit_field(ctx):
         assert rms3(got, exp) < 1e-5 * scale + 1e-6
 
 
+@pytest.mark.parametrize("shape", [(16, 16, 16), (64, 16, 32), (16, 128, 64), (32, 16, 1024), (16, 32, 512)])
+def test_read_shifts_over_grid_shapes(ctx, shape):
+    """Displacements written in 2 x 2 x 2 bricks and read by k_gather on grids
+    of every x-pass shape: particles in every cell of the first and last two
+    planes of each axis (both halves of a brick, the periodic wrap) and at
+    random, on cell corners and inside."""
+    nz, ny, nx = shape
+    rng = np.random.default_rng(43)
+    field = rng.standard_normal(shape).astype(F32)
+    L = np.array([4.0 * nx, 4.0 * ny, 4.0 * nz], F32)
+    kw = dict(box_kw(500.0), box_size=[float(v) for v in L], box_min=[0.0] * 3)
+    ends = [np.array([0, 1, n - 2, n - 1]) for n in (nx, ny, nz)]
+    cells = np.stack(np.meshgrid(*ends, indexing="ij"), -1).reshape(-1, 3)
+    frac = np.concatenate([np.zeros_like(cells), rng.random(cells.shape)])
+    pos = (np.concatenate([cells, cells]) + frac) * 4.0
+    pos = np.concatenate([pos, rng.random((2000, 3)) * L])
+    pos = np.minimum(pos.astype(F32), np.nextafter(L, F32(0)))
+    x, y, z = (np.ascontiguousarray(pos[:, a]) for a in range(3))
+    rec = bh.IterativeRecon(**kw)
+    got = bh.read_shifts(rec, x, y, z, field, field="disp")
+    exp = orc.read_shifts(orc.IterativeRecon(**kw), x, y, z, field=field, kind="disp")
+    scale = max(np.abs(e).max() for e in exp)
+    for g, e in zip(got, exp):
+        assert np.max(np.abs(g - e)) < 2e-5 * scale
+
+
 # ------------------------------------------------------------------ multigrid
 
 def mg_rec(los=None, L=1000.0):
