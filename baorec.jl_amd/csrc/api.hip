@@ -1879,23 +1879,21 @@ void check_cosmology(baorec_ctx *c, const baorec_cosmology *cp) {
 CosmoTable cosmo_table(baorec_ctx *c, const baorec_cosmology *cp) {
     check_cosmology(c, cp);
     const int num = cp->z_tab_num;
-    double *zk = bufT<double>(c, "cosmo_z", num);
-    double *rk = bufT<double>(c, "cosmo_r", num);
-    int *guide = bufT<int>(c, "cosmo_guide", num);
-    CosmoTable t{zk, rk, num, cp->z_tab_min, (double)(num - 1) / (cp->z_tab_max - cp->z_tab_min), guide, num,
-                 0.0, 0.0};
+    double2 *kn = bufT<double2>(c, "cosmo_zr", num);
+    float2 *guide = bufT<float2>(c, "cosmo_guide", kCosmoGuide);
+    CosmoTable t{kn, num, cp->z_tab_min, (double)(num - 1) / (cp->z_tab_max - cp->z_tab_min), guide, 0.0, 0.0};
     if (!c->cosmo_valid || memcmp(&c->cosmo, cp, sizeof(*cp)) != 0) {
         std::vector<double> h(num);
         cosmo_knots(cp, h.data());
-        hipchk(c, hipMemcpyAsync(zk, h.data(), sizeof(double) * num, hipMemcpyHostToDevice, c->stream), "H2D");
         double *seg = bufT<double>(c, "cosmo_seg", num);
-        hipchk(c, launch_cosmo_table(cosmo_args(cp), zk, seg, rk, num, c->stream), "cosmology table");
+        hipchk(c, hipMemcpyAsync(seg, h.data(), sizeof(double) * num, hipMemcpyHostToDevice, c->stream), "H2D");
+        hipchk(c, launch_cosmo_table(cosmo_args(cp), seg, kn, num, c->stream), "cosmology table");
         double ends[2];
-        hipchk(c, hipMemcpyAsync(&ends[0], rk, sizeof(double), hipMemcpyDeviceToHost, c->stream), "D2H");
-        hipchk(c, hipMemcpyAsync(&ends[1], rk + num - 1, sizeof(double), hipMemcpyDeviceToHost, c->stream), "D2H");
+        hipchk(c, hipMemcpyAsync(&ends[0], &kn[0].y, sizeof(double), hipMemcpyDeviceToHost, c->stream), "D2H");
+        hipchk(c, hipMemcpyAsync(&ends[1], &kn[num - 1].y, sizeof(double), hipMemcpyDeviceToHost, c->stream), "D2H");
         hipchk(c, hipStreamSynchronize(c->stream), "cosmology table");
         c->cosmo_r0 = ends[0];
-        c->cosmo_dr_inv = (double)num / (ends[1] - ends[0]);
+        c->cosmo_dr_inv = (double)kCosmoGuide / (ends[1] - ends[0]);
         t.r0 = c->cosmo_r0;
         t.dr_inv = c->cosmo_dr_inv;
         hipchk(c, launch_cosmo_guide(t, guide, c->stream), "cosmology guide");
@@ -1956,12 +1954,11 @@ double time_min(baorec_ctx *c, int reps, F &&fn) {
 // passes that address to the kernels.
 namespace {
 constexpr int kNoallocMaxKnots = 131072;
-// zk, rk, seg (FP64, kNoallocMaxKnots each), guide (int32), error flag (int32)
-constexpr size_t kNoallocZk = 0;
-constexpr size_t kNoallocRk = kNoallocZk + sizeof(double) * kNoallocMaxKnots;
-constexpr size_t kNoallocSeg = kNoallocRk + sizeof(double) * kNoallocMaxKnots;
+// knots (z, r) and seg (FP64, kNoallocMaxKnots each), guide, error flag (int32)
+constexpr size_t kNoallocKn = 0;
+constexpr size_t kNoallocSeg = kNoallocKn + sizeof(double2) * kNoallocMaxKnots;
 constexpr size_t kNoallocGuide = kNoallocSeg + sizeof(double) * kNoallocMaxKnots;
-constexpr size_t kNoallocErr = kNoallocGuide + sizeof(int) * kNoallocMaxKnots;
+constexpr size_t kNoallocErr = kNoallocGuide + sizeof(float2) * kCosmoGuide;
 constexpr size_t kNoallocBytes = kNoallocErr + 256;
 constexpr int kNoallocMaxDevices = 64;
 
@@ -2858,26 +2855,25 @@ int baorec_sky_to_cartesian_noalloc(baorec_ctx *c, const baorec_cosmology *cp, c
         std::lock_guard<std::mutex> lk(g_noalloc_lock);
         NoallocDevice &d = g_noalloc[c->device];
         if (!d.ptr) fail(c, BAOREC_ERR_HIP, "allocation-free scratch not set up on this device");
-        double *zk = reinterpret_cast<double *>(d.ptr + kNoallocZk);
-        double *rk = reinterpret_cast<double *>(d.ptr + kNoallocRk);
+        double2 *kn = reinterpret_cast<double2 *>(d.ptr + kNoallocKn);
         double *seg = reinterpret_cast<double *>(d.ptr + kNoallocSeg);
-        int *guide = reinterpret_cast<int *>(d.ptr + kNoallocGuide);
+        float2 *guide = reinterpret_cast<float2 *>(d.ptr + kNoallocGuide);
         int *err = reinterpret_cast<int *>(d.ptr + kNoallocErr);
         if (!d.table_valid || memcmp(&d.cosmo, cp, sizeof(*cp)) != 0) {
             d.table_valid = 0;
             cosmo_knots(cp, g_noalloc_knots);
-            hipchk(c, hipMemcpyAsync(zk, g_noalloc_knots, sizeof(double) * num, hipMemcpyHostToDevice, c->stream),
+            hipchk(c, hipMemcpyAsync(seg, g_noalloc_knots, sizeof(double) * num, hipMemcpyHostToDevice, c->stream),
                    "H2D knots");
-            hipchk(c, launch_cosmo_table(cosmo_args(cp), zk, seg, rk, num, c->stream), "cosmology table");
+            hipchk(c, launch_cosmo_table(cosmo_args(cp), seg, kn, num, c->stream), "cosmology table");
             double ends[2];
-            hipchk(c, hipMemcpyAsync(&ends[0], rk, sizeof(double), hipMemcpyDeviceToHost, c->stream), "D2H");
-            hipchk(c, hipMemcpyAsync(&ends[1], rk + num - 1, sizeof(double), hipMemcpyDeviceToHost, c->stream),
+            hipchk(c, hipMemcpyAsync(&ends[0], &kn[0].y, sizeof(double), hipMemcpyDeviceToHost, c->stream), "D2H");
+            hipchk(c, hipMemcpyAsync(&ends[1], &kn[num - 1].y, sizeof(double), hipMemcpyDeviceToHost, c->stream),
                    "D2H");
             sync(c);
             d.r0 = ends[0];
-            d.dr_inv = (double)num / (ends[1] - ends[0]);
-            CosmoTable g{zk, rk, num, cp->z_tab_min, (double)(num - 1) / (cp->z_tab_max - cp->z_tab_min),
-                         guide, num, d.r0, d.dr_inv};
+            d.dr_inv = (double)kCosmoGuide / (ends[1] - ends[0]);
+            CosmoTable g{kn, num, cp->z_tab_min, (double)(num - 1) / (cp->z_tab_max - cp->z_tab_min),
+                         guide, d.r0, d.dr_inv};
             hipchk(c, launch_cosmo_guide(g, guide, c->stream), "cosmology guide");
             d.cosmo = *cp;
             d.table_valid = 1;
@@ -2886,8 +2882,8 @@ int baorec_sky_to_cartesian_noalloc(baorec_ctx *c, const baorec_cosmology *cp, c
             sync(c);
             return;
         }
-        CosmoTable t{zk, rk, num, cp->z_tab_min, (double)(num - 1) / (cp->z_tab_max - cp->z_tab_min), guide,
-                     num, d.r0, d.dr_inv};
+        CosmoTable t{kn, num, cp->z_tab_min, (double)(num - 1) / (cp->z_tab_max - cp->z_tab_min), guide,
+                     d.r0, d.dr_inv};
         hipLaunchKernelGGL(k_zero_flag, dim3(1), dim3(64), 0, c->stream, err);
         hipchk(c, hipGetLastError(), "clear flag");
         const float hh = (cp->h * 100.0f) / 100.0f;   // cosmo.H0 / 100 in Float32, as the driver uses

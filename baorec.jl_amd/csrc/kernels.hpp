@@ -252,17 +252,17 @@ struct CosmoArgs {
 // Comoving-distance table: num knots zk (increasing, uniform) and distances
 // rk (Mpc, increasing).  Interval lookup: direct index on the uniform z knots;
 // for r, guide[j] = last knot with rk <= r0 + j / dr_inv (nguide entries).
+constexpr int kCosmoGuide = 1024;
 struct CosmoTable {
-    const double *zk, *rk;
+    const double2 *kn;   // knots (z, r)
     int num;
     double z0, dz_inv;
-    const int *guide;
-    int nguide;
+    const float2 *guide;   // kCosmoGuide entries: guess of the knot of r
     double r0, dr_inv;
 };
-hipError_t launch_cosmo_guide(const CosmoTable &t, int *guide, hipStream_t s);
-hipError_t launch_cosmo_table(const CosmoArgs &c, const double *zk, double *seg, double *rk, int num,
-                              hipStream_t s);
+hipError_t launch_cosmo_guide(const CosmoTable &t, float2 *guide, hipStream_t s);
+// kn from the knots' z, which seg (num entries, overwritten) holds at entry
+hipError_t launch_cosmo_table(const CosmoArgs &c, double *seg, double2 *kn, int num, hipStream_t s);
 hipError_t launch_comoving_distance(const CosmoTable &t, const double *z, double *r, int64_t n, int *err,
                                     hipStream_t s);
 hipError_t launch_sky_to_cart(const CosmoTable &t, float hh, const float *ra, const float *dec, const float *red,

@@ -809,6 +809,37 @@ def test_cartesian_to_sky_matches_oracle(ctx):
     assert np.all(got[0] <= 0) and np.all(got[0] > -360)
 
 
+@pytest.mark.parametrize("num", [2, 37, 100000])
+def test_sky_conversions_over_angles_and_tables(ctx, num):
+    """Both conversions where their trigonometry and table look-up change
+    branch: multiples of 45 degrees and their neighbours, zeros of either
+    sign, tiny and very large angles (both sides of the reduction's limit of
+    2^17 radians), every octant and axis, and tables of few and many knots;
+    each value within one FP32 ulp of the oracle as above (the angles of the
+    way back within one ulp of the largest).  The oracle interpolates the GPU's
+    own table: with few knots the quadratures of the two differ."""
+    c, o = bh.Cosmology(z_tab_num=num), orc.Cosmology(z_tab_num=num)
+    zk = orc.distance_table(o)[0]
+    table = zk, bh.comoving_distance(zk, c, ctx=ctx)
+    rng = np.random.default_rng(97)
+    base = np.arange(-16, 17).astype(F32) * F32(45.0)
+    ang = np.concatenate([base, np.nextafter(base, F32(1e9)), np.nextafter(base, F32(-1e9)),
+                          np.array([0.0, -0.0, 1e-30, -1e-30, 1e-5, 7509870.0, 7509872.0, -7509880.0, 1e9, -3e8], F32),
+                          rng.uniform(-2000.0, 2000.0, 4000).astype(F32)])
+    ra, dec = ang, rng.permutation(ang)
+    red = rng.uniform(table[0][0] + 1e-3, table[0][-1] - 1e-3, ang.size).astype(F32)
+    for g, r in zip(bh.sky_to_cartesian(ra, dec, red, c, ctx=ctx), orc.sky_to_cartesian(ra, dec, red, o, table)):
+        assert ulp_err(g, r) <= 1.0
+    axes = np.array([(i, j, k) for i in (-1, -0.0, 0.0, 1) for j in (-1, -0.0, 0.0, 1) for k in (-1, 0.0, 1)
+                     if i or j or k], F32)
+    pos = np.concatenate([axes * F32(700.0), rng.uniform(-900.0, 900.0, (4000, 3)).astype(F32),
+                          (axes + F32(1e-6) * rng.standard_normal(axes.shape).astype(F32)) * F32(500.0)])
+    x, y, z = (np.ascontiguousarray(pos[:, a]) for a in range(3))
+    got, ref = bh.cartesian_to_sky(x, y, z, c, ctx=ctx), orc.cartesian_to_sky(x, y, z, o, table)
+    for g, r in zip(got, ref):
+        assert np.max(np.abs(g.astype(np.float64) - r)) <= np.max(np.spacing(np.abs(r))) + 1e-12
+
+
 def test_sky_outside_table_raises(ctx):
     c = bh.Cosmology(z_tab_num=1001)
     with pytest.raises(bh.BoundsError):
