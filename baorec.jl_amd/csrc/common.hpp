@@ -54,6 +54,11 @@ struct Slot {
 // Twiddles come from one table: tw[S + i] = exp(-2 pi i * i / S) for every
 // power of two S <= 2048 (4096 float2 in total).
 
+// Workgroup barrier for exchanges through LDS alone: __syncthreads without its
+// fence on memory, which would wait for copies into LDS that are still in
+// flight (k_y_iter's).
+__device__ __forceinline__ void lds_barrier() { asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory"); }
+
 template <int M, bool INV>
 struct Plan {
     static constexpr int LOG = (M == 8) ? 3 : (M == 16) ? 4 : (M == 32) ? 5 : (M == 64) ? 6
@@ -132,7 +137,7 @@ __device__ __forceinline__ void fft_stages(float2 (&v)[8], float2 *lds, const La
         constexpr int RP = P::radix(ST - 1);
         constexpr int NSP = P::ns(ST - 1);
         constexpr int NBP = 8 / RP;
-        __syncthreads();
+        lds_barrier();
 #pragma unroll
         for (int s = 0; s < NBP; s++) {
             int j = t + s * (M / 8);
@@ -141,7 +146,7 @@ __device__ __forceinline__ void fft_stages(float2 (&v)[8], float2 *lds, const La
 #pragma unroll
             for (int q = 0; q < RP; q++) lds[lay(base + q * NSP)] = v[s * RP + q];
         }
-        __syncthreads();
+        lds_barrier();
 #pragma unroll
         for (int s = 0; s < NB; s++) {
             int j = t + s * (M / 8);
@@ -212,7 +217,7 @@ __device__ __forceinline__ void fft_stages_c(float2 (&v)[8], float2 *lds, const 
         constexpr int RP = P::radix(ST - 1);
         constexpr int NSP = P::ns(ST - 1);
         constexpr int NBP = 8 / RP;
-        __syncthreads();
+        lds_barrier();
 #pragma unroll
         for (int s = 0; s < NBP; s++) {
             int j = t + s * (M / 8);
@@ -221,7 +226,7 @@ __device__ __forceinline__ void fft_stages_c(float2 (&v)[8], float2 *lds, const 
 #pragma unroll
             for (int q = 0; q < RP; q++) lds[lay(base + q * NSP)] = v[s * RP + q];
         }
-        __syncthreads();
+        lds_barrier();
 #pragma unroll
         for (int s = 0; s < NB; s++) {
             int j = t + s * (M / 8);
@@ -265,7 +270,7 @@ __device__ __forceinline__ void fft_stages2(float2 (&v)[2][8], float4 *lds, cons
         constexpr int RP = P::radix(ST - 1);
         constexpr int NSP = P::ns(ST - 1);
         constexpr int NBP = 8 / RP;
-        __syncthreads();
+        lds_barrier();
 #pragma unroll
         for (int s = 0; s < NBP; s++) {
             int j = t + s * (M / 8);
@@ -277,7 +282,7 @@ __device__ __forceinline__ void fft_stages2(float2 (&v)[2][8], float4 *lds, cons
                 lds[lay(base + q * NSP)] = make_float4(a.x, a.y, b.x, b.y);
             }
         }
-        __syncthreads();
+        lds_barrier();
 #pragma unroll
         for (int s = 0; s < NB; s++) {
             int j = t + s * (M / 8);

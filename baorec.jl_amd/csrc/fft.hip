@@ -704,20 +704,23 @@ k_strided2(StridedArgs a) {
 
 // ------------------------------------------------------------ y: local-LOS iteration
 
-// The pointer as an opaque value: table loads through it are not hoisted
-// across the transforms that use it (which would keep them all live).
-template <class T>
-__device__ __forceinline__ T *opaque(T *p) {
-    asm volatile("" : "+s"(p));
-    return p;
-}
-
+// Bound by its traffic (three spectra read, three written: 3.2 GB per 512^3) and
+// by 2000 vector instructions per thread, at two workgroups per CU whose
+// phases overlap little; so no load waits behind a store (they return in
+// order) or for memory: an input goes straight into LDS (the wave's own
+// share of it, so no barrier) during the transform before its first use, and
+// its second and third use read it there.  Registers have no room for that: two
+// accumulators, a line and the twiddles fill the 128 that let two
+// workgroups share a CU.
 template <int M>
 __global__ void __launch_bounds__(SShape<M>::NT) __attribute__((amdgpu_waves_per_eu(4)))
 k_y_iter(YIterArgs a) {
-    constexpr int B = SShape<M>::B;
+    constexpr int B = SShape<M>::B, NT = SShape<M>::NT;
+    constexpr bool STASH = NT >= 64;   // whole waves
     using PI = Plan<M, true>;
     __shared__ float2 lds[lay_strided_size(M, B)];
+    __shared__ __align__(16) float2 stash[STASH ? 8 * NT : 1];
+    __shared__ float kyl[M], yl[M];
     const int tid = threadIdx.x;
     const int col = tid % B, t = tid / B;
     const int ncg = (a.Pv + B - 1) / B;
@@ -726,77 +729,124 @@ k_y_iter(YIterArgs a) {
     const int kxi = cg * B + col;
     const bool valid = kxi < a.Pv;
     const int64_t b = blockIdx.z;
-    const int64_t base = b * a.cstride + (int64_t)iz * a.PZ + kxi;
-    const int64_t rs = a.P;
+    const int64_t tile0 = b * a.cstride + (int64_t)iz * a.PZ + cg * B;   // the tile's first column, y = 0
+    // byte offset of row r, column c of the tile (a plane is below 2^31 bytes)
+    const int rs = (int)a.P;
+    auto at = [&](auto *p, int r, int c) {
+        using T = std::remove_pointer_t<decltype(p)>;
+        using Byte = std::conditional_t<std::is_const_v<T>, const char, char>;
+        return reinterpret_cast<T *>(reinterpret_cast<Byte *>(p + tile0) + (uint32_t)((r * rs + c) * 8));
+    };
+    // keeps a value where it is computed: moved to its use, the coordinates
+    // it is made of spill
+    auto pin = [](float2 &x) { asm volatile("" : "+v"(x.x), "+v"(x.y)); };
     const float *ky = a.ktab + b * a.ktabStride + a.Pv;
     const float *xv = a.xtab + b * a.xtabStride;
+    // Input g into the stash: register index i of the wave's 64 threads is 512
+    // bytes in lane order, and an instruction moves two of them, 16 bytes
+    // (two columns, which may lie past Pv inside the row pitch) per lane.
+    const int lane = tid & 63;
+    float2 *mine = stash + (STASH ? __builtin_amdgcn_readfirstlane(tid >> 6) * 512 : 0);
+    const int tp = (tid >> 6) * (64 / B) + (lane & 31) / (B / 2);   // row thread of the lane's pair
+    const int pc = 2 * ((lane & 31) % (B / 2));
+    auto fetch = [&](const float2 *g) {
+        if constexpr (STASH) {
+#pragma unroll
+            for (int j = 0; j < 4; j++) {
+                const int r = lane < 32 ? PI::in_pos(tp, 2 * j) : PI::in_pos(tp, 2 * j + 1);
+                __builtin_amdgcn_global_load_lds(
+                    (const __attribute__((address_space(1))) void *)at(g, r, pc),
+                    (__attribute__((address_space(3))) void *)(mine + j * 128), 16, 0, 0);
+            }
+        }
+    };
+    // the fetched input is there / its values have been read
+    auto arrived = [&] { asm volatile("s_waitcnt vmcnt(0)" ::: "memory"); };
+    auto released = [&] { asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory"); };
+    // v = G ky^p in the inverse plan's input order
+    auto get = [&](const float2 *g, int p, float2 (&v)[8]) {
+#pragma unroll
+        for (int i = 0; i < 8; i++) {
+            const int r = PI::in_pos(t, i);
+            float2 x;
+            if constexpr (STASH)
+                x = mine[i * 64 + lane];
+            else
+                x = valid ? *at(g, r, col) : make_float2(0.f, 0.f);
+            const float k = kyl[r];
+            v[i] = p == 0 ? x : cscale(x, p == 1 ? k : k * k);
+        }
+    };
+    fetch(a.g[0]);
+    for (int i = tid; i < M; i += NT) {
+        kyl[i] = ky[i];
+        yl[i] = xv[a.nx + i];
+    }
     const float zc = xv[a.nx + a.ny + iz];
     LayStrided lay{col, B};
     TwCache<M, true> tc;
     tc.load(t, g_tw);
     const float fxx = a.fac[0], fxy = a.fac[1], fxz = a.fac[2];
     const float fyy = a.fac[3], fyz = a.fac[4], fzz = a.fac[5];
-    // in: v = G[i] * ky^p (in the inverse plan's input order)
-    auto load = [&](const float2 *g0, int p, float2 (&v)[8]) {
-        // opaque: each transform loads its own input (no reuse across
-        // transforms that would keep a whole line live)
-        const float2 *g = opaque(g0);
-        const float *kyo = opaque(ky);
-#pragma unroll
-        for (int i = 0; i < 8; i++) {
-            const int r = PI::in_pos(t, i);
-            const float2 x = valid ? g[base + r * rs] : make_float2(0.f, 0.f);
-            const float k = kyo[r];
-            v[i] = p == 0 ? x : cscale(x, p == 1 ? k : k * k);
-        }
-    };
+    __syncthreads();
+    arrived();
     // The six transforms in an order that keeps at most two accumulators and
-    // one line live: G0 terms of A, B and C; then G1 (read twice: for B and
-    // for C); then G2.
+    // one line live: G0 terms of A, B and C; then G1 (for B and for C); then G2.
     float2 v[8], accb[8], accc[8];
     // A = fxx IFFT(G0)
-    load(a.g[0], 0, v);
+    get(a.g[0], 0, v);
     fft_line_c<M, true>(v, lds, lay, t, tc);
     if (valid) {
 #pragma unroll
-        for (int i = 0; i < 8; i++) a.out[0][base + PI::out_pos(t, i) * rs] = cscale(v[i], fxx);
+        for (int i = 0; i < 8; i++) *at(a.out[0], PI::out_pos(t, i), col) = cscale(v[i], fxx);
     }
     // B = fxy y IFFT(ky G0) + ...
-    load(a.g[0], 1, v);
-    fft_line_c<M, true>(v, lds, lay, t, tc);
-#pragma unroll
-    for (int i = 0; i < 8; i++) accb[i] = cscale(v[i], fxy * opaque(xv)[a.nx + PI::out_pos(t, i)]);
-    // C = fyy y^2 IFFT(ky^2 G0) + ...
-    load(a.g[0], 2, v);
+    get(a.g[0], 1, v);
     fft_line_c<M, true>(v, lds, lay, t, tc);
 #pragma unroll
     for (int i = 0; i < 8; i++) {
-        const float yc = opaque(xv)[a.nx + PI::out_pos(t, i)];
+        accb[i] = cscale(v[i], fxy * yl[PI::out_pos(t, i)]);
+        pin(accb[i]);
+    }
+    // C = fyy y^2 IFFT(ky^2 G0) + ...
+    get(a.g[0], 2, v);
+    released();
+    fetch(a.g[1]);
+    fft_line_c<M, true>(v, lds, lay, t, tc);
+#pragma unroll
+    for (int i = 0; i < 8; i++) {
+        const float yc = yl[PI::out_pos(t, i)];
         accc[i] = cscale(v[i], fyy * (yc * yc));
+        pin(accc[i]);
     }
     // B += fxz z IFFT(G1)
-    load(a.g[1], 0, v);
+    arrived();
+    get(a.g[1], 0, v);
     fft_line_c<M, true>(v, lds, lay, t, tc);
     if (valid) {
 #pragma unroll
         for (int i = 0; i < 8; i++)
-            a.out[1][base + PI::out_pos(t, i) * rs] = cadd(accb[i], cscale(v[i], fxz * zc));
+            *at(a.out[1], PI::out_pos(t, i), col) = cadd(accb[i], cscale(v[i], fxz * zc));
     }
     // C += fyz y z IFFT(ky G1)
-    load(a.g[1], 1, v);
+    get(a.g[1], 1, v);
+    released();
+    fetch(a.g[2]);
     fft_line_c<M, true>(v, lds, lay, t, tc);
 #pragma unroll
     for (int i = 0; i < 8; i++) {
-        const float yc = opaque(xv)[a.nx + PI::out_pos(t, i)];
+        const float yc = yl[PI::out_pos(t, i)];
         accc[i] = cadd(accc[i], cscale(v[i], fyz * (yc * zc)));
+        pin(accc[i]);
     }
     // C += fzz z^2 IFFT(G2)
-    load(a.g[2], 0, v);
+    arrived();
+    get(a.g[2], 0, v);
     fft_line_c<M, true>(v, lds, lay, t, tc);
     if (valid) {
 #pragma unroll
         for (int i = 0; i < 8; i++)
-            a.out[2][base + PI::out_pos(t, i) * rs] = cadd(accc[i], cscale(v[i], fzz * (zc * zc)));
+            *at(a.out[2], PI::out_pos(t, i), col) = cadd(accc[i], cscale(v[i], fzz * (zc * zc)));
     }
 }
 
