@@ -10,6 +10,9 @@
 // broadcasts are folded into these passes instead of running as extra sweeps.
 #include <math.h>
 
+#include <algorithm>
+#include <type_traits>
+
 #include "kernels.hpp"
 
 namespace baorec {
@@ -493,15 +496,22 @@ __device__ __forceinline__ float2 apply_mul(float2 F, float kx, float ky, float 
             const double g = exp(-0.5 * (double)R2 * (double)k2);
             return make_float2((float)((double)F.x * g), (float)((double)F.y * g));
         }
-        case MUL_INVK2:
-            return k2 > 0.f ? make_float2(F.x / k2, F.y / k2) : make_float2(0.f, 0.f);
+        case MUL_INVK2: {
+            const float d = k2 > 0.f ? k2 : 1.f, y = refined_rcp(d);
+            F = make_float2(div_by(F.x, d, y), div_by(F.y, d, y));
+            return k2 > 0.f ? F : make_float2(0.f, 0.f);
+        }
         case MUL_FIXEDLOS: {
             if (!(k2 > 0.f)) return make_float2(0.f, 0.f);
             const float m = ((kx * kx) * l0 + (ky * ky) * l1) + (kz * kz) * l2;
-            return cscale(make_float2(F.x / k2, F.y / k2), m);
+            const float y = refined_rcp(k2);
+            return cscale(make_float2(div_by(F.x, k2, y), div_by(F.y, k2, y)), m);
         }
-        case MUL_I_INVK2:
-            return k2 > 0.f ? make_float2(-F.y / k2, F.x / k2) : make_float2(0.f, 0.f);
+        case MUL_I_INVK2: {
+            const float d = k2 > 0.f ? k2 : 1.f, y = refined_rcp(d);
+            F = make_float2(div_by(-F.y, d, y), div_by(F.x, d, y));
+            return k2 > 0.f ? F : make_float2(0.f, 0.f);
+        }
         case MUL_I:
             return make_float2(-F.y, F.x);
         case MUL_GAUSS1: {
@@ -702,161 +712,311 @@ k_strided2(StridedArgs a) {
     }
 }
 
+constexpr int kStridedNPv = 513;   // kx columns k_strided_n holds
+
+// The same pass for jobs of two or three outputs at M = 256 and 512 (the
+// local-LOS iteration's and the displacement's z and y passes), with 16
+// columns (whole 128-byte lines of memory per row; with 8, what bounded the
+// pass at 512 was the half lines: 713 us) and by workgroups that stay, 16 waves
+// per CU, each walking over tiles.  The next tile's lines load into registers
+// while the current one is transformed, the twiddles of the forward transform
+// and the k tables stand in LDS for all tiles, and no load waits behind a store
+// (they complete in order).  Columns past Pv (inside the row pitch) are
+// transformed and stored like the others; nothing reads them.  NOUT: the most
+// outputs of a job.  The iteration's z pass (2.15 GB at 512^3): 585 us, 716
+// by k_strided; 65 and 82 at 256^3.
+template <int M, int MODE, int MK, int NOUT>
+__global__ void __launch_bounds__(2 * M) __attribute__((amdgpu_waves_per_eu(4)))
+k_strided_n(StridedArgs a) {
+    constexpr int B = 16, NT = 2 * M;
+    using PF = Plan<M, false>;
+    using PI = Plan<M, true>;
+    using PL = Plan<M, MODE != 2>;   // the plan of the first transform
+    __shared__ float2 lds[lay_strided_size(M, B)];
+    __shared__ float2 twl[MODE == 2 ? 2 * M : 1];
+    __shared__ float kal[M], kxl[kStridedNPv];
+    const int tid = threadIdx.x;
+    const int col = tid % B;
+    int t = tid / B;
+    const StridedJob &J = a.job[blockIdx.y];
+    const int64_t b = blockIdx.z;
+    const float *kt = a.ktab + b * a.ktabStride;
+    const float *kax = a.axis == 1 ? kt + a.kyo : kt + a.kyo + a.ny;
+    const float *kot = a.axis == 1 ? kt + a.kyo + a.ny : kt + a.kyo;
+    const int ncg = (a.Pv + B - 1) / B, nother = a.axis == 1 ? a.nz : a.ny;
+    const int rs = a.axis == 1 ? a.P : (int)a.PZ;
+    const int64_t os = a.axis == 1 ? a.PZ : a.P;
+    // this XCD's tiles: t0 .. t0 + cnt, its workgroups side by side on them
+    const int nt = ncg * nother, xc = blockIdx.x & 7;
+    const int t0 = xc * (nt >> 3) + min(xc, nt & 7), cnt = (nt >> 3) + (xc < (nt & 7) ? 1 : 0);
+    const int step = gridDim.x >> 3;
+    // byte offset of row r of the thread's column from a tile's first column (below 2^32)
+    auto at = [&](auto *p, int r) {
+        using T = std::remove_pointer_t<decltype(p)>;
+        using Byte = std::conditional_t<std::is_const_v<T>, const char, char>;
+        return reinterpret_cast<T *>(reinterpret_cast<Byte *>(p) + ((uint32_t)r * (uint32_t)rs + (uint32_t)col) * 8u);
+    };
+    auto tile0 = [&](int u) { return b * a.cstride + (int64_t)((t0 + u) / ncg) * os + (t0 + u) % ncg * B; };
+    float2 nxt[8];
+    auto fetch = [&](int u) {
+        const float2 *src = J.in + tile0(u);
+#pragma unroll
+        for (int i = 0; i < 8; i++) nxt[i] = *at(src, PL::in_pos(t, i));
+    };
+    int u = blockIdx.x >> 3;
+    if (u >= cnt) return;
+    fetch(u);
+    if constexpr (MODE == 2)
+        for (int i = tid; i < 2 * M; i += NT) twl[i] = g_tw[i];
+    for (int i = tid; i < M; i += NT) kal[i] = kax[i];
+    for (int i = tid; i < a.Pv; i += NT) kxl[i] = kt[i];
+    TwCache<M, true> tc;
+    tc.load(t, g_tw);
+    const LayStrided lay{col, B};
+    __syncthreads();
+    // vmcnt(0), once: the twiddles' loads would otherwise be waited for, with
+    // the next tile's behind them, in every round of the loop
+    __builtin_amdgcn_s_waitcnt(0x0f70);
+    for (;;) {
+        asm volatile("" : "+v"(t));   // no address of a tile is kept in registers for the next
+        float2 f[8], v[8];
+#pragma unroll
+        for (int i = 0; i < 8; i++) f[i] = nxt[i];
+        const int next = u + step;
+        if (next < cnt) fetch(next);
+        if constexpr (MODE == 2) {
+            fft_line<M, false>(f, lds, lay, t, twl);
+            const int other = (t0 + u) / ncg, kxi = (t0 + u) % ncg * B + col;
+            const float kxv = kxi < a.Pv ? kxl[kxi] : 0.f;
+            // a scalar load: one in line with the vector ones would wait for the next tile's
+            const float ko = *(const __attribute__((address_space(4))) float *)(uintptr_t)(kot + other);
+#pragma unroll
+            for (int i = 0; i < 8; i++) {
+                const float k = kal[PF::out_pos(t, i)];
+                f[i] = apply_mul<MK>(f[i], kxv, a.axis == 1 ? k : ko, a.axis == 1 ? ko : k, a);
+            }
+        }
+        const int64_t o0 = tile0(u);
+#pragma unroll
+        for (int o = 0; o < NOUT; o++) {
+            if (o > 0 && o >= J.nout) break;
+            const int pw = J.pw[o];
+            if (pw == 0) {
+#pragma unroll
+                for (int i = 0; i < 8; i++) v[i] = f[i];
+            } else {
+#pragma unroll
+                for (int i = 0; i < 8; i++) {
+                    const float k = kal[PI::in_pos(t, i)];
+                    v[i] = cscale(f[i], pw == 1 ? k : k * k);
+                }
+            }
+            fft_line_c<M, true>(v, lds, lay, t, tc);
+            float2 *dst = J.out[o] + o0;
+#pragma unroll
+            for (int i = 0; i < 8; i++) *at(dst, PI::out_pos(t, i)) = v[i];
+        }
+        if (next >= cnt) break;
+        u = next;
+    }
+}
+
 // ------------------------------------------------------------ y: local-LOS iteration
 
-// Bound by its traffic (three spectra read, three written: 3.2 GB per 512^3) and
-// by 2000 vector instructions per thread, at two workgroups per CU whose
-// phases overlap little; so no load waits behind a store (they return in
-// order) or for memory: an input goes straight into LDS (the wave's own
-// share of it, so no barrier) during the transform before its first use, and
-// its second and third use read it there.  Registers have no room for that: two
-// accumulators, a line and the twiddles fill the 128 that let two
-// workgroups share a CU.
+// Columns and threads per workgroup: whole 128-byte lines of memory per row.
 template <int M>
-__global__ void __launch_bounds__(SShape<M>::NT) __attribute__((amdgpu_waves_per_eu(4)))
+struct YShape {
+    static constexpr int B = M >= 1024 ? 8 : 16;
+    static constexpr int NT = B * M / 8;
+    static constexpr int PER_CU = NT >= 1024 ? 1 : 1024 / NT;   // four waves per SIMD
+};
+
+// Bound by its traffic (three spectra read, three written: 3.2 GB per 512^3)
+// and by 1800 vector instructions per thread.  Workgroups stay and walk over
+// tiles; no load waits behind a store (they complete in order) or for
+// memory: an input goes straight into LDS (the wave's own share of it, so no
+// barrier) during the transform before its first use, and its second and
+// third use read it there.  Registers have no room for that: two accumulators, a
+// line and the twiddles fill the 128 of four waves per SIMD.  Columns past Pv
+// (inside the row pitch) are transformed and stored like the others; nothing
+// reads them.  512^3: 748 us (1016 with 8 columns per workgroup of one tile
+// that read each input before each transform, 832 with the inputs through
+// LDS), 256^3: 98 (132).
+template <int M>
+__global__ void __launch_bounds__(YShape<M>::NT) __attribute__((amdgpu_waves_per_eu(4)))
 k_y_iter(YIterArgs a) {
-    constexpr int B = SShape<M>::B, NT = SShape<M>::NT;
+    constexpr int B = YShape<M>::B, NT = YShape<M>::NT;
     constexpr bool STASH = NT >= 64;   // whole waves
     using PI = Plan<M, true>;
     __shared__ float2 lds[lay_strided_size(M, B)];
     __shared__ __align__(16) float2 stash[STASH ? 8 * NT : 1];
     __shared__ float kyl[M], yl[M];
-    const int tid = threadIdx.x;
-    const int col = tid % B, t = tid / B;
+    const int tid = threadIdx.x, lane = tid & 63;
+    const int col = tid % B;
+    int t = tid / B;
     const int ncg = (a.Pv + B - 1) / B;
-    const int tile = xcd_tile(blockIdx.x, gridDim.x);
-    const int cg = tile % ncg, iz = tile / ncg;
-    const int kxi = cg * B + col;
-    const bool valid = kxi < a.Pv;
     const int64_t b = blockIdx.z;
-    const int64_t tile0 = b * a.cstride + (int64_t)iz * a.PZ + cg * B;   // the tile's first column, y = 0
-    // byte offset of row r, column c of the tile (a plane is below 2^31 bytes)
+    const float *ky = a.ktab + b * a.ktabStride + a.Pv;
+    const float *xv = a.xtab + b * a.xtabStride;
+    // this XCD's tiles: t0 .. t0 + cnt, its workgroups side by side on them
+    const int nt = ncg * a.nz, xc = blockIdx.x & 7;
+    const int t0 = xc * (nt >> 3) + min(xc, nt & 7), cnt = (nt >> 3) + (xc < (nt & 7) ? 1 : 0);
+    const int step = gridDim.x >> 3;
+    int u = blockIdx.x >> 3;
+    if (u >= cnt) return;
+    // a tile's first column at y = 0
+    auto tile0 = [&](int u) { return b * a.cstride + (int64_t)((t0 + u) / ncg) * a.PZ + (t0 + u) % ncg * B; };
+    // byte offset of row r, column c of a tile (a plane is below 2^31 bytes)
     const int rs = (int)a.P;
     auto at = [&](auto *p, int r, int c) {
         using T = std::remove_pointer_t<decltype(p)>;
         using Byte = std::conditional_t<std::is_const_v<T>, const char, char>;
-        return reinterpret_cast<T *>(reinterpret_cast<Byte *>(p + tile0) + (uint32_t)((r * rs + c) * 8));
+        return reinterpret_cast<T *>(reinterpret_cast<Byte *>(p) + (uint32_t)((r * rs + c) * 8));
     };
     // keeps a value where it is computed: moved to its use, the coordinates
     // it is made of spill
     auto pin = [](float2 &x) { asm volatile("" : "+v"(x.x), "+v"(x.y)); };
-    const float *ky = a.ktab + b * a.ktabStride + a.Pv;
-    const float *xv = a.xtab + b * a.xtabStride;
-    // Input g into the stash: register index i of the wave's 64 threads is 512
-    // bytes in lane order, and an instruction moves two of them, 16 bytes
-    // (two columns, which may lie past Pv inside the row pitch) per lane.
-    const int lane = tid & 63;
+    // Input g of a tile into the stash: register index i of the wave's 64
+    // threads is 512 bytes in lane order, and an instruction moves two of
+    // them, 16 bytes (two columns) per lane.
     float2 *mine = stash + (STASH ? __builtin_amdgcn_readfirstlane(tid >> 6) * 512 : 0);
-    const int tp = (tid >> 6) * (64 / B) + (lane & 31) / (B / 2);   // row thread of the lane's pair
+    int tp = (tid >> 6) * (64 / B) + (lane & 31) / (B / 2);   // row thread of the lane's pair
     const int pc = 2 * ((lane & 31) % (B / 2));
     auto fetch = [&](const float2 *g) {
         if constexpr (STASH) {
 #pragma unroll
             for (int j = 0; j < 4; j++) {
                 const int r = lane < 32 ? PI::in_pos(tp, 2 * j) : PI::in_pos(tp, 2 * j + 1);
-                __builtin_amdgcn_global_load_lds(
-                    (const __attribute__((address_space(1))) void *)at(g, r, pc),
-                    (__attribute__((address_space(3))) void *)(mine + j * 128), 16, 0, 0);
+                __builtin_amdgcn_global_load_lds((const __attribute__((address_space(1))) void *)at(g, r, pc),
+                                                 (__attribute__((address_space(3))) void *)(mine + j * 128), 16, 0, 0);
             }
         }
     };
-    // the fetched input is there / its values have been read
+    // The fetched input is there.
     auto arrived = [&] { asm volatile("s_waitcnt vmcnt(0)" ::: "memory"); };
-    auto released = [&] { asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory"); };
-    // v = G ky^p in the inverse plan's input order
+    // v = G ky^p in the inverse plan's input order.  The stash is read in one
+    // asm block with its wait: the compiler would wait for every store in
+    // flight before a read of memory that a copy into LDS wrote.
     auto get = [&](const float2 *g, int p, float2 (&v)[8]) {
+        typedef float f32x4 __attribute__((ext_vector_type(4)));
+        f32x4 q[4];
+        if constexpr (STASH) {
+            const uint32_t from =
+                (uint32_t)(uintptr_t)(__attribute__((address_space(3))) void *)(mine + lane);
+            asm volatile("ds_read2st64_b64 %0, %4 offset1:1\n\t"
+                         "ds_read2st64_b64 %1, %4 offset0:2 offset1:3\n\t"
+                         "ds_read2st64_b64 %2, %4 offset0:4 offset1:5\n\t"
+                         "ds_read2st64_b64 %3, %4 offset0:6 offset1:7\n\t"
+                         "s_waitcnt lgkmcnt(0)"
+                         : "=&v"(q[0]), "=&v"(q[1]), "=&v"(q[2]), "=&v"(q[3])
+                         : "v"(from)
+                         : "memory");
+        }
 #pragma unroll
         for (int i = 0; i < 8; i++) {
             const int r = PI::in_pos(t, i);
             float2 x;
             if constexpr (STASH)
-                x = mine[i * 64 + lane];
+                x = i & 1 ? make_float2(q[i >> 1].z, q[i >> 1].w) : make_float2(q[i >> 1].x, q[i >> 1].y);
             else
-                x = valid ? *at(g, r, col) : make_float2(0.f, 0.f);
+                x = *at(g, r, col);
             const float k = kyl[r];
             v[i] = p == 0 ? x : cscale(x, p == 1 ? k : k * k);
         }
     };
-    fetch(a.g[0]);
+    // addresses are not kept in registers beyond this point
+    auto forget = [&] { asm volatile("" : "+v"(t), "+v"(tp)); };
+    fetch(a.g[0] + tile0(u));
     for (int i = tid; i < M; i += NT) {
         kyl[i] = ky[i];
         yl[i] = xv[a.nx + i];
     }
-    const float zc = xv[a.nx + a.ny + iz];
     LayStrided lay{col, B};
     TwCache<M, true> tc;
     tc.load(t, g_tw);
     const float fxx = a.fac[0], fxy = a.fac[1], fxz = a.fac[2];
     const float fyy = a.fac[3], fyz = a.fac[4], fzz = a.fac[5];
     __syncthreads();
-    arrived();
-    // The six transforms in an order that keeps at most two accumulators and
-    // one line live: G0 terms of A, B and C; then G1 (for B and for C); then G2.
-    float2 v[8], accb[8], accc[8];
-    // A = fxx IFFT(G0)
-    get(a.g[0], 0, v);
-    fft_line_c<M, true>(v, lds, lay, t, tc);
-    if (valid) {
+    __builtin_amdgcn_s_waitcnt(0x0f70);   // vmcnt(0): the twiddles, and the first input
+    for (;;) {
+        const int64_t o0 = tile0(u);
+        const int next = u + step;
+        // a scalar load: one in line with the vector ones would wait for them
+        const float zc = *(const __attribute__((address_space(4))) float *)(uintptr_t)(xv + a.nx + a.ny + (t0 + u) / ncg);
+        // The six transforms in an order that keeps at most two accumulators and
+        // one line live: G0 terms of A, B and C; then G1 (for B and for C); then G2.
+        float2 v[8], accb[8], accc[8];
+        // A = fxx IFFT(G0)
+        forget();
+        get(a.g[0] + o0, 0, v);
+        fft_line_c<M, true>(v, lds, lay, t, tc);
 #pragma unroll
-        for (int i = 0; i < 8; i++) *at(a.out[0], PI::out_pos(t, i), col) = cscale(v[i], fxx);
-    }
-    // B = fxy y IFFT(ky G0) + ...
-    get(a.g[0], 1, v);
-    fft_line_c<M, true>(v, lds, lay, t, tc);
+        for (int i = 0; i < 8; i++) *at(a.out[0] + o0, PI::out_pos(t, i), col) = cscale(v[i], fxx);
+        // B = fxy y IFFT(ky G0) + ...
+        get(a.g[0] + o0, 1, v);
+        fft_line_c<M, true>(v, lds, lay, t, tc);
 #pragma unroll
-    for (int i = 0; i < 8; i++) {
-        accb[i] = cscale(v[i], fxy * yl[PI::out_pos(t, i)]);
-        pin(accb[i]);
-    }
-    // C = fyy y^2 IFFT(ky^2 G0) + ...
-    get(a.g[0], 2, v);
-    released();
-    fetch(a.g[1]);
-    fft_line_c<M, true>(v, lds, lay, t, tc);
+        for (int i = 0; i < 8; i++) {
+            accb[i] = cscale(v[i], fxy * yl[PI::out_pos(t, i)]);
+            pin(accb[i]);
+        }
+        // C = fyy y^2 IFFT(ky^2 G0) + ...
+        get(a.g[0] + o0, 2, v);
+        fetch(a.g[1] + o0);
+        fft_line_c<M, true>(v, lds, lay, t, tc);
 #pragma unroll
-    for (int i = 0; i < 8; i++) {
-        const float yc = yl[PI::out_pos(t, i)];
-        accc[i] = cscale(v[i], fyy * (yc * yc));
-        pin(accc[i]);
-    }
-    // B += fxz z IFFT(G1)
-    arrived();
-    get(a.g[1], 0, v);
-    fft_line_c<M, true>(v, lds, lay, t, tc);
-    if (valid) {
-#pragma unroll
-        for (int i = 0; i < 8; i++)
-            *at(a.out[1], PI::out_pos(t, i), col) = cadd(accb[i], cscale(v[i], fxz * zc));
-    }
-    // C += fyz y z IFFT(ky G1)
-    get(a.g[1], 1, v);
-    released();
-    fetch(a.g[2]);
-    fft_line_c<M, true>(v, lds, lay, t, tc);
-#pragma unroll
-    for (int i = 0; i < 8; i++) {
-        const float yc = yl[PI::out_pos(t, i)];
-        accc[i] = cadd(accc[i], cscale(v[i], fyz * (yc * zc)));
-        pin(accc[i]);
-    }
-    // C += fzz z^2 IFFT(G2)
-    arrived();
-    get(a.g[2], 0, v);
-    fft_line_c<M, true>(v, lds, lay, t, tc);
-    if (valid) {
+        for (int i = 0; i < 8; i++) {
+            const float yc = yl[PI::out_pos(t, i)];
+            accc[i] = cscale(v[i], fyy * (yc * yc));
+            pin(accc[i]);
+        }
+        // B += fxz z IFFT(G1)
+        forget();
+        arrived();
+        get(a.g[1] + o0, 0, v);
+        fft_line_c<M, true>(v, lds, lay, t, tc);
 #pragma unroll
         for (int i = 0; i < 8; i++)
-            *at(a.out[2], PI::out_pos(t, i), col) = cadd(accc[i], cscale(v[i], fzz * (zc * zc)));
+            *at(a.out[1] + o0, PI::out_pos(t, i), col) = cadd(accb[i], cscale(v[i], fxz * zc));
+        // C += fyz y z IFFT(ky G1)
+        get(a.g[1] + o0, 1, v);
+        fetch(a.g[2] + o0);
+        fft_line_c<M, true>(v, lds, lay, t, tc);
+#pragma unroll
+        for (int i = 0; i < 8; i++) {
+            const float yc = yl[PI::out_pos(t, i)];
+            accc[i] = cadd(accc[i], cscale(v[i], fyz * (yc * zc)));
+            pin(accc[i]);
+        }
+        // C += fzz z^2 IFFT(G2), the next tile's G0 on its way
+        forget();
+        arrived();
+        get(a.g[2] + o0, 0, v);
+        if (next < cnt) fetch(a.g[0] + tile0(next));
+        fft_line_c<M, true>(v, lds, lay, t, tc);
+#pragma unroll
+        for (int i = 0; i < 8; i++)
+            *at(a.out[2] + o0, PI::out_pos(t, i), col) = cadd(accc[i], cscale(v[i], fzz * (zc * zc)));
+        if (next >= cnt) break;
+        u = next;
+        asm volatile("s_waitcnt vmcnt(8)" ::: "memory");   // all but the eight stores since the copy
     }
 }
 
 // ------------------------------------------------------------ launchers
 
+// Workgroups (a multiple of the 8 XCDs) of a kernel whose workgroups walk over
+// nt tiles of each of n jobs, `slots` of them at a time on the GPU.
+static unsigned stay_grid(int nt, int slots, int n) {
+    const int per = std::min(std::max(slots / n, 64), nt + 7) & ~7;
+    return (unsigned)per;
+}
+
 template <int M>
 static hipError_t y_iter_m(const YIterArgs &a, int nbatch, hipStream_t s) {
-    using S = SShape<M>;
-    const int ncg = (a.Pv + S::B - 1) / S::B;
-    dim3 grid((unsigned)(ncg * a.nz), 1, nbatch);
+    using S = YShape<M>;
+    const int nt = (a.Pv + S::B - 1) / S::B * a.nz;
+    dim3 grid(stay_grid(nt, 256 * S::PER_CU, nbatch), 1, nbatch);
     hipLaunchKernelGGL(k_y_iter<M>, grid, dim3(S::NT), 0, s, a);
     return hipGetLastError();
 }
@@ -967,6 +1127,25 @@ static hipError_t strided_m(const StridedArgs &a, int njobs, int nbatch, hipStre
         }
     }
     const int ncg = (a.Pv + S::B - 1) / S::B;
+    if constexpr (M == 256 || M == 512) {
+        int nout = 0;
+        for (int j = 0; j < njobs; j++) nout = std::max(nout, a.job[j].nout);
+        using K = decltype(&k_strided_n<M, 1, MUL_NONE, 2>);
+        K kernel = nullptr;
+        if (a.pair != 0 && a.Pv <= kStridedNPv) {   // (pair = 0: k_strided for every pass of the axis)
+            if (a.mode == 1 && nout == 2) kernel = k_strided_n<M, 1, MUL_NONE, 2>;
+            if (a.mode == 2 && nout == 2 && a.mul == MUL_I_INVK2) kernel = k_strided_n<M, 2, MUL_I_INVK2, 2>;
+            if (a.mode == 2 && nout == 2 && a.mul == MUL_I) kernel = k_strided_n<M, 2, MUL_I, 2>;
+            if (a.mode == 2 && nout == 3 && a.mul == MUL_INVK2) kernel = k_strided_n<M, 2, MUL_INVK2, 3>;
+        }
+        if (kernel) {
+            // 16 waves per CU over all jobs and batch items
+            const int nt = (a.Pv + 15) / 16 * nother;
+            dim3 grid(stay_grid(nt, 256 * 512 / M, njobs * nbatch), njobs, nbatch);
+            hipLaunchKernelGGL(kernel, grid, dim3(2 * M), 0, s, a);
+            return hipGetLastError();
+        }
+    }
     dim3 grid((unsigned)(ncg * nother), njobs, nbatch);
     hipLaunchKernelGGL(k_strided<M>, grid, dim3(S::NT), 0, s, a);
     return hipGetLastError();

@@ -51,8 +51,9 @@ struct StridedArgs {
     int mul;                   // MulKind (mode 2)
     float R2;                  // smoothing radius squared (FP32)
     float los[3];
-    int pair;                  // kernel of single-output jobs: -1 the library's rule,
-                               // 0 one column per thread, 1 two columns per thread
+    int pair;                  // kernel: -1 the library's rule, 0 k_strided (one column per
+                               // thread) for every job, 1 as -1 with two columns per
+                               // thread for single-output jobs
     // MUL_MG_INV: symbol sum_a gp[a] (2 - 2 cos t_a) + sum_{a<b} cross[ab]
     // sin t_a sin t_b with t_a = k_a cell[a] (cross: xy, xz, yz)
     float mg_gp[3], mg_cross[3], mg_cell[3];

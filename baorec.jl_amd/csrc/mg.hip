@@ -701,21 +701,6 @@ __global__ void __launch_bounds__(kGbThreads) k_mg_gs_tile(float *__restrict__ v
     }
 }
 
-// The reciprocal of b for div_by: one Newton step on v_rcp_f32.
-__device__ __forceinline__ float refined_rcp(float b) {
-    const float y = __builtin_amdgcn_rcpf(b);
-    return __builtin_fmaf(__builtin_fmaf(-b, y, 1.0f), y, y);
-}
-// a / b from y = refined_rcp(b): the correction steps of the IEEE division, so
-// its result where no operand needs scaling (|a| >= 2^-104 or 0, normal b and
-// quotient); zeros, infinities and NaN by v_div_fixup_f32.
-__device__ __forceinline__ float div_by(float a, float b, float y) {
-    float q = a * y;
-    q = __builtin_fmaf(__builtin_fmaf(-b, q, a), y, q);
-    q = __builtin_fmaf(__builtin_fmaf(-b, q, a), y, q);
-    return __builtin_amdgcn_div_fixupf(q, b, a);
-}
-
 // S = 1 or 2 damped Jacobi sweeps in one launch, out of place: vout is what S
 // launches of k_mg_jacobi leave (the same cell arithmetic on the same
 // values, so the same bits).  A workgroup owns a 64 x TY column of tz planes

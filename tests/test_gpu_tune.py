@@ -11,6 +11,8 @@ from baorec_hip import synth
 
 pytestmark = pytest.mark.gpu
 
+F32 = np.float32
+
 
 def box_kw(ctx, los=(0.0, 0.0, 1.0)):
     return dict(bias=2.0, f=0.8, smoothing_radius=15.0, box_size=[1000.0] * 3, box_min=[0.0] * 3,
@@ -78,3 +80,35 @@ def test_failed_tuning_leaves_no_forced_choice():
         rec = bh.IterativeRecon(**box_kw(c))
         out.append(bh.run_(rec, (64, 64, 64), x.copy(), y.copy(), z.copy(), w))
     np.testing.assert_array_equal(out[0], out[1])
+
+
+@pytest.mark.parametrize("los", [(0.0, 0.0, 1.0), None])
+@pytest.mark.parametrize("g", [(16, 256, 512), (1024, 16, 256), (32, 512, 16), (64, 256, 32)])
+def test_staying_passes_match_the_general_ones(tmp_path, g, los):
+    """y and z passes of several outputs at 256 and 512 by workgroups that walk
+    over tiles, against the general kernel (a table that asks for one column
+    per thread), single catalogs and batches, with columns past the last one
+    and fewer tiles than workgroups.  The table also changes the passes of one
+    output, whose two kernels round differently: about 30 FP32 transforms of
+    rms error eps sqrt(log2 n) each, five times that at the largest of 10^6
+    cells is 1e-5 of the field, twice that is allowed (a position: 2e-5 of its
+    displacement, at least that of 20 Mpc/h, and two roundings)."""
+    path = tmp_path / "general.json"
+    path.write_text('{"scatter": [],\n "strided": [\n' +
+                    ",\n".join(f'  {{"axis": {a}, "n": {n}, "pair": 0}}' for a in (1, 2) for n in (256, 512)) + "]}\n")
+    plain, general = bh.Context(0), bh.Context(0)
+    bh.tune_load(path, general)
+    x, y, z, w = synth.box_catalog(60000, L=1000.0, mesh=64, seed=44)
+    off = np.array([0, 20000, 20001, 60000])
+    out = []
+    for ctx in (plain, general):
+        rec = bh.IterativeRecon(**box_kw(ctx, los))
+        d = bh.run_(rec, g, x.copy(), y.copy(), z.copy(), w)
+        p = bh.reconstructed_positions(rec, x, y, z, field="sum")
+        b = bh.run_batch(rec, g, x, y, z, w, off)
+        out.append([d, *p, *b])
+    (d0, *p0), (d1, *p1) = out
+    assert np.max(np.abs(d0 - d1)) <= 2e-5 * np.max(np.abs(d1))
+    for a, b, at in zip(p0, p1, (x, y, z) * 2):
+        shift = np.maximum(np.abs(b - at), 20.0)   # 85 Mpc/h in the catalog of one particle
+        assert np.all(np.abs(a - b) <= 2e-5 * shift + 2 * np.spacing(F32(1000.0)))
