@@ -376,8 +376,8 @@ void scatter(baorec_ctx *c, const Grid &G, const baorec_params *p, Slot *slot, f
     hipchk(c, launch_zero_words(a.wmax, 64, c->stream), "zero");
     (void)tag;
     if (sort_fits(a)) {
-        const int nblk = sort_nblk(n);
         const int T = a.ntx * a.nty * a.ntz;
+        const int nblk = sort_nblk(n, T);
         uint32_t *H = bufT<uint32_t>(c, "sc_hist", (size_t)(nblk > 0 ? nblk : 1) * T);
         ProfScope ps(c, "scatter_bin", (double)n * (a.mutate && wrap ? 40.0 : 28.0) + 16.0 * n * 1.2);
         hipchk(c, launch_sort(a, nblk, H, nullptr, nullptr, nullptr, c->stream), "scatter sort");

@@ -194,7 +194,7 @@ hipError_t launch_zero(float *a, int64_t n, hipStream_t s);
 bool sort_fits(const ScatterArgs &a);
 // Upper bound on the blocks sort_blocks makes for a handful of catalogs.
 constexpr int kSortTableBlocks = 1024;
-int sort_nblk(int64_t n);  // blocks of a single catalog (tables may then be NULL)
+int sort_nblk(int64_t n, int T);  // blocks of a single catalog on T tiles (tables may then be NULL)
 int sort_blocks(int64_t n, const int64_t *offsets_host, int ncat, std::vector<int> &blk_cat,
                 std::vector<int64_t> &blk_beg, std::vector<int> &cat_blk0);
 hipError_t launch_sort(ScatterArgs &a, int nblk, uint32_t *H, const int *blk_cat, const int64_t *blk_beg,

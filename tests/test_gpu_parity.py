@@ -116,6 +116,26 @@ def test_cic_matches_oracle(ctx, grid):
     np.testing.assert_array_equal(gy, oy)
 
 
+@pytest.mark.parametrize("n", [1, 1024, 1025, 9000, 600000])
+@pytest.mark.parametrize("grid", [(32, 32, 16), (256, 128, 64)])
+def test_cic_over_catalog_sizes(ctx, n, grid):
+    """Catalogs of one sort block, a block and a particle, several rows of the
+    block table and all 512, with the largest weight in the first, a middle or
+    the last block (the fixed-point scale comes from it), on few tiles and many."""
+    nx, ny, nz = grid
+    rng = np.random.default_rng(5)
+    x, y, z = (rng.random(n).astype(F32) * F32(1000.0) for _ in range(3))
+    rec = bh.IterativeRecon(**box_kw(1000.0))
+    for at in sorted({0, n // 2, n - 1}):
+        w = (rng.random(n) + 0.5).astype(F32)
+        w[at] = F32(40.0)
+        rho, ref = np.zeros((nz, ny, nx), F32), np.zeros((nz, ny, nx), F32)
+        bh.cic_(rho, x.copy(), y.copy(), z.copy(), w, rec, wrap=True)
+        orc.cic(ref, x.copy(), y.copy(), z.copy(), w, rec.box_size, rec.box_min, wrap=True)
+        assert rel_l2(rho, ref) < 1e-6
+        assert abs(rho.sum(dtype=np.float64) - w.sum(dtype=np.float64)) < 1e-4 * w.sum()
+
+
 def test_cic_nowrap_out_of_box_raises(ctx):
     rec = bh.IterativeRecon(**box_kw(1000.0))
     rho = np.zeros((16, 16, 16), F32)
