@@ -796,6 +796,7 @@ struct MGPyr {
     std::vector<int> zero;             // 1: v is zero and not stored (its next fused sweep reads none)
     int lc = 0;                        // levels >= lc run in one k_mg_coarse or k_mg_small launch
     bool small = false;                // k_mg_small: levels >= lc stay in LDS
+    const double *cop = nullptr;       // its coarsest level's operator (mg_coarse_op)
 };
 
 // Levels of at most this many cells are latency-bound: they run inside one
@@ -980,6 +981,7 @@ void mg_small(baorec_ctx *c, MGPyr &P, const baorec_params *p, int fmg, int gs, 
     a.f = P.dbl[l] ? static_cast<const void *>(P.Fd[l]) : static_cast<const void *>(P.F[l]);
     a.vin = zero || fmg ? nullptr : v;
     a.vout = v;
+    a.cop = gs ? P.cop : nullptr;
     a.fmg = fmg;
     a.gs = gs;
     a.beta = p->beta;
@@ -990,6 +992,18 @@ void mg_small(baorec_ctx *c, MGPyr &P, const baorec_params *p, int fmg, int gs, 
     a.vcycles = p->vcycle_niterations;
     ProfScope ps(c, "mg_small", 0.0);
     hipchk(c, launch_mg_small(a, c->stream), "mg small levels");
+}
+
+// Once per RBGS solve: what the coarsest level's sweeps before and after (16
+// times the others') leave from zero, as a matrix, where k_mg_small runs it
+// below another level.
+void mg_coarse_op(baorec_ctx *c, MGPyr &P, const baorec_params *p) {
+    const int l = (int)P.g.size() - 1;
+    if (!P.small || l <= P.lc || !P.dbl[l] || P.g[l].R() > 64) return;
+    double *cop = bufT<double>(c, "mg_cop", 64 * 64);
+    ProfScope ps(c, "mg_coarse_op", 0.0);
+    hipchk(c, launch_mg_coarse_op(P.L[l], 32 * p->rb_sweeps, p->beta, p->has_los, cop, c->stream), "coarse operator");
+    P.cop = cop;
 }
 
 // The FP32 residual of level l restricted to the right-hand side of level
@@ -1424,6 +1438,7 @@ void multigrid_solve(baorec_ctx *c, const Grid &G, baorec_params *p, Slot *slot,
     float *rb[2] = {bufT<float>(c, "mg_r0", N), bufT<float>(c, "mg_r1", N)};
     double *phi = bufT<double>(c, "mg_phi64", N);   // FP64 solution (set by the first residual call)
     MGPyr P = mg_build(c, G, p, slot, v0, rb[0], p->fp64_coarse_max);
+    mg_coarse_op(c, P, p);
     // With sides that are multiples of 64, 16 and 8 the refinement step
     // (phi += e - mean(e), r = f - alpha - A phi, sum r) is one z-marching
     // pass (k_mg_refine) and the shift with both norms another; otherwise

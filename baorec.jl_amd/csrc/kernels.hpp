@@ -326,10 +326,15 @@ struct MGSmall {
         off_p[kMGSmallLevels];   // bytes
     const void *f, *vin;
     void *vout;
+    const double *cop;   // gs: the coarsest level's operator (launch_mg_coarse_op), or NULL
     int fmg, gs;
     float beta, omega;
     int has_los, jacobi_n, rb_sweeps, vcycles;
 };
+// cop[j][i]: cell i of a level L of n <= 64 cells (power-of-two sides) after
+// `sweeps` FP64 colour sweeps from zero on the right-hand side that is 1 in
+// cell j and 0 elsewhere.
+hipError_t launch_mg_coarse_op(const MGLevel &L, int sweeps, float beta, int has_los, double *cop, hipStream_t s);
 bool mg_small_layout(MGSmall &a);
 hipError_t launch_mg_small(const MGSmall &a, hipStream_t s);
 

@@ -1671,10 +1671,11 @@ __global__ void __launch_bounds__(1024) k_mg_coarse(MGCoarse<T> a) {
 // stage is a round trip to the L2 and levels above 512 cells a launch per
 // stage.  Every address is an index into `pool` from masked coordinates; the
 // host checks that the levels' arrays fit (mg_small_layout).  What remains is
-// the coarsest FP64 level's serial colour passes (256 per V-cycle).  Measured
-// for 16^3 (FP32) | 8^3 | 4^3 (FP64): 71 us per V-cycle, against 138 us in
-// k_mg_coarse for the lower two alone and eight launches for 16^3; the Jacobi
-// levels 16^3 .. 4^3 of a reference V-cycle 58 us.
+// a barrier per colour pass and stage.  Measured for 16^3 (FP32) | 8^3 | 4^3
+// (FP64): 48 us per V-cycle (71 with the coarsest level's 256 colour passes
+// instead of a.cop), against 138 us in k_mg_coarse for the lower two alone and
+// eight launches for 16^3; the Jacobi levels 16^3 .. 4^3 of a reference
+// V-cycle 58 us.
 constexpr int kMGSmallPool = 120 * 1024;   // bytes
 
 template <typename T>
@@ -1987,6 +1988,7 @@ __device__ __forceinline__ void small_prolong(const LdsLevel<T> &l, const LdsLev
 template <int GS>
 __global__ void __launch_bounds__(1024) k_mg_small(MGSmall a) {
     __shared__ __align__(16) char pool[kMGSmallPool];
+    __shared__ double red[GS ? 16 : 1][64];
     const int nl = a.nl;
     uint32_t swapped = 0;   // bit l: an odd number of Jacobi sweeps so far, v and r exchanged
     auto lev = [&](auto tag, int l) {
@@ -2050,10 +2052,28 @@ __global__ void __launch_bounds__(1024) k_mg_small(MGSmall a) {
             small_prolong<float, float>(lev(float(), l), lev(float(), l + 1), add);
     };
     // down from level top (pre-smooth, residual, restrict) to the coarsest,
-    // which smooths twice, and up again (prolong and add, post-smooth)
+    // which smooths twice (with a.cop: both at once, its v being zero), and up
+    // again (prolong and add, post-smooth)
     auto vcycle = [&](int top) __attribute__((always_inline)) {
         bool pre = true;
         for (int l = top;;) {
+            if (GS && a.cop && l + 1 == nl && l > top) {
+                const auto d = lev(double(), l);
+                const int i = threadIdx.x & 63, w = threadIdx.x >> 6;
+                double s = 0.0;
+                for (int j = w; j < d.n; j += 16) s = mg_fma(a.cop[j * 64 + i], d.f[j], s);
+                red[w][i] = s;
+                __syncthreads();
+                if (threadIdx.x < d.n) {
+                    s = red[0][i];
+                    for (int k = 1; k < 16; k++) s += red[k][i];
+                    d.v[i] = s;
+                }
+                __syncthreads();
+                pre = false;
+                l--;
+                up(l, true);
+            }
             smooth(l);
             if (pre && l + 1 < nl) {
                 down(l);
@@ -2120,6 +2140,36 @@ __global__ void __launch_bounds__(1024) k_mg_small(MGSmall a) {
         out(double());
     else
         out(float());
+}
+
+// launch_mg_coarse_op: workgroup j (one wave) runs the sweeps on the unit vector
+// of cell j.  A V-cycle's coarsest level starts from zero, so what its sweeps
+// (2 x 32 x 4 dependent colour passes by default, 24 of the 71 us of k_mg_small)
+// leave is this matrix times its right-hand side, the same for all V-cycles
+// of a solve: 24 us once, then 1 us each.
+__global__ void __launch_bounds__(64) k_mg_coarse_op(MGLevel L, int sweeps, float beta, int has_los, int lx, int ly,
+                                                     int lz, double *cop) {
+    __shared__ double v[64], f[64], p[192];
+    const int i = threadIdx.x;
+    v[i] = 0.0;
+    f[i] = i == (int)blockIdx.x ? 1.0 : 0.0;
+    if (!has_los)
+        for (int k = i; k < L.n[0] + L.n[1] + L.n[2]; k += 64) {
+            const float cell = k < L.n[0] ? L.cell[0] : (k < L.n[0] + L.n[1] ? L.cell[1] : L.cell[2]);
+            p[k] = (double)L.xv[k] / (double)cell;
+        }
+    __syncthreads();
+    LdsLevel<double> d;
+    d.v = v;
+    d.f = f;
+    d.r = nullptr;
+    d.p = p;
+    d.lx = lx;
+    d.ly = ly;
+    d.lz = lz;
+    d.n = 1 << (lx + ly + lz);
+    small_gs_wave(d, L, sweeps, beta, has_los);
+    cop[blockIdx.x * 64 + i] = v[i];
 }
 
 // Cell centres of every level (x_vec per level, src/multigrid.jl:656).
@@ -2501,6 +2551,19 @@ hipError_t launch_mg_small(const MGSmall &a0, hipStream_t s) {
             if (a.dbl[l]) return hipErrorInvalidValue;
         hipLaunchKernelGGL(k_mg_small<0>, dim3(1), dim3(1024), 0, s, a);
     }
+    return hipGetLastError();
+}
+
+hipError_t launch_mg_coarse_op(const MGLevel &L, int sweeps, float beta, int has_los, double *cop, hipStream_t s) {
+    int lg[3], n = 1;
+    for (int k = 0; k < 3; k++) {
+        if (L.n[k] < 2 || (L.n[k] & (L.n[k] - 1))) return hipErrorInvalidValue;
+        lg[k] = __builtin_ctz((unsigned)L.n[k]);
+        n *= L.n[k];
+    }
+    if (n > 64) return hipErrorInvalidValue;
+    hipLaunchKernelGGL(k_mg_coarse_op, dim3((unsigned)n), dim3(64), 0, s, L, sweeps, beta, has_los, lg[0], lg[1],
+                       lg[2], cop);
     return hipGetLastError();
 }
 
