@@ -905,7 +905,7 @@ double *votherd(MGPyr &P, int l) { return P.cur[l] ? P.Ad[l] : P.Bd[l]; }
 // between a (the input) and b; returns the one holding the result.  On
 // grids of at least 128^3 cells whose sides are multiples of 64, 16 and 8,
 // sweeps run two per z-marching launch, and an odd one as such a launch of
-// its own (the same bits).
+// its own (the same bits either way).
 static float *jacobi_sweeps(baorec_ctx *c, const MGLevel &L, int64_t R, float *a, float *b, const float *f,
                             const baorec_params *p, int n) {
     const bool tb = mg_jacobi_tb_ok(L) && R >= ((int64_t)1 << 21);

@@ -701,9 +701,54 @@ __global__ void __launch_bounds__(kGbThreads) k_mg_gs_tile(float *__restrict__ v
     }
 }
 
-// S = 1 or 2 damped Jacobi sweeps in one launch, out of place: vout is what S
-// launches of k_mg_jacobi leave (the same cell arithmetic on the same
-// values, so the same bits).  A workgroup owns a 64 x TY column of tz planes
+// The damped Jacobi update of the z-marching launches, jacobi! of
+// src/multigrid.jl:193-210 with its sums as fused multiply-adds: 44
+// operations per update where the reference's order of products and sums took
+// 70, each result rounded fewer times than there.  The divisions are
+// refined_rcp and one correction of the quotient (within 0.51 ulp).  Against
+// FP64, local LOS, rms: 6.2e-8 after one sweep of 128^3 (6.4e-8 in the reference's
+// order), 1.7e-7 after six (1.8e-7).
+struct JbCell {
+    float px, py, pz, px2, py2, pz2;   // LOS component in cell units, squared
+};
+__device__ __forceinline__ float jb_div(float a, float b) {
+    const float y = refined_rcp(b), q = a * y;
+    return __builtin_fmaf(__builtin_fmaf(-b, q, a), y, q);
+}
+// beta / |x|^2 of a cell
+__device__ __forceinline__ float jb_g(const MGLevel &L, const JbCell &c, float beta) {
+    return jb_div(beta, __builtin_fmaf(L.cell2[1], c.py2, L.cell2[0] * c.px2) + L.cell2[2] * c.pz2);
+}
+// the new value from f, the 18 neighbours (argument order of nbr_of) and the value
+template <int LOS>
+__device__ __forceinline__ float jb_update(const MGLevel &L, const JbCell &c, float g, float omega, float f, float v,
+                                           float vxp, float vxm, float vyp, float vym, float vzp, float vzm, float xpyp,
+                                           float xmym, float xmyp, float xpym, float xpzp, float xmzm, float xmzp,
+                                           float xpzm, float ypzp, float ymzm, float ymzp, float ypzm) {
+    const float gx = __builtin_fmaf(g, c.px2, L.icell2[0]), gy = __builtin_fmaf(g, c.py2, L.icell2[1]);
+    const float gz = __builtin_fmaf(g, c.pz2, L.icell2[2]);
+    float j = __builtin_fmaf(gx, vxp + vxm, f);
+    j = __builtin_fmaf(gy, vyp + vym, j);
+    j = __builtin_fmaf(gz, vzp + vzm, j);
+    const float exy = (xpyp + xmym) - (xmyp + xpym), exz = (xpzp + xmzm) - (xmzp + xpzm);
+    const float eyz = (ypzp + ymzm) - (ymzp + ypzm);
+    const float hx = 0.5f * c.px, hz = 0.5f * c.pz;
+    float t = (hx * c.py) * exy;
+    t = __builtin_fmaf(hx * c.pz, exz, t);
+    t = __builtin_fmaf(hz * c.py, eyz, t);
+    if (!LOS) {
+        t = __builtin_fmaf(c.px, vxp - vxm, t);
+        t = __builtin_fmaf(c.py, vyp - vym, t);
+        t = __builtin_fmaf(c.pz, vzp - vzm, t);
+    }
+    j = __builtin_fmaf(g, t, j);
+    // j / (2 (gx + gy + gz)), the 1/2 in the weight
+    return __builtin_fmaf(0.5f * omega, jb_div(j, (gx + gy) + gz), (1.0f - omega) * v);
+}
+
+// S = 1 or 2 damped Jacobi sweeps in one launch, out of place: S = 2 leaves
+// what two launches of S = 1 do (the same operations on the same values, so
+// the same bits).  A workgroup owns a 64 x TY column of tz planes
 // and marches up z; sweep level t (t = 1..S) of the tile, grown by S - t cells
 // in x and y, lives in a ring of 4 LDS planes (level 0: the old values,
 // loaded).  Step k loads plane P = z0 - S + k and computes level t on plane
@@ -711,18 +756,18 @@ __global__ void __launch_bounds__(kGbThreads) k_mg_gs_tile(float *__restrict__ v
 // in earlier steps, and the stages of one step touch disjoint planes, so one
 // barrier per step orders them.  Level S goes straight to vout.
 //
-// What bounds it is the arithmetic (about 65 operations per update in the
-// reference's order, two of them divisions), so the mapping saves
+// What bounds it is the arithmetic, so the mapping saves
 // instructions: a wave owns 4 rows of the tile, a column per lane, at every
 // level.  Its y and z coefficients are uniform, a row's loads serve the row
 // beside it (28 LDS reads per 2 cells instead of 38), and a cell's g and f stay
-// in registers from level 1 to level 2, two steps later: one IEEE division
-// per cell and pass.  The division by the diagonal has no scaling steps
-// (div_by).  The tile's halo cells of level 1 (rows -1 and TY, columns -1 and
+// in registers from level 1 to level 2, two steps later.  The tile's halo
+// cells of level 1 (rows -1 and TY, columns -1 and
 // 64) are one extra cell per lane.  Three waves per SIMD, 168 VGPRs: with the
 // reciprocals kept as well it spilled (401 against 324 us per sweep), and tiles
 // of 32 rows, one workgroup per CU, ran 376-430 us.
-// Per sweep, local LOS, 512^3 / 256^3 / 128^3: 324 / 47 / 12 us; with two
+// Per sweep, local LOS, 512^3 / 256^3 / 128^3: 298 / 44 / 12 us (one sweep per
+// pass 336 / 39 / 12, at the copy rate); with the reference's
+// order of operations 347 / 53 / 13 us; with two IEEE
 // divisions per update and cells dealt to the threads level by level, 2 or 3
 // sweeps per launch, 560 / 73 / 14 us.
 constexpr int kJbTX = 64, kJbRing = 4, kJbMaxTz = 128;
@@ -779,7 +824,7 @@ __global__ void __launch_bounds__(JbShape<S>::Threads, 3) k_mg_jacobi_zm(float *
     };
     // the lane's column and the wave's rows 4 wave .. 4 wave + 3
     const int row0 = 4 * wave;
-    const float px = LOS ? L.losn[0] : L.pv[x0 + lane], px2 = px * px, qx = L.cell2[0] * px2;
+    const float px = LOS ? L.losn[0] : L.pv[x0 + lane];
     float py[4];
 #pragma unroll
     for (int j = 0; j < 4; j++) py[j] = LOS ? L.losn[1] : L.pv[nx + y0 + row0 + j];
@@ -817,14 +862,6 @@ __global__ void __launch_bounds__(JbShape<S>::Threads, 3) k_mg_jacobi_zm(float *
     };
     // p of a plane of the tile or of its halo
     auto pz_of = [&](int P) { return LOS ? L.losn[2] : L.pv[nx + ny + gs_wrap(P, nz)]; };
-    // the new value of a cell from its coefficients, diagonal, f, neighbour
-    // sums and value (jacobi_value's operations in its order)
-    auto update = [&](const Coef<float> &c, float D, float fv, const Nbr<float> &s, float v) {
-        float j = fv + s.A + s.B + s.C + s.X;
-        if (!LOS) j += s.G;
-        j = div_by(j, D, refined_rcp(D));
-        return (1.0f - omega) * v + omega * j;
-    };
     // four rows of one level: from the ring planes below, at and above, row
     // pitch W, at word w (row0 of the lane's column); level 1 (FIRST) makes
     // the coefficients, a later level takes them from the ring
@@ -832,7 +869,6 @@ __global__ void __launch_bounds__(JbShape<S>::Threads, 3) k_mg_jacobi_zm(float *
                     int slot, float (&out)[4]) {
         constexpr bool FIRST = decltype(first)::value;
         constexpr int W = decltype(wpitch)::value;
-        const float pz2 = pz * pz, qz = L.cell2[2] * pz2;
         // two rows at a time (all four rows' values at once cost registers and
         // with them a wave per SIMD); the level's start and end are kept apart
         // from the other level's, whose loads would otherwise be hoisted
@@ -859,24 +895,12 @@ __global__ void __launch_bounds__(JbShape<S>::Threads, 3) k_mg_jacobi_zm(float *
 #pragma unroll
             for (int j = 0; j < 2; j++) {
                 const int jr = h + j;
-                const float py2 = py[jr] * py[jr];
-                Coef<float> c;
-                c.px = px;
-                c.py = py[jr];
-                c.pz = pz;
-                if constexpr (FIRST)
-                    c.g = beta / ((qx + L.cell2[1] * py2) + qz);
-                else
-                    c.g = gr[slot][jr];
-                c.gpx2 = L.icell2[0] + c.g * px2;
-                c.gpy2 = L.icell2[1] + c.g * py2;
-                c.gpz2 = L.icell2[2] + c.g * pz2;
-                const float D = 2.0f * (c.gpx2 + c.gpy2 + c.gpz2);
-                if constexpr (FIRST) gr[slot][jr] = c.g;
-                const Nbr<float> s =
-                    nbr_of<float>(c, r0[j + 1], l0[j + 1], c0[j + 2], c0[j], cp[j + 1], cm[j + 1], r0[j + 2], l0[j],
-                                  l0[j + 2], r0[j], rp[j], lm[j], lp[j], rm[j], cp[j + 2], cm[j], cp[j], cm[j + 2]);
-                out[jr] = update(c, D, fr[slot][jr], s, c0[j + 1]);
+                const JbCell c{px, py[jr], pz, px * px, py[jr] * py[jr], pz * pz};
+                const float g = FIRST ? jb_g(L, c, beta) : gr[slot][jr];
+                if constexpr (FIRST) gr[slot][jr] = g;
+                out[jr] = jb_update<LOS>(L, c, g, omega, fr[slot][jr], c0[j + 1], r0[j + 1], l0[j + 1], c0[j + 2],
+                                         c0[j], cp[j + 1], cm[j + 1], r0[j + 2], l0[j], l0[j + 2], r0[j], rp[j], lm[j],
+                                         lp[j], rm[j], cp[j + 2], cm[j], cp[j], cm[j + 2]);
             }
         }
         __builtin_amdgcn_sched_barrier(0);
@@ -909,16 +933,14 @@ __global__ void __launch_bounds__(JbShape<S>::Threads, 3) k_mg_jacobi_zm(float *
 #pragma unroll
                 for (int j = 0; j < 4; j++) pl[w1 + j * J::W1] = o[j];
                 if (ex_on) {
-                    const Coef<float> c = coef_p<float>(L, ex_px, ex_py, pz, beta);
-                    const float D = 2.0f * (c.gpx2 + c.gpy2 + c.gpz2);
+                    const JbCell c{ex_px, ex_py, pz, ex_px * ex_px, ex_py * ex_py, pz * pz};
 #define A0(q) p0[ex_w0 + (q)]
 #define AM(q) pm[ex_w0 + (q)]
 #define AP(q) pp[ex_w0 + (q)]
-                    const Nbr<float> s = nbr_of<float>(
-                        c, A0(1), A0(-1), A0(J::W0), A0(-J::W0), AP(0), AM(0), A0(J::W0 + 1), A0(-J::W0 - 1),
-                        A0(J::W0 - 1), A0(-J::W0 + 1), AP(1), AM(-1), AP(-1), AM(1), AP(J::W0), AM(-J::W0),
-                        AP(-J::W0), AM(J::W0));
-                    pl[ex_w1] = update(c, D, exf, s, A0(0));
+                    pl[ex_w1] = jb_update<LOS>(
+                        L, c, jb_g(L, c, beta), omega, exf, A0(0), A0(1), A0(-1), A0(J::W0), A0(-J::W0), AP(0), AM(0),
+                        A0(J::W0 + 1), A0(-J::W0 - 1), A0(J::W0 - 1), A0(-J::W0 + 1), AP(1), AM(-1), AP(-1), AM(1),
+                        AP(J::W0), AM(-J::W0), AP(-J::W0), AM(J::W0));
 #undef A0
 #undef AM
 #undef AP
