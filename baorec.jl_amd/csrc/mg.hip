@@ -705,7 +705,8 @@ __global__ void __launch_bounds__(kGbThreads) k_mg_gs_tile(float *__restrict__ v
 // src/multigrid.jl:193-210 with its sums as fused multiply-adds: 44
 // operations per update where the reference's order of products and sums took
 // 70, each result rounded fewer times than there.  The divisions are
-// refined_rcp and one correction of the quotient (within 0.51 ulp).  Against
+// refined_rcp and one correction of the quotient (within 0.51 ulp; zeros,
+// infinities and NaN by v_div_fixup_f32, as in an IEEE division).  Against
 // FP64, local LOS, rms: 6.2e-8 after one sweep of 128^3 (6.4e-8 in the reference's
 // order), 1.7e-7 after six (1.8e-7).
 struct JbCell {
@@ -713,7 +714,7 @@ struct JbCell {
 };
 __device__ __forceinline__ float jb_div(float a, float b) {
     const float y = refined_rcp(b), q = a * y;
-    return __builtin_fmaf(__builtin_fmaf(-b, q, a), y, q);
+    return __builtin_amdgcn_div_fixupf(__builtin_fmaf(__builtin_fmaf(-b, q, a), y, q), b, a);
 }
 // beta / |x|^2 of a cell
 __device__ __forceinline__ float jb_g(const MGLevel &L, const JbCell &c, float beta) {
@@ -765,8 +766,8 @@ __device__ __forceinline__ float jb_update(const MGLevel &L, const JbCell &c, fl
 // 64) are one extra cell per lane.  Three waves per SIMD, 168 VGPRs: with the
 // reciprocals kept as well it spilled (401 against 324 us per sweep), and tiles
 // of 32 rows, one workgroup per CU, ran 376-430 us.
-// Per sweep, local LOS, 512^3 / 256^3 / 128^3: 298 / 44 / 12 us (one sweep per
-// pass 336 / 39 / 12, at the copy rate); with the reference's
+// Per sweep, local LOS, 512^3 / 256^3 / 128^3: 306 / 45 / 12 us (one sweep per
+// pass 341 / 40 / 12, at the copy rate); with the reference's
 // order of operations 347 / 53 / 13 us; with two IEEE
 // divisions per update and cells dealt to the threads level by level, 2 or 3
 // sweeps per launch, 560 / 73 / 14 us.

@@ -95,7 +95,7 @@ def test_zmarching_jacobi_matches_oracle(ctx, shape, los, sweeps):
     """The z-marching Jacobi launches (one and two sweeps) on grids whose
     tiles' halos wrap onto themselves in y or z, odd numbers of tiles
     included, against the FP32 oracle's sweeps (jacobi!, src/multigrid.jl:
-    193-210): the same operations in the same order, so at most the rounding
+    193-210): the same sums, their products fused, so at most the rounding
     of one update (a few 1e-7 of the largest value) per sweep apart."""
     v, f = fields(shape, 11 + sweeps)
     rec = recon(shape, los, ctx)
@@ -107,6 +107,26 @@ def test_zmarching_jacobi_matches_oracle(ctx, shape, los, sweeps):
     err = float(np.max(np.abs(got - exp)) / np.abs(exp).max())
     print(f"{shape} los {los} x{sweeps}: max |diff| / max |v| {err:.1e}")
     assert err < 5e-7 * sweeps
+
+
+@pytest.mark.parametrize("sweeps", [1, 2])
+def test_zmarching_jacobi_keeps_infinities(ctx, sweeps):
+    """A cell of f at +-infinity or NaN gives the z-marching launches the
+    infinities and NaN that the oracle's division gives, at the same cells."""
+    shape = (128, 128, 128)
+    v, f = fields(shape, 17)
+    for i, bad in enumerate((np.inf, -np.inf, np.nan)):
+        f.flat[(1 + i) * 500001] = bad
+    rec = recon(shape, None, ctx)
+    rec.jacobi_niterations = sweeps
+    o = orc.MultigridRecon(bias=2.0, f=0.8, smoothing_radius=15.0, box_size=rec.box_size, box_min=rec.box_min,
+                           los=None)
+    got = bh.jacobi_(v.copy(), f, rec)
+    with np.errstate(invalid="ignore"):
+        exp = orc.mg_jacobi(v.copy(), f, o.box_size, o.box_min, o.beta, 0.4, sweeps, los=o.los)
+    np.testing.assert_array_equal(np.isnan(got), np.isnan(exp))
+    np.testing.assert_array_equal(got == np.inf, exp == np.inf)
+    np.testing.assert_array_equal(got == -np.inf, exp == -np.inf)
 
 
 @pytest.mark.parametrize("shape,los", [((128, 128, 128), None), ((64, 64, 512), [0.0, 0.0, 1.0]),
