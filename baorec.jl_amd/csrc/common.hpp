@@ -54,19 +54,10 @@ struct Slot {
 // Twiddles come from one table: tw[S + i] = exp(-2 pi i * i / S) for every
 // power of two S <= 2048 (4096 float2 in total).
 
-// The reciprocal of b for div_by: one Newton step on v_rcp_f32.
+// The reciprocal of b: one Newton step on v_rcp_f32.
 __device__ __forceinline__ float refined_rcp(float b) {
     const float y = __builtin_amdgcn_rcpf(b);
     return __builtin_fmaf(__builtin_fmaf(-b, y, 1.0f), y, y);
-}
-// a / b from y = refined_rcp(b): the correction steps of the IEEE division, so
-// its result where no operand needs scaling (|a| >= 2^-104 or 0, normal b and
-// quotient); zeros, infinities and NaN by v_div_fixup_f32.
-__device__ __forceinline__ float div_by(float a, float b, float y) {
-    float q = a * y;
-    q = __builtin_fmaf(__builtin_fmaf(-b, q, a), y, q);
-    q = __builtin_fmaf(__builtin_fmaf(-b, q, a), y, q);
-    return __builtin_amdgcn_div_fixupf(q, b, a);
 }
 
 // Workgroup barrier for exchanges through LDS alone: __syncthreads without its

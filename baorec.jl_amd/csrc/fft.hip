@@ -496,22 +496,19 @@ __device__ __forceinline__ float2 apply_mul(float2 F, float kx, float ky, float 
             const double g = exp(-0.5 * (double)R2 * (double)k2);
             return make_float2((float)((double)F.x * g), (float)((double)F.y * g));
         }
-        case MUL_INVK2: {
-            const float d = k2 > 0.f ? k2 : 1.f, y = refined_rcp(d);
-            F = make_float2(div_by(F.x, d, y), div_by(F.y, d, y));
-            return k2 > 0.f ? F : make_float2(0.f, 0.f);
-        }
+        // IEEE quotients: any k^2 that is not zero (boxes in any unit of length) and
+        // an overflow to infinity come out as they should.  The divisions cost the
+        // 512^3 passes 2% (606 us; 596 with a shared reciprocal and corrected
+        // quotients, which lose k^2 above 2^126 and give NaN for an overflow).
+        case MUL_INVK2:
+            return k2 > 0.f ? make_float2(F.x / k2, F.y / k2) : make_float2(0.f, 0.f);
         case MUL_FIXEDLOS: {
             if (!(k2 > 0.f)) return make_float2(0.f, 0.f);
             const float m = ((kx * kx) * l0 + (ky * ky) * l1) + (kz * kz) * l2;
-            const float y = refined_rcp(k2);
-            return cscale(make_float2(div_by(F.x, k2, y), div_by(F.y, k2, y)), m);
+            return cscale(make_float2(F.x / k2, F.y / k2), m);
         }
-        case MUL_I_INVK2: {
-            const float d = k2 > 0.f ? k2 : 1.f, y = refined_rcp(d);
-            F = make_float2(div_by(-F.y, d, y), div_by(F.x, d, y));
-            return k2 > 0.f ? F : make_float2(0.f, 0.f);
-        }
+        case MUL_I_INVK2:
+            return k2 > 0.f ? make_float2(-F.y / k2, F.x / k2) : make_float2(0.f, 0.f);
         case MUL_I:
             return make_float2(-F.y, F.x);
         case MUL_GAUSS1: {

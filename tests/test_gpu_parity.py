@@ -912,3 +912,54 @@ def test_power_multipoles_full_size_poisson(ctx):
     sig = shot / np.sqrt(out["nmodes"][ok])
     assert ok.sum() > 30
     assert np.all(np.abs(out["p0"][ok]) < 5 * sig + 0.01 * shot)
+
+
+# ------------------------------------------------------------------ units of length
+
+def unit_scale(k2, limit=127.9):
+    """The largest s for which boxes 2^s times smaller keep the value k2 (in
+    1 / length^2) below 2^limit: between 2^126, above which v_rcp_f32 flushes
+    its result to zero, and the largest float."""
+    s = int(np.floor((limit - np.log2(k2)) / 2))
+    assert 126 < np.log2(k2) + 2 * s < 128
+    return s
+
+
+@pytest.mark.parametrize("los", [[0.0, 0.0, 1.0], None])
+@pytest.mark.parametrize("grid", [(32, 32, 32), (16, 32, 256), (32, 512, 16)])
+def test_reconstruction_in_any_unit_of_length(ctx, grid, los):
+    """A box 2^s times smaller gives the same overdensity and displacements
+    2^s times smaller: scaling by powers of two is exact in every step, up to
+    the few smallest modes of F / k^2 that become subnormal.  s brings the
+    largest k^2 close to the largest float, beyond the range of a hardware
+    reciprocal."""
+    L = np.array([1000.0, 900.0, 1100.0])
+    s = unit_scale(sum((np.pi * n / l) ** 2 for n, l in zip(grid, L)))
+    x, y, z, w = synth.box_catalog(60000, L=900.0, mesh=64, seed=45)
+    out = []
+    for u in (1.0, 2.0 ** -s):
+        rec = bh.IterativeRecon(bias=2.0, f=0.8, smoothing_radius=4.0 * u, box_size=[float(l * u) for l in L],
+                                box_min=[200.0 * u] * 3, los=los, ctx=ctx)
+        p = [(v + F32(200.0)) * F32(u) for v in (x, y, z)]
+        d = bh.run_(rec, grid, *(v.copy() for v in p), w)
+        out.append((d, [a / F32(u) for a in bh.read_shifts(rec, *p, d, field="disp")]))
+    (d0, p0), (d1, p1) = out
+    assert rel_l2(d1, d0) < 1e-6
+    for a, b in zip(p1, p0):
+        assert rel_l2(a, b) < 1e-6
+
+
+@pytest.mark.parametrize("los", [[0.6, 0.0, 0.8], None])
+def test_small_levels_fmg_in_any_unit_of_length(ctx, los):
+    """The same for the reference's multigrid schedule on levels in one
+    workgroup's LDS, the diagonal of the finest one above 2^126."""
+    f = np.random.default_rng(46).standard_normal((16, 16, 16)).astype(F32)
+    f -= f.mean()
+    s = unit_scale(2 * 3.4 * (16 / 1000.0) ** 2)
+    out = []
+    for u, scale in ((1.0, 1.0), (2.0 ** -s, 2.0 ** 30)):
+        rec = bh.MultigridRecon(bias=2.0, f=0.8, smoothing_radius=15.0, box_size=[1000.0 * u] * 3,
+                                box_min=[600.0 * u, -200.0 * u, 300.0 * u], los=los, ctx=ctx)
+        out.append(bh.fmg(f * F32(scale), rec).astype(np.float64) / (scale * u * u))
+    assert np.all(np.isfinite(out[1]))
+    assert rel_l2(out[1], out[0]) < 1e-6
