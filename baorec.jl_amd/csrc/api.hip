@@ -908,7 +908,7 @@ double *votherd(MGPyr &P, int l) { return P.cur[l] ? P.Ad[l] : P.Bd[l]; }
 // its own (the same bits either way).
 static float *jacobi_sweeps(baorec_ctx *c, const MGLevel &L, int64_t R, float *a, float *b, const float *f,
                             const baorec_params *p, int n) {
-    const bool tb = mg_jacobi_tb_ok(L) && R >= ((int64_t)1 << 21);
+    const bool tb = mg_jacobi_tb_ok(L, p->beta) && R >= ((int64_t)1 << 21);
     for (int left = n; left > 0;) {
         const int k = tb && left >= 2 ? 2 : 1;
         ProfScope ps(c, k == 1 ? "mg_jacobi" : "mg_jacobi_tb", 12.0 * R);

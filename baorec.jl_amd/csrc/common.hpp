@@ -54,12 +54,6 @@ struct Slot {
 // Twiddles come from one table: tw[S + i] = exp(-2 pi i * i / S) for every
 // power of two S <= 2048 (4096 float2 in total).
 
-// The reciprocal of b: one Newton step on v_rcp_f32.
-__device__ __forceinline__ float refined_rcp(float b) {
-    const float y = __builtin_amdgcn_rcpf(b);
-    return __builtin_fmaf(__builtin_fmaf(-b, y, 1.0f), y, y);
-}
-
 // Workgroup barrier for exchanges through LDS alone: __syncthreads without its
 // fence on memory, which would wait for copies into LDS that are still in
 // flight (k_y_iter's).

@@ -364,7 +364,7 @@ hipError_t launch_mg_rbgs(T *v, const T *f, const MGLevel &L, float beta, int ha
                           hipStream_t s);
 // 1 or 2 damped Jacobi sweeps in one z-marching launch, out of place (vout !=
 // vin), bitwise that many launch_mg_jacobi calls; sides multiples of 64, 16, 8.
-bool mg_jacobi_tb_ok(const MGLevel &L);
+bool mg_jacobi_tb_ok(const MGLevel &L, float beta);
 hipError_t launch_mg_jacobi_tb(float *vout, const float *vin, const float *f, const MGLevel &L, float beta,
                                float omega, int has_los, int sweeps, hipStream_t s);
 // One whole 4-colour sweep out of place (vout != vin), bitwise the four

@@ -704,28 +704,40 @@ __global__ void __launch_bounds__(kGbThreads) k_mg_gs_tile(float *__restrict__ v
 // The damped Jacobi update of the z-marching launches, jacobi! of
 // src/multigrid.jl:193-210 with its sums as fused multiply-adds: 44
 // operations per update where the reference's order of products and sums took
-// 70, each result rounded fewer times than there.  The divisions are
-// refined_rcp and one correction of the quotient (within 0.51 ulp; zeros,
-// infinities and NaN by v_div_fixup_f32, as in an IEEE division).  Against
+// 70, each result rounded fewer times than there.  Against
 // FP64, local LOS, rms: 6.2e-8 after one sweep of 128^3 (6.4e-8 in the reference's
 // order), 1.7e-7 after six (1.8e-7).
 struct JbCell {
     float px, py, pz, px2, py2, pz2;   // LOS component in cell units, squared
 };
-__device__ __forceinline__ float jb_div(float a, float b) {
-    const float y = refined_rcp(b), q = a * y;
-    return __builtin_amdgcn_div_fixupf(__builtin_fmaf(__builtin_fmaf(-b, q, a), y, q), b, a);
+// a / b within 0.51 ulp where nothing leaves the range of normal numbers: one
+// Newton step on v_rcp_f32 and one correction of the quotient.  A divisor that
+// is subnormal, above 2^126, zero, infinite or NaN, an overflow and a
+// non-finite a make it zero, infinite or NaN (v_rcp_f32 flushes subnormal
+// results, inf - inf in the remainder); jb_g and jb_update check for those.
+__device__ __forceinline__ float jb_quot(float a, float b) {
+    const float r = __builtin_amdgcn_rcpf(b), y = __builtin_fmaf(__builtin_fmaf(-b, r, 1.0f), r, r), q = a * y;
+    return __builtin_fmaf(__builtin_fmaf(-b, q, a), y, q);
 }
-// beta / |x|^2 of a cell
-__device__ __forceinline__ float jb_g(const MGLevel &L, const JbCell &c, float beta) {
-    return jb_div(beta, __builtin_fmaf(L.cell2[1], c.py2, L.cell2[0] * c.px2) + L.cell2[2] * c.pz2);
+constexpr int kFpNormal = 0x108, kFpZero = 0x060;   // classes of v_cmp_class_f32
+// beta / |x|^2 of a cell.  EXACT: with the IEEE division where jb_quot's result
+// does not do; otherwise ok is cleared there.  Zero is fine for beta = 0.
+template <bool EXACT>
+__device__ __forceinline__ float jb_g(const MGLevel &L, const JbCell &c, float beta, bool &ok) {
+    const float r2 = __builtin_fmaf(L.cell2[1], c.py2, L.cell2[0] * c.px2) + L.cell2[2] * c.pz2;
+    const float g = jb_quot(beta, r2);
+    const bool in = __builtin_amdgcn_classf(g, beta == 0.0f ? kFpNormal | kFpZero : kFpNormal);
+    ok = ok && in;
+    return EXACT && !in ? beta / r2 : g;
 }
-// the new value from f, the 18 neighbours (argument order of nbr_of) and the value
-template <int LOS>
-__device__ __forceinline__ float jb_update(const MGLevel &L, const JbCell &c, float g, float omega, float f, float v,
-                                           float vxp, float vxm, float vyp, float vym, float vzp, float vzm, float xpyp,
-                                           float xmym, float xmyp, float xpym, float xpzp, float xmzm, float xmzp,
-                                           float xpzm, float ypzp, float ymzm, float ymzp, float ypzm) {
+// The new value from f, the 18 neighbours (argument order of nbr_of) and the
+// value; EXACT and ok as above (a zero quotient is right: mg_jacobi_tb_ok
+// bounds the diagonal).
+template <int LOS, bool EXACT>
+__device__ __forceinline__ float jb_update(bool &ok, const MGLevel &L, const JbCell &c, float g, float omega, float f,
+                                           float v, float vxp, float vxm, float vyp, float vym, float vzp, float vzm,
+                                           float xpyp, float xmym, float xmyp, float xpym, float xpzp, float xmzm,
+                                           float xmzp, float xpzm, float ypzp, float ymzm, float ymzp, float ypzm) {
     const float gx = __builtin_fmaf(g, c.px2, L.icell2[0]), gy = __builtin_fmaf(g, c.py2, L.icell2[1]);
     const float gz = __builtin_fmaf(g, c.pz2, L.icell2[2]);
     float j = __builtin_fmaf(gx, vxp + vxm, f);
@@ -744,7 +756,10 @@ __device__ __forceinline__ float jb_update(const MGLevel &L, const JbCell &c, fl
     }
     j = __builtin_fmaf(g, t, j);
     // j / (2 (gx + gy + gz)), the 1/2 in the weight
-    return __builtin_fmaf(0.5f * omega, jb_div(j, (gx + gy) + gz), (1.0f - omega) * v);
+    const float D = (gx + gy) + gz, q = jb_quot(j, D), keep = (1.0f - omega) * v;
+    const bool in = __builtin_amdgcn_classf(q, kFpNormal | kFpZero);
+    ok = ok && in;
+    return EXACT && !in ? __builtin_fmaf(omega, j / (2.0f * D), keep) : __builtin_fmaf(0.5f * omega, q, keep);
 }
 
 // S = 1 or 2 damped Jacobi sweeps in one launch, out of place: S = 2 leaves
@@ -865,11 +880,13 @@ __global__ void __launch_bounds__(JbShape<S>::Threads, 3) k_mg_jacobi_zm(float *
     auto pz_of = [&](int P) { return LOS ? L.losn[2] : L.pv[nx + ny + gs_wrap(P, nz)]; };
     // four rows of one level: from the ring planes below, at and above, row
     // pitch W, at word w (row0 of the lane's column); level 1 (FIRST) makes
-    // the coefficients, a later level takes them from the ring
-    auto rows = [&](auto first, auto wpitch, const float *pm, const float *p0, const float *pp, int w, float pz,
-                    int slot, float (&out)[4]) {
+    // the coefficients, a later level takes them from the ring.  False if a
+    // division has to be done again.
+    auto fast_rows = [&](auto first, auto wpitch, const float *pm, const float *p0, const float *pp, int w, float pz,
+                         int slot, float (&out)[4]) __attribute__((always_inline)) {
         constexpr bool FIRST = decltype(first)::value;
         constexpr int W = decltype(wpitch)::value;
+        bool ok = true;
         // two rows at a time (all four rows' values at once cost registers and
         // with them a wave per SIMD); the level's start and end are kept apart
         // from the other level's, whose loads would otherwise be hoisted
@@ -897,14 +914,47 @@ __global__ void __launch_bounds__(JbShape<S>::Threads, 3) k_mg_jacobi_zm(float *
             for (int j = 0; j < 2; j++) {
                 const int jr = h + j;
                 const JbCell c{px, py[jr], pz, px * px, py[jr] * py[jr], pz * pz};
-                const float g = FIRST ? jb_g(L, c, beta) : gr[slot][jr];
+                const float g = FIRST ? jb_g<false>(L, c, beta, ok) : gr[slot][jr];
                 if constexpr (FIRST) gr[slot][jr] = g;
-                out[jr] = jb_update<LOS>(L, c, g, omega, fr[slot][jr], c0[j + 1], r0[j + 1], l0[j + 1], c0[j + 2],
-                                         c0[j], cp[j + 1], cm[j + 1], r0[j + 2], l0[j], l0[j + 2], r0[j], rp[j], lm[j],
-                                         lp[j], rm[j], cp[j + 2], cm[j], cp[j], cm[j + 2]);
+                out[jr] = jb_update<LOS, false>(ok, L, c, g, omega, fr[slot][jr], c0[j + 1], r0[j + 1], l0[j + 1],
+                                                c0[j + 2], c0[j], cp[j + 1], cm[j + 1], r0[j + 2], l0[j], l0[j + 2],
+                                                r0[j], rp[j], lm[j], lp[j], rm[j], cp[j + 2], cm[j], cp[j], cm[j + 2]);
             }
         }
         __builtin_amdgcn_sched_barrier(0);
+        return ok;
+    };
+    // one cell at word w, its divisions checked one by one
+    auto cell = [&](auto first, auto wpitch, const float *pm, const float *p0, const float *pp, int w, float cx, float cy,
+                    float cz, float fv, float &g) __attribute__((always_inline)) {
+        constexpr int W = decltype(wpitch)::value;
+        const JbCell c{cx, cy, cz, cx * cx, cy * cy, cz * cz};
+        bool ok = true;
+        if (decltype(first)::value) g = jb_g<true>(L, c, beta, ok);
+#define A0(q) p0[w + (q)]
+#define AM(q) pm[w + (q)]
+#define AP(q) pp[w + (q)]
+        return jb_update<LOS, true>(ok, L, c, g, omega, fv, A0(0), A0(1), A0(-1), A0(W), A0(-W), AP(0), AM(0),
+                                    A0(W + 1), A0(-W - 1), A0(W - 1), A0(-W + 1), AP(1), AM(-1), AP(-1), AM(1), AP(W),
+                                    AM(-W), AP(-W), AM(W));
+#undef A0
+#undef AM
+#undef AP
+    };
+    // The checks cost a compare per division and a branch per four rows, which
+    // leaves the loop to be scheduled as one piece (a branch per division: 152
+    // us per two-sweep launch of an FMG solve on average, 149 here, 144 unchecked).
+    auto rows = [&](auto first, auto wpitch, const float *pm, const float *p0, const float *pp, int w, float pz,
+                    int slot, float (&out)[4]) __attribute__((always_inline)) {
+        if (__builtin_expect(!fast_rows(first, wpitch, pm, p0, pp, w, pz, slot, out), 0)) {
+#pragma unroll
+            for (int j = 0; j < 4; j++) {
+                float cx = px, cz = pz;
+                asm volatile("" : "+v"(w), "+v"(cx), "+v"(cz));   // keeps no value from above in registers for this
+                out[j] = cell(first, wpitch, pm, p0, pp, w + j * decltype(wpitch)::value, cx, py[j], cz, fr[slot][j],
+                              gr[slot][j]);
+            }
+        }
     };
     using True = std::integral_constant<bool, true>;
     using False = std::integral_constant<bool, false>;
@@ -934,17 +984,9 @@ __global__ void __launch_bounds__(JbShape<S>::Threads, 3) k_mg_jacobi_zm(float *
 #pragma unroll
                 for (int j = 0; j < 4; j++) pl[w1 + j * J::W1] = o[j];
                 if (ex_on) {
-                    const JbCell c{ex_px, ex_py, pz, ex_px * ex_px, ex_py * ex_py, pz * pz};
-#define A0(q) p0[ex_w0 + (q)]
-#define AM(q) pm[ex_w0 + (q)]
-#define AP(q) pp[ex_w0 + (q)]
-                    pl[ex_w1] = jb_update<LOS>(
-                        L, c, jb_g(L, c, beta), omega, exf, A0(0), A0(1), A0(-1), A0(J::W0), A0(-J::W0), AP(0), AM(0),
-                        A0(J::W0 + 1), A0(-J::W0 - 1), A0(J::W0 - 1), A0(-J::W0 + 1), AP(1), AM(-1), AP(-1), AM(1),
-                        AP(J::W0), AM(-J::W0), AP(-J::W0), AM(J::W0));
-#undef A0
-#undef AM
-#undef AP
+                    float g;
+                    pl[ex_w1] = cell(True{}, std::integral_constant<int, J::W0>{}, pm, p0, pp, ex_w0, ex_px, ex_py, pz,
+                                     exf, g);
                 }
             }
         }
@@ -2474,14 +2516,18 @@ static hipError_t jacobi_zm(float *vout, const float *vin, const float *f, const
     return hipGetLastError();
 }
 
-bool mg_jacobi_tb_ok(const MGLevel &L) {
+bool mg_jacobi_tb_ok(const MGLevel &L, float beta) {
+    // the diagonal, at most (1 + |beta|) sum 1 / cell^2, far from the ends of FP32 (jb_update)
+    if (!(fabsf(beta) <= 0x1p20f)) return false;
+    for (int a = 0; a < 3; a++)
+        if (!(L.icell2[a] >= 0x1p-100f && L.icell2[a] <= 0x1p100f)) return false;
     return L.n[0] % kJbTX == 0 && L.n[1] % JbShape<1>::TY == 0 && L.n[2] % 8 == 0 && L.n[2] >= 8 &&
            (int64_t)L.n[0] * L.n[1] * L.n[2] < ((int64_t)1 << 31);
 }
 
 hipError_t launch_mg_jacobi_tb(float *vout, const float *vin, const float *f, const MGLevel &L, float beta,
                                float omega, int has_los, int sweeps, hipStream_t s) {
-    if (!mg_jacobi_tb_ok(L) || vout == vin || (sweeps != 1 && sweeps != 2)) return hipErrorInvalidValue;
+    if (!mg_jacobi_tb_ok(L, beta) || vout == vin || (sweeps != 1 && sweeps != 2)) return hipErrorInvalidValue;
     return sweeps == 1 ? jacobi_zm<1>(vout, vin, f, L, beta, omega, has_los, s)
                        : jacobi_zm<2>(vout, vin, f, L, beta, omega, has_los, s);
 }

@@ -232,3 +232,45 @@ def test_small_levels_fmg_matches_oracle(ctx, shape, sweeps):
     bh.vcycle_(v, f, rec)
     exp = orc.mg_vcycle(f.copy(), f, rec.box_size, rec.box_min, rec.beta, 0.4, sweeps)
     assert np.linalg.norm(v - exp) < 2e-5 * np.linalg.norm(exp)
+
+
+@pytest.mark.parametrize("los", [None, [0.3, -0.4, 0.866]])
+@pytest.mark.parametrize("sweeps", [1, 2])
+def test_zmarching_jacobi_overflows_as_the_oracle(ctx, los, sweeps):
+    """Quotients of finite numbers around the largest float: infinite where
+    the oracle's division is, finite below (also where the quotient by half
+    the diagonal overflows)."""
+    shape = (128, 128, 128)
+    v, f = fields(shape, 19)
+    for i, big in enumerate((3e38, -3e38, 1e38, -1e38, 2e37)):
+        f.flat[(1 + i) * 300007] = big
+    rec = recon(shape, los, ctx)
+    rec.jacobi_niterations = sweeps
+    got = bh.jacobi_(v.copy(), f, rec)
+    with np.errstate(invalid="ignore", over="ignore"):
+        exp = orc.mg_jacobi(v.copy(), f, rec.box_size, rec.box_min, rec.beta, 0.4, sweeps, los=los)
+    assert np.isinf(exp).sum() >= 2 and np.isfinite(exp.flat[3 * 300007])
+    np.testing.assert_array_equal(np.isnan(got), np.isnan(exp))
+    np.testing.assert_array_equal(got == np.inf, exp == np.inf)
+    np.testing.assert_array_equal(got == -np.inf, exp == -np.inf)
+    on = np.isfinite(exp) & (np.abs(exp) > 1e30)
+    assert on.sum() >= 3
+    np.testing.assert_allclose(got[on], exp[on], rtol=5e-7 * sweeps)
+
+
+@pytest.mark.parametrize("sweeps", [1, 2])
+@pytest.mark.parametrize("growth,cell", [(0.0, 4.0), (0.8, 3.1 * 2.0 ** -64), (0.8, 2.0 ** 55), (8e6, 4.0)])
+def test_large_grid_jacobi_over_coefficients(ctx, growth, cell, sweeps):
+    """The sweeps of grids of 128^3 and more without redshift-space distortions
+    (beta = 0), with cells so small that the operator's diagonal passes 2^126,
+    with very large ones and with a very large beta."""
+    shape = (128, 128, 128)
+    v, f = (a * F32(0.01) for a in fields(shape, 20))
+    f *= F32(1.0 / cell) * F32(1.0 / cell)
+    rec = bh.MultigridRecon(bias=2.0, f=growth, smoothing_radius=15.0, box_size=[128 * cell] * 3,
+                            box_min=[50 * cell, -75 * cell, 125 * cell], los=None, ctx=ctx)
+    rec.jacobi_niterations = sweeps
+    got = bh.jacobi_(v.copy(), f, rec)
+    exp = orc.mg_jacobi(v.copy(), f, rec.box_size, rec.box_min, rec.beta, 0.4, sweeps, los=None)
+    assert np.all(np.isfinite(exp))
+    assert np.max(np.abs(got - exp)) < 5e-7 * sweeps * np.abs(exp).max()
