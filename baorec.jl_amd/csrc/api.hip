@@ -60,6 +60,7 @@ struct baorec_ctx {
     // (nx, ny, nz, tsc, floor(log2 n)); strided kernel per (axis, line length)
     std::map<std::array<int64_t, 5>, std::array<int, 3>> tune_tile;
     std::map<std::array<int, 2>, int> tune_pair;
+    std::map<std::array<int, 2>, int> tune_stay;   // the same for passes of several outputs (tables only)
     int force_tile[3] = {0, 0, 0};   // set while tuning
     int force_pair = -1;
     // learned warm start: the network of baorec_warmstart_init / _load
@@ -498,16 +499,21 @@ void tables(baorec_ctx *c, const Grid &G, const Slot *slot, FFTBufs &f) {
 
 void strided(baorec_ctx *c, const Grid &G, const StridedArgs &a0, int njobs, int nbatch, const char *what) {
     StridedArgs a = a0;
-    // kernel choice of single-output passes: being timed, tuned, or the rule
+    // kernel of single-output passes: being timed, tuned, or the rule; of passes
+    // of several outputs: the rule, unless a table says otherwise
+    const std::array<int, 2> key{a.axis, a.axis == 1 ? G.ny : G.nz};
     a.pair = c->force_pair;
     if (a.pair < 0) {
-        auto it = c->tune_pair.find({a.axis, a.axis == 1 ? G.ny : G.nz});
+        auto it = c->tune_pair.find(key);
         if (it != c->tune_pair.end()) a.pair = it->second;
     }
+    auto it = c->tune_stay.find(key);
+    a.stay = it == c->tune_stay.end() ? 1 : it->second;
     double bytes = 0.0;
     for (int j = 0; j < njobs; j++) bytes += 8.0 * G.Cdense() * (1 + a.job[j].nout);
-    const bool pair = strided_uses_pair(a, njobs);
-    ProfScope ps(c, a.axis == 1 ? (pair ? "fft_y_pair" : "fft_y") : (pair ? "fft_z_pair" : "fft_z"), bytes * nbatch);
+    const char *const label[2][3] = {{"fft_y", "fft_y_pair", "fft_y_staying"}, {"fft_z", "fft_z_pair", "fft_z_staying"}};
+    const int kind = strided_uses_pair(a, njobs) ? 1 : (strided_uses_staying(a, njobs) ? 2 : 0);
+    ProfScope ps(c, label[a.axis == 1 ? 0 : 1][kind], bytes * nbatch);
     hipchk(c, launch_strided(a, njobs, nbatch, c->stream), what);
 }
 
@@ -2359,9 +2365,13 @@ static std::string graph_key(const baorec_params *p, const int32_t grid[3], cons
         put(kv.first.data(), sizeof(int64_t) * kv.first.size());
         put(kv.second.data(), sizeof(int) * kv.second.size());
     }
-    for (const auto &kv : c->tune_pair) {
-        put(kv.first.data(), sizeof(int) * kv.first.size());
-        put(&kv.second, sizeof(int));
+    for (const auto *m : {&c->tune_pair, &c->tune_stay}) {
+        const size_t entries = m->size();
+        put(&entries, sizeof entries);
+        for (const auto &kv : *m) {
+            put(kv.first.data(), sizeof(int) * kv.first.size());
+            put(&kv.second, sizeof(int));
+        }
     }
     return k;
 }
@@ -3176,13 +3186,17 @@ int64_t baorec_tune_report(baorec_ctx *c, char *buf, int64_t len) {
     }
     js += "],\n \"strided\": [";
     first = true;
-    for (const auto &e : c->tune_pair) {
-        char line[128];
-        snprintf(line, sizeof line, "%s\n  {\"axis\": %d, \"n\": %d, \"pair\": %d}", first ? "" : ",", e.first[0],
-                 e.first[1], e.second);
-        js += line;
-        first = false;
-    }
+    auto put = [&](const std::map<std::array<int, 2>, int> &m, const char *what) {
+        for (const auto &e : m) {
+            char line[128];
+            snprintf(line, sizeof line, "%s\n  {\"axis\": %d, \"n\": %d, \"%s\": %d}", first ? "" : ",", e.first[0],
+                     e.first[1], what, e.second);
+            js += line;
+            first = false;
+        }
+    };
+    put(c->tune_pair, "pair");
+    put(c->tune_stay, "staying");
     js += "]}\n";
     if (buf && len > 0) {
         strncpy(buf, js.c_str(), (size_t)len - 1);
@@ -3224,7 +3238,7 @@ int baorec_tune_load(baorec_ctx *c, const char *path) {
         return BAOREC_ERR_INVALID_ARGUMENT;
     }
     std::map<std::array<int64_t, 5>, std::array<int, 3>> tiles;
-    std::map<std::array<int, 2>, int> pairs;
+    std::map<std::array<int, 2>, int> pairs, stay;
     char line[512];
     bool bad = false;
     while (fgets(line, sizeof line, fp)) {
@@ -3242,12 +3256,14 @@ int baorec_tune_load(baorec_ctx *c, const char *path) {
                 break;
             }
             tiles[{g0, g1, g2, tsc, l2}] = {t0, t1, t2};
-        } else if (sscanf(s, " {\"axis\": %d, \"n\": %d, \"pair\": %d}", &ax, &nn, &pr) == 3) {
+        } else {
+            const bool single = sscanf(s, " {\"axis\": %d, \"n\": %d, \"pair\": %d}", &ax, &nn, &pr) == 3;
+            if (!single && sscanf(s, " {\"axis\": %d, \"n\": %d, \"staying\": %d}", &ax, &nn, &pr) != 3) continue;
             if ((ax != 1 && ax != 2) || (pr != 0 && pr != 1)) {
                 bad = true;
                 break;
             }
-            pairs[{ax, nn}] = pr;
+            (single ? pairs : stay)[{ax, nn}] = pr;
         }
     }
     fclose(fp);
@@ -3257,6 +3273,7 @@ int baorec_tune_load(baorec_ctx *c, const char *path) {
     }
     for (const auto &e : tiles) c->tune_tile[e.first] = e.second;
     for (const auto &e : pairs) c->tune_pair[e.first] = e.second;
+    for (const auto &e : stay) c->tune_stay[e.first] = e.second;
     return BAOREC_OK;
 }
 

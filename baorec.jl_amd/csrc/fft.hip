@@ -1104,6 +1104,21 @@ bool strided_uses_pair(const StridedArgs &a, int njobs) {
     return M >= 256 && M <= 1024 && single;
 }
 
+// The most outputs of a job of k_strided_n's instance for this pass, 0 if
+// there is none.
+static int staying_nout(const StridedArgs &a, int njobs) {
+    int nout = 0;
+    for (int j = 0; j < njobs; j++) nout = std::max(nout, a.job[j].nout);
+    const bool two = a.mode == 1 || (a.mode == 2 && (a.mul == MUL_I_INVK2 || a.mul == MUL_I));
+    const bool three = a.mode == 2 && a.mul == MUL_INVK2;
+    return (nout == 2 && two) || (nout == 3 && three) ? nout : 0;
+}
+
+bool strided_uses_staying(const StridedArgs &a, int njobs) {
+    const int M = a.axis == 1 ? a.ny : a.nz;
+    return a.stay != 0 && (M == 256 || M == 512) && a.Pv <= kStridedNPv && staying_nout(a, njobs) > 0;
+}
+
 template <int M>
 static hipError_t strided_m(const StridedArgs &a, int njobs, int nbatch, hipStream_t s) {
     using S = SShape<M>;
@@ -1125,17 +1140,12 @@ static hipError_t strided_m(const StridedArgs &a, int njobs, int nbatch, hipStre
     }
     const int ncg = (a.Pv + S::B - 1) / S::B;
     if constexpr (M == 256 || M == 512) {
-        int nout = 0;
-        for (int j = 0; j < njobs; j++) nout = std::max(nout, a.job[j].nout);
-        using K = decltype(&k_strided_n<M, 1, MUL_NONE, 2>);
-        K kernel = nullptr;
-        if (a.pair != 0 && a.Pv <= kStridedNPv) {   // (pair = 0: k_strided for every pass of the axis)
-            if (a.mode == 1 && nout == 2) kernel = k_strided_n<M, 1, MUL_NONE, 2>;
-            if (a.mode == 2 && nout == 2 && a.mul == MUL_I_INVK2) kernel = k_strided_n<M, 2, MUL_I_INVK2, 2>;
-            if (a.mode == 2 && nout == 2 && a.mul == MUL_I) kernel = k_strided_n<M, 2, MUL_I, 2>;
-            if (a.mode == 2 && nout == 3 && a.mul == MUL_INVK2) kernel = k_strided_n<M, 2, MUL_INVK2, 3>;
-        }
-        if (kernel) {
+        if (strided_uses_staying(a, njobs)) {
+            using K = decltype(&k_strided_n<M, 1, MUL_NONE, 2>);
+            const K kernel = a.mode == 1               ? k_strided_n<M, 1, MUL_NONE, 2>
+                             : a.mul == MUL_INVK2       ? k_strided_n<M, 2, MUL_INVK2, 3>
+                             : a.mul == MUL_I_INVK2     ? k_strided_n<M, 2, MUL_I_INVK2, 2>
+                                                        : k_strided_n<M, 2, MUL_I, 2>;
             // 16 waves per CU over all jobs and batch items
             const int nt = (a.Pv + 15) / 16 * nother;
             dim3 grid(stay_grid(nt, 256 * 512 / M, njobs * nbatch), njobs, nbatch);

@@ -51,9 +51,9 @@ struct StridedArgs {
     int mul;                   // MulKind (mode 2)
     float R2;                  // smoothing radius squared (FP32)
     float los[3];
-    int pair;                  // kernel: -1 the library's rule, 0 k_strided (one column per
-                               // thread) for every job, 1 as -1 with two columns per
-                               // thread for single-output jobs
+    int pair;                  // kernel of single-output jobs: -1 the library's rule, 0 one
+                               // column per thread, 1 two columns per thread
+    int stay;                  // kernel of jobs of several outputs: 0 always k_strided, else the rule
     // MUL_MG_INV: symbol sum_a gp[a] (2 - 2 cos t_a) + sum_{a<b} cross[ab]
     // sin t_a sin t_b with t_a = k_a cell[a] (cross: xy, xz, yz)
     float mg_gp[3], mg_cross[3], mg_cell[3];
@@ -142,6 +142,7 @@ hipError_t launch_strided(const StridedArgs &a, int njobs, int nbatch, hipStream
 // True when launch_strided runs the pass with two columns per thread
 // (k_strided2: lines of 256..1024, every job with one output).
 bool strided_uses_pair(const StridedArgs &a, int njobs);
+bool strided_uses_staying(const StridedArgs &a, int njobs);
 bool fft_side_ok(int n);
 
 // ---------------------------------------------------------------- tables

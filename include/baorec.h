@@ -488,7 +488,7 @@ int baorec_run_batch(baorec_ctx *ctx, baorec_params *p, const int32_t grid[3],
  *    assignment and catalog size class (floor(log2 n));
  *  - per FFT line length >= 256 and axis, the kernel of single-output strided
  *    passes (one or two columns per thread).
- * The transforms are identical for every choice; the density grids agree
+ * The two kernels of the transforms round differently; the density grids agree
  * to the fixed-point quantum of the scatter (2^-61 of a tile's total weight,
  * in practice bitwise).  Needs box_size and box_min in params; the inputs
  * are not modified.
@@ -499,7 +499,10 @@ int baorec_autotune(baorec_ctx *ctx, const baorec_params *p, const int32_t grid[
  * the terminating NUL. */
 int64_t baorec_tune_report(baorec_ctx *ctx, char *buf, int64_t len);
 /* Writes the tuned choices to a JSON file / adds those of a file written by
- * baorec_tune_save (entries the library cannot use are rejected). */
+ * baorec_tune_save (entries the library cannot use are rejected).  A file may
+ * also hold {"axis": a, "n": n, "staying": 0}: passes of several outputs of
+ * that axis and length by the general kernel instead of the one whose
+ * workgroups stay (for comparing the two; nothing tunes it). */
 int baorec_tune_save(baorec_ctx *ctx, const char *path);
 int baorec_tune_load(baorec_ctx *ctx, const char *path);
 
