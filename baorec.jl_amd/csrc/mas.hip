@@ -517,8 +517,12 @@ __global__ void __launch_bounds__(kAccumThreads) k_scatter_accum(ScatterArgs a, 
 constexpr int kSortThreads = 1024;
 // Particles per block, at least: small blocks fill the GPU for small catalogs
 // (20000 particles in 32 tiles: histogram and place pass 6.4 + 5.2 us at 1024,
-// 12.4 + 11.4 at 8192), but every block costs a row of tile counts, so a
-// single catalog's have at least half as many particles as there are tiles.
+// 12.4 + 11.4 at 8192), but every block costs a row of T tile counts.  A single
+// catalog's blocks have T / 2 particles between the two bounds; above 8192
+// tiles the row costs less than idle CUs (16384 tiles, sum of the three passes
+// at 4096 / 8192: 200000 particles 31 / 41 us, 1 million 49 / 53, 3 million 122
+// / 126).  Several catalogs together need no smaller blocks than 4096 to fill
+// the GPU (four of 100000 in 16384 tiles 37 / 46 us, of 500000 92 / 80).
 constexpr int kSortBlockMin = 4096, kSortBlockMin1 = 1024;
 constexpr int kSortMaxBlocks = 512;        // two 64 KB-histogram blocks per CU on 256 CUs
 constexpr int kSortMaxTiles = 16384;        // LDS histogram capacity (64 KB)
@@ -755,8 +759,8 @@ __global__ void k_add_count(uint32_t *cursor, const uint32_t *count, int64_t n) 
     if (i < n) cursor[i] += count[i];
 }
 
-// Blocks of a single catalog on T tiles: equal ranges of at least
-// kSortBlockMin1 .. kSortBlockMin particles, at most kSortMaxBlocks (one wave
+// Blocks of a single catalog on T tiles: equal ranges of at least T / 2
+// particles (kSortBlockMin1 .. kSortBlockMin), at most kSortMaxBlocks (one wave
 // of blocks, no ragged tail).
 int sort_nblk(int64_t n, int T) {
     const int least = std::min(std::max(T / 2, kSortBlockMin1), kSortBlockMin);
