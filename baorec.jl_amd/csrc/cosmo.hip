@@ -241,13 +241,19 @@ __device__ __forceinline__ void sincos_f32(float xf, double &s, double &c) {
     c = (q + 1) & 2 ? -b : b;
 }
 
-// atan2 in FP64 of finite FP32 arguments.  With a = min, b = max of the
+// atan2 in FP64 of FP32 arguments.  With a = min, b = max of the
 // magnitudes, atan(a / b) = pi/4 + atan((a - b) / (a + b)) beyond tan(pi/8),
 // so one division and |u| <= tan(pi/8); atan(u) / u is a polynomial of degree
 // 11 in u^2, the Chebyshev fit on that interval (1.3e-18), below the rounding of
-// its evaluation.  Signs, zeros and quadrants as atan2's.
+// its evaluation.  Signs, zeros, infinities, NaN and quadrants as atan2's.
 __device__ __forceinline__ double atan2_f32(float yf, float xf) {
-    const double y = fabs((double)yf), x = fabs((double)xf);
+    double y = fabs((double)yf), x = fabs((double)xf);
+    const double sum = x + y;
+    if (__builtin_expect(!(sum < HUGE_VAL), 0)) {   // infinities: the angle of their directions
+        if (sum != sum) return sum;
+        x = x < HUGE_VAL ? 0.0 : 1.0;
+        y = y < HUGE_VAL ? 0.0 : 1.0;
+    }
     const double a = fmin(x, y), b = fmax(x, y);
     const bool far = a > 0.41421356237309503 * b;
     const double n = far ? a - b : a, d = far ? a + b : b;

@@ -5,6 +5,8 @@ displacements and shifted positions within 1e-4 Mpc/h RMS.  Primitives that
 are pure FP32 arithmetic in the reference's order (scatter, gather, Jacobi,
 residual, restriction, prolongation) are held to tighter bounds.
 """
+import ctypes
+
 import numpy as np
 import pytest
 
@@ -963,3 +965,28 @@ def test_small_levels_fmg_in_any_unit_of_length(ctx, los):
         out.append(bh.fmg(f * F32(scale), rec).astype(np.float64) / (scale * u * u))
     assert np.all(np.isfinite(out[1]))
     assert rel_l2(out[1], out[0]) < 1e-6
+
+
+def test_cartesian_to_sky_angles_of_rejected_positions(ctx):
+    """Positions without a redshift in the table raise; the C entry still leaves
+    every galaxy's angles, those of infinite and NaN coordinates as atan2's,
+    and NaN for its redshift."""
+    inf, nan = np.inf, np.nan
+    pos = np.array([(700, -300, 200), (nan, 1, 1), (1, nan, 1), (1, 1, nan), (inf, 2, 3), (-inf, 2, 3), (2, inf, 3),
+                    (2, -inf, 3), (2, 3, inf), (2, 3, -inf), (inf, -inf, 1), (-inf, -inf, inf), (inf, 1, -inf),
+                    (-3e38, 2e38, 1e38), (1e5, 0, 0)], F32)
+    x, y, z = (np.ascontiguousarray(pos[:, a]) for a in range(3))
+    out = [np.zeros(len(pos), F32) for _ in range(3)]
+    c = bh.Cosmology(z_tab_num=1001).struct()
+    p = [v.ctypes.data_as(ctypes.c_void_p) for v in (x, y, z, *out)]
+    with pytest.raises(bh.BoundsError):
+        ctx.check(ctx.lib.baorec_cartesian_to_sky(ctx.handle, ctypes.byref(c), 0, *p[:3], len(pos), *p[3:]))
+    with np.errstate(invalid="ignore", over="ignore"):
+        s = np.sqrt(x * x + y * y)
+        pi = F32(np.pi)
+        lon = np.arctan2(y.astype(np.float64), x.astype(np.float64)).astype(F32) * F32(180) / pi
+        lat = np.arctan2(z.astype(np.float64), s.astype(np.float64)).astype(F32) * F32(180) / pi
+        ra = np.fmod(lon - F32(360), F32(360))
+    np.testing.assert_allclose(out[0], ra, rtol=2.0 ** -23, atol=0)
+    np.testing.assert_allclose(out[1], lat, rtol=2.0 ** -23, atol=0)
+    assert np.isfinite(out[2][0]) and np.all(np.isnan(out[2][1:]))
