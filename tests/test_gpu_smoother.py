@@ -63,6 +63,11 @@ def test_fused_sweep_rejects_unsupported_shape(ctx):
     bh.gauss_seidel_(v, f, recon(shape, None, ctx), fused=False)
 
 
+# One sweep per call is a z-marching launch of its own on these grids: this test
+# holds the two-sweep launches against the one-sweep ones, which share their
+# arithmetic (launches are of two sweeps and one, not of three and two as the
+# docstring has it).  The comparison with an independent sweep is
+# test_zmarching_jacobi_error_against_fp64's.
 @pytest.mark.parametrize("shape,los,sweeps", [
     ((128, 128, 128), None, 5),
     ((128, 128, 128), [0.0, 0.0, 1.0], 3),
@@ -274,3 +279,67 @@ def test_large_grid_jacobi_over_coefficients(ctx, growth, cell, sweeps):
     exp = orc.mg_jacobi(v.copy(), f, rec.box_size, rec.box_min, rec.beta, 0.4, sweeps, los=None)
     assert np.all(np.isfinite(exp))
     assert np.max(np.abs(got - exp)) < 5e-7 * sweeps * np.abs(exp).max()
+
+
+def fp64_sweep(v, f, box_size, box_min, beta, omega, los):
+    """One damped Jacobi sweep (jacobi!, src/multigrid.jl:14-135) in FP64 from
+    the FP32 cell centres, and a bound of an FP32 sweep's rounding per cell in
+    units of 2^-24: the summed magnitude of the update's terms times the most
+    roundings that one of them passes (6 in a coefficient, 2 in a difference,
+    7 in the sum), 8 of the diagonal, 2 of the quotient and its weight, 3 of
+    the part that is kept."""
+    h = [float(F32(F32(L) / F32(n))) for L, n in zip(box_size, v.shape[::-1])]
+    if los is None:
+        p = [x / F32(c) for x, c in zip(orc.x_vec(v.shape[::-1], box_size, box_min), h)]
+        p = [p[0][None, None, :], p[1][None, :, None], p[2][:, None, None]]
+    else:
+        p = [F32(w) / F32(c) for w, c in zip(los, h)]
+    px, py, pz = (np.asarray(a, np.float64) for a in p)
+
+    def at(dx, dy, dz):
+        return np.roll(v, (-dz, -dy, -dx), (0, 1, 2))
+    g = beta / ((h[0] * px) ** 2 + (h[1] * py) ** 2 + (h[2] * pz) ** 2)
+    total, size, diag = f.copy(), np.abs(f), 0.0
+    for a, (e, q) in enumerate(zip(np.eye(3, dtype=int), (px, py, pz))):
+        w, up, dn = 1 / h[a] ** 2 + g * q * q, at(*e), at(*-e)
+        total += w * (up + dn)
+        size += w * (np.abs(up) + np.abs(dn))
+        diag = diag + w
+        if los is None:
+            total += g * q * (up - dn)
+            size += np.abs(g * q) * (np.abs(up) + np.abs(dn))
+    for i, j, w in ((0, 1, px * py), (0, 2, px * pz), (1, 2, py * pz)):
+        e, k = np.eye(3, dtype=int)[i], np.eye(3, dtype=int)[j]
+        t = [at(*(e + k)), at(*(-e - k)), at(*(k - e)), at(*(e - k))]
+        total += g / 2 * w * (t[0] + t[1] - t[2] - t[3])
+        size += np.abs(g / 2 * w) * sum(np.abs(s) for s in t)
+    q = total / (2 * diag)
+    return (1 - omega) * v + omega * q, omega * 25 * size / (2 * diag) + 3 * np.abs(v)
+
+
+@pytest.mark.parametrize("shape,los", [((128, 128, 128), None), ((64, 128, 256), None),
+                                       ((128, 128, 128), [0.3, -0.4, 0.866])])
+@pytest.mark.parametrize("sweeps", [1, 2])
+def test_zmarching_jacobi_error_against_fp64(ctx, shape, los, sweeps):
+    """What the one- and two-sweep launches' fused sums and corrected quotients
+    cost in accuracy: nothing against the reference's order of operations in
+    FP32 (the oracle's sweeps on the same fields).  Their rms error against
+    FP64 sweeps is no larger (2 % for the scatter of the largest roundings),
+    and after one sweep every cell is within its rounding bound."""
+    v, f = fields(shape, 23)
+    v *= F32(50.0)
+    rec = recon(shape, los, ctx)
+    rec.jacobi_niterations = sweeps
+    beta, omega = float(F32(rec.beta)), float(F32(0.4))
+    exact = v.astype(np.float64)
+    for _ in range(sweeps):
+        exact, bound = fp64_sweep(exact, f.astype(np.float64), rec.box_size, rec.box_min, beta, omega, los)
+    got = bh.jacobi_(v.copy(), f, rec) - exact
+    ref = orc.mg_jacobi(v.copy(), f, rec.box_size, rec.box_min, rec.beta, 0.4, sweeps, los=los) - exact
+    rms = [float(np.sqrt(np.mean(e * e) / np.mean(exact * exact))) for e in (got, ref)]
+    worst = float(np.max(np.abs(got) / bound)) * 2.0 ** 24
+    print(f"{shape} los {los} x{sweeps}: rms error {rms[0]:.2e}, the reference's order {rms[1]:.2e}, "
+          f"largest / bound {worst:.2f}")
+    assert rms[0] <= 1.02 * rms[1]
+    if sweeps == 1:
+        assert worst <= 1.0
