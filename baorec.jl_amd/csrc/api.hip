@@ -910,13 +910,18 @@ double *votherd(MGPyr &P, int l) { return P.cur[l] ? P.Ad[l] : P.Bd[l]; }
 // n damped Jacobi sweeps (jacobi!, src/multigrid.jl:193-210) ping-ponging
 // between a (the input) and b; returns the one holding the result.  On
 // grids of at least 128^3 cells whose sides are multiples of 64, 16 and 8,
-// sweeps run two per z-marching launch, and an odd one as such a launch of
-// its own (the same bits either way).
+// z-marching launches of one or two sweeps (the same bits either way).  Two
+// save a pass over memory and a launch, but repeat the halo's updates.  Where
+// the three arrays fit the 256 MB Infinity Cache a pass is cheap, and from 2^23
+// cells a launch is no matter: one sweep.  us per sweep by two / by one: 2^21
+// cells 12.7 / 13.2, 2^22 15.6 / 16.8, 4.9 million 17.3 / 17.8; 2^23 24.6 /
+// 23.2, 2^24 44.0 / 38.8; 33 million 84.6 / 87.3, 2^26 159 / 174, 2^27 306 / 342.
 static float *jacobi_sweeps(baorec_ctx *c, const MGLevel &L, int64_t R, float *a, float *b, const float *f,
                             const baorec_params *p, int n) {
     const bool tb = mg_jacobi_tb_ok(L, p->beta) && R >= ((int64_t)1 << 21);
+    const bool two = tb && (R < ((int64_t)1 << 23) || 12 * R > (int64_t)256 << 20);
     for (int left = n; left > 0;) {
-        const int k = tb && left >= 2 ? 2 : 1;
+        const int k = two && left >= 2 ? 2 : 1;
         ProfScope ps(c, k == 1 ? "mg_jacobi" : "mg_jacobi_tb", 12.0 * R);
         if (!tb)
             hipchk(c, launch_mg_jacobi(b, a, f, L, p->beta, p->jacobi_damping_factor, p->has_los, c->stream),

@@ -343,3 +343,22 @@ def test_zmarching_jacobi_error_against_fp64(ctx, shape, los, sweeps):
     assert rms[0] <= 1.02 * rms[1]
     if sweeps == 1:
         assert worst <= 1.0
+
+
+@pytest.mark.parametrize("shape,sweeps", [((120, 256, 256), 3), ((128, 256, 256), 2), ((280, 256, 320), 3)])
+def test_zmarching_jacobi_over_launch_sizes(ctx, shape, sweeps):
+    """Several sweeps in one call (by two or by one per launch, as the grid's
+    size has it: just below and at 2^23 cells, and above the size of the
+    Infinity Cache) and one call per sweep: the same bits; one against the
+    oracle as above."""
+    v, f = fields(shape, 29)
+    rec = recon(shape, None, ctx)
+    rec.jacobi_niterations = sweeps
+    got = bh.jacobi_(v.copy(), f, rec)
+    rec.jacobi_niterations = 1
+    exp = bh.jacobi_(v.copy(), f, rec)
+    ref = orc.mg_jacobi(v.copy(), f, rec.box_size, rec.box_min, rec.beta, 0.4, 1)
+    assert np.max(np.abs(exp - ref)) < 5e-7 * np.abs(ref).max()
+    for _ in range(sweeps - 1):
+        bh.jacobi_(exp, f, rec)
+    np.testing.assert_array_equal(got, exp)
