@@ -1732,12 +1732,13 @@ __global__ void __launch_bounds__(1024) k_mg_coarse(MGCoarse<T> a) {
 // 1024-thread workgroup that keeps them in LDS: one V-cycle from the top one
 // (gs: four-colour Gauss-Seidel, FP32 and FP64 levels mixed; else damped
 // Jacobi, FP32) or the whole FMG (fmg), the per-cell arithmetic and the order
-// of k_mg_coarse.  These levels are bound by latency: through k_mg_coarse every
+// of k_mg_coarse except on a coarsest FP64 level of at most 64 cells
+// (small_gs_wave, a.cop).  These levels are bound by latency: through k_mg_coarse every
 // stage is a round trip to the L2 and levels above 512 cells a launch per
 // stage.  Every address is an index into `pool` from masked coordinates; the
 // host checks that the levels' arrays fit (mg_small_layout).  What remains is
 // a barrier per colour pass and stage.  Measured for 16^3 (FP32) | 8^3 | 4^3
-// (FP64): 48 us per V-cycle (71 with the coarsest level's 256 colour passes
+// (FP64): 49 us per V-cycle (71 with the coarsest level's 256 colour passes
 // instead of a.cop), against 138 us in k_mg_coarse for the lower two alone and
 // eight launches for 16^3; the Jacobi levels 16^3 .. 4^3 of a reference
 // V-cycle 58 us.
@@ -1803,20 +1804,22 @@ struct SmallNbr {
 template <typename T>
 struct SmallCell {
     GsCoef<T> k;
-    T rD;   // reciprocal of the diagonal (FP32: mg_div's v_rcp_f32)
+    T D;   // the diagonal (FP32: mg_div's reciprocal of it)
     int me;
     __device__ __forceinline__ void set(const LdsLevel<T> &l, const MGLevel &L, const SmallNbr &o, int x, int y, int z,
                                         float beta, int has_los) {
         k = small_gs_coef<T>(l, L, x, y, z, beta, has_los);
-        rD = mg_div<T, true>((T)1, (T)2 * ((k.gx + k.gy) + k.gz));
+        D = (T)2 * ((k.gx + k.gy) + k.gz);
+        if constexpr (std::is_same<T, float>::value) D = mg_div<T, true>(1.0f, D);
         me = o.x + o.y + o.z;
     }
-    // gs_update without its division
+    // gs_update, the FP32 reciprocal kept
     __device__ __forceinline__ T update(T f, T vxp, T vxm, T vyp, T vym, T vzp, T vzm, T xpyp, T xmym, T xmyp, T xpym,
                                         T xpzp, T xmzm, T xmzp, T xpzm, T ypzp, T ymzm, T ymzp, T ypzm,
                                         int has_los) const {
-        return gs_sum<T>(k, f, vxp, vxm, vyp, vym, vzp, vzm, xpyp, xmym, xmyp, xpym, xpzp, xmzm, xmzp, xpzm, ypzp, ymzm,
-                         ymzp, ypzm, has_los) * rD;
+        const T j = gs_sum<T>(k, f, vxp, vxm, vyp, vym, vzp, vzm, xpyp, xmym, xmyp, xpym, xpzp, xmzm, xmzp, xpzm, ypzp,
+                              ymzm, ymzp, ypzm, has_los);
+        return std::is_same<T, float>::value ? j * D : j / D;
     }
 };
 
@@ -1899,7 +1902,12 @@ __device__ __forceinline__ double quad_swap(double a) {
 // after): one wave, four lanes per cell of the current colour.  The update is
 // linear, v = f / D + sum_k w_k v_k; lane q of a cell's quad keeps the weights
 // and offsets of neighbours q, q + 4, .. for its cell of each colour, and the
-// quad's partial sums meet by two cross-lane adds.
+// quad's partial sums meet by two cross-lane adds.  Other roundings than the
+// division by D: 64 sweeps of a 4^3 level from zero, emulated against 80-bit
+// floats over twelve operators, leave a relative error of 0.3e-15 to 2.9e-15,
+// 1.7 times the division's, and as a matrix (a.cop) 1.1e-15 to 3.4e-15, 2.7
+// times: FP64 rounding of a correction that the level above adds in FP32 or
+// smooths again.
 __device__ __forceinline__ void small_gs_wave(const LdsLevel<double> &l, const MGLevel &L, int sweeps, float beta,
                                               int has_los) {
     if (threadIdx.x < 64) {
