@@ -1003,7 +1003,8 @@ k_y_iter(YIterArgs a) {
 // ------------------------------------------------------------ launchers
 
 // Workgroups (a multiple of the 8 XCDs) of a kernel whose workgroups walk over
-// nt tiles of each of n jobs, `slots` of them at a time on the GPU.
+// nt tiles of each of n jobs, `slots` of them at a time on the GPU (gfx950's 256
+// CUs times the workgroups of a CU; with fewer CUs the rest wait for their turn).
 static unsigned stay_grid(int nt, int slots, int n) {
     const int per = std::min(std::max(slots / n, 64), nt + 7) & ~7;
     return (unsigned)per;
@@ -1114,6 +1115,9 @@ static int staying_nout(const StridedArgs &a, int njobs) {
     return (nout == 2 && two) || (nout == 3 && three) ? nout : 0;
 }
 
+// 1024 lines of 16 columns would need 2048 threads.  Below 256 the gain does
+// not pay for eight more instances: 128^3, three outputs 14.7 us, two 13.1, and
+// 14.9 on average by k_strided; at 256^3 65 and 82, at 512^3 below.
 bool strided_uses_staying(const StridedArgs &a, int njobs) {
     const int M = a.axis == 1 ? a.ny : a.nz;
     return a.stay != 0 && (M == 256 || M == 512) && a.Pv <= kStridedNPv && staying_nout(a, njobs) > 0;

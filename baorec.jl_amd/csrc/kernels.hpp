@@ -251,15 +251,18 @@ struct CosmoArgs {
     double omega_nu0, omega_g0, omega_b0, omega_c0, omega_k0, omega_l0;
     double w0, wa, h100;
 };
-// Comoving-distance table: num knots zk (increasing, uniform) and distances
-// rk (Mpc, increasing).  Interval lookup: direct index on the uniform z knots;
-// for r, guide[j] = last knot with rk <= r0 + j / dr_inv (nguide entries).
+// Comoving-distance table: num knots (z, r) side by side, z increasing and
+// uniform, r (Mpc) increasing.  Interval lookup: direct index on the uniform z
+// knots; for r, guide[j] = (index, with its fraction between knots, of the
+// distance r0 + j / dr_inv; its change over one step), interpolated linearly.
+// Either is a guess, too low or too high by some knots, from which the look-up
+// walks in both directions (Interp::get).
 constexpr int kCosmoGuide = 1024;
 struct CosmoTable {
     const double2 *kn;   // knots (z, r)
     int num;
     double z0, dz_inv;
-    const float2 *guide;   // kCosmoGuide entries: guess of the knot of r
+    const float2 *guide;   // kCosmoGuide entries
     double r0, dr_inv;
 };
 hipError_t launch_cosmo_guide(const CosmoTable &t, float2 *guide, hipStream_t s);
@@ -364,7 +367,10 @@ template <typename T>
 hipError_t launch_mg_rbgs(T *v, const T *f, const MGLevel &L, float beta, int has_los, int color,
                           hipStream_t s);
 // 1 or 2 damped Jacobi sweeps in one z-marching launch, out of place (vout !=
-// vin), bitwise that many launch_mg_jacobi calls; sides multiples of 64, 16, 8.
+// vin); 2 are bitwise two launches of 1.  They differ from launch_mg_jacobi by
+// rounding (fused sums and corrected quotients; no larger an error against
+// FP64).  Sides multiples of 64, 16, 8; cell sizes and beta within what
+// mg_jacobi_tb_ok allows.
 bool mg_jacobi_tb_ok(const MGLevel &L, float beta);
 hipError_t launch_mg_jacobi_tb(float *vout, const float *vin, const float *f, const MGLevel &L, float beta,
                                float omega, int has_los, int sweeps, hipStream_t s);

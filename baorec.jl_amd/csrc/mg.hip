@@ -1,8 +1,9 @@
 // Multigrid kernels for gfx950: the anisotropic 19-point operator of
 // src/multigrid.jl (damped Jacobi, residual, 27-point restriction, trilinear
 // prolongation) and the multicolour Gauss-Seidel smoother of the RBGS
-// schedule.  The FP32 kernels keep the reference's operation order; the
-// templated ones also run FP64 coarse levels.
+// schedule.  The FP32 kernels keep the reference's operation order, except the
+// z-marching damped Jacobi of large grids (jb_update) and the smoother of the
+// RBGS schedule; the templated ones also run FP64 coarse levels.
 #include <math.h>
 
 #include <type_traits>
@@ -19,8 +20,8 @@ struct Coef {
 // Reciprocal for the Gauss-Seidel smoother's FP32 arithmetic: v_rcp_f32
 // (1 ulp) instead of an IEEE division.  The smoother only approximates the
 // solve inside the FP64-refined iteration, so its rounding does not reach
-// the converged potential; the reference-ordered kernels (Jacobi, residual)
-// keep IEEE divisions.
+// the converged potential; the reference-ordered kernels (Jacobi below 128^3,
+// residual) keep IEEE divisions.
 template <typename T, bool FAST>
 __device__ __forceinline__ T mg_div(T a, T b) {
     if constexpr (FAST && std::is_same<T, float>::value) return a * __builtin_amdgcn_rcpf(b);

@@ -223,7 +223,7 @@ def kernel_symbol(label, grid, rand):
             "gather": "k_gather", "mg_jacobi": "k_mg_jacobi", "mg_residual": "k_mg_residual<float>",
             "mg_reduce": "k_mg_reduce<float, float>", "mg_prolong": "k_mg_prolong<float, float>",
             "mg_mcgs": "k_mg_mcgs<float>", "mg_mcgs64": "k_mg_mcgs<double>", "mg_gs4": "k_mg_gs4",
-            "mg_refine": "k_mg_refine", "mg_residual_fp64": "k_mg_residual_mixed", "mg_jacobi_tb": "k_mg_jacobi_tb",
+            "mg_refine": "k_mg_refine", "mg_residual_fp64": "k_mg_residual_mixed", "mg_jacobi_zm": "k_mg_jacobi_zm",
             "mg_correct": "k_add_correction<double>",
             "mg_coarse": "k_mg_coarse<float>", "mg_coarse64": "k_mg_coarse<double>"}.get(label)
 

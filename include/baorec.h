@@ -370,8 +370,8 @@ int baorec_sky_to_cartesian(baorec_ctx *ctx, const baorec_cosmology *c, int mem,
  * conversion and results as baorec_sky_to_cartesian with mem =
  * BAOREC_MEM_DEVICE: ra, dec, red, x, y, z are device pointers on the
  * context's GPU, and the call makes no hipMalloc, hipFree or other allocating
- * call.  Its distance table (zk, rk, interval integrals, guide) and error flag
- * live in a static device array of 3.67 MB that each GPU the library runs on
+ * call.  Its distance table (knots, interval integrals, guide) and error flag
+ * live in a static device array of 3.15 MB that each GPU the library runs on
  * holds until the process ends; z_tab_num is therefore limited to 131072
  * knots (more returns BAOREC_ERR_UNSUPPORTED).  The table is kept between
  * calls and rebuilt when the cosmology changes.  All calls in a process share
