@@ -498,7 +498,7 @@ __device__ __forceinline__ float2 apply_mul(float2 F, float kx, float ky, float 
         }
         // IEEE quotients: any k^2 that is not zero (boxes in any unit of length) and
         // an overflow to infinity come out as they should.  The divisions cost the
-        // 512^3 passes 2% (606 us; 596 with a shared reciprocal and corrected
+        // 512^3 passes 2% (606 us, 596 with a shared reciprocal and corrected
         // quotients, which lose k^2 above 2^126 and give NaN for an overflow).
         case MUL_INVK2:
             return k2 > 0.f ? make_float2(F.x / k2, F.y / k2) : make_float2(0.f, 0.f);
@@ -720,8 +720,8 @@ constexpr int kStridedNPv = 513;   // kx columns k_strided_n holds
 // and the k tables stand in LDS for all tiles, and no load waits behind a store
 // (they complete in order).  Columns past Pv (inside the row pitch) are
 // transformed and stored like the others; nothing reads them.  NOUT: the most
-// outputs of a job.  The iteration's z pass (2.15 GB at 512^3): 585 us, 716
-// by k_strided; 65 and 82 at 256^3.
+// outputs of a job.  The iteration's z pass (2.15 GB at 512^3): 610 us, 716
+// by k_strided; 66 and 82 at 256^3.
 template <int M, int MODE, int MK, int NOUT>
 __global__ void __launch_bounds__(2 * M) __attribute__((amdgpu_waves_per_eu(4)))
 k_strided_n(StridedArgs a) {
@@ -838,7 +838,7 @@ struct YShape {
 // (inside the row pitch) are transformed and stored like the others; nothing
 // reads them.  512^3: 748 us (1016 with 8 columns per workgroup of one tile
 // that read each input before each transform, 832 with the inputs through
-// LDS), 256^3: 98 (132).
+// LDS), 256^3: 97 (132).
 template <int M>
 __global__ void __launch_bounds__(YShape<M>::NT) __attribute__((amdgpu_waves_per_eu(4)))
 k_y_iter(YIterArgs a) {
@@ -1117,7 +1117,7 @@ static int staying_nout(const StridedArgs &a, int njobs) {
 
 // 1024 lines of 16 columns would need 2048 threads.  Below 256 the gain does
 // not pay for eight more instances: 128^3, three outputs 14.7 us, two 13.1, and
-// 14.9 on average by k_strided; at 256^3 65 and 82, at 512^3 below.
+// 14.9 on average by k_strided.  512^3 610 and 716 us, 256^3 66 and 82.
 bool strided_uses_staying(const StridedArgs &a, int njobs) {
     const int M = a.axis == 1 ? a.ny : a.nz;
     return a.stay != 0 && (M == 256 || M == 512) && a.Pv <= kStridedNPv && staying_nout(a, njobs) > 0;

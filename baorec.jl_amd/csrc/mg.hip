@@ -782,11 +782,11 @@ __device__ __forceinline__ float jb_update(bool &ok, const MGLevel &L, const JbC
 // 64) are one extra cell per lane.  Three waves per SIMD, 168 VGPRs: with the
 // reciprocals kept as well it spilled (401 against 324 us per sweep), and tiles
 // of 32 rows, one workgroup per CU, ran 376-430 us.
-// Per sweep, local LOS, 512^3 / 256^3 / 128^3: 306 / 45 / 12 us (one sweep per
-// pass 341 / 40 / 12, at the copy rate); with the reference's
-// order of operations 347 / 53 / 13 us; with two IEEE
-// divisions per update and cells dealt to the threads level by level, 2 or 3
-// sweeps per launch, 560 / 73 / 14 us.
+// Per sweep, local LOS, 512^3 / 256^3 / 128^3: 306 / 44 / 12.7 us (one sweep per
+// pass 342 / 38.8 / 13.2, at the copy rate); with the reference's order of
+// operations by two 347 / 53 / 13 us; with two IEEE divisions per update and
+// cells dealt to the threads level by level, 2 or 3 sweeps per launch, 560 / 73
+// / 14 us.
 constexpr int kJbTX = 64, kJbRing = 4, kJbMaxTz = 128;
 
 template <int S>
